@@ -31,6 +31,9 @@ hipError_t launch_triattn_core(const void* qkg, const void* vt, const void* tb, 
 hipError_t launch_triattn_core_f16_mfma(const void* qkg, const void* vt, const void* tb, const float* mask,
                                         int64_t mask_si, int64_t mask_sk, float inf, void* out, int64_t N,
                                         int64_t ldk, int H, int C, hipStream_t st);
+hipError_t launch_triattn_core_f32_x3(const void* qkg, const void* vt, const void* tb, const float* mask,
+                                      int64_t mask_si, int64_t mask_sk, float inf, void* out, int64_t N, int64_t ldk,
+                                      int H, hipStream_t st);
 hipError_t launch_triattn_core_simple(const void* qkg, const void* vt, const void* tb, const float* mask,
                                       int64_t mask_si, int64_t mask_sk, float inf, void* out, int dt, int64_t N,
                                       int64_t ldk, int H, int C, hipStream_t st);

@@ -76,6 +76,21 @@ BZPF_HD inline bool core_shape_ok(int64_t N, int64_t ldk, int C, int64_t mask_sk
          core_m_extent(N, mask_sk) <= 0x7fffffffLL;
 }
 
+// ---- the fp32 attention core on split operands (bzpf_triattn_x3.hip): 32-key stages of 4-byte elements (thread t stages
+// channels 4 (t % 8) .. + 3 of key t / 8, and keys 4 (t % 8) .. + 3 of channel t / 8; lane l reads key l % 32's mask).
+// Stage kb is half kb % 2 of bias block kb / 2: load v < 4 holds the lane's elements 16 (kb % 2) + 4 v .. + 3.
+constexpr int XCORE_BK = 32;
+BZPF_HD inline int xcore_k_lane(int t, int C) { return ((t >> 3) * C + (t & 7) * 4) * 4; }
+BZPF_HD inline int xcore_k_stage(int kb, int C) { return kb * XCORE_BK * C * 4; }
+BZPF_HD inline int xcore_v_lane(int t, int64_t ldk) { return (int)(((t >> 3) * ldk + (t & 7) * 4) * 4); }
+BZPF_HD inline int xcore_v_stage(int kb) { return kb * XCORE_BK * 4; }
+BZPF_HD inline int xcore_b_lane(int v, int l) { return 2048 * (v >> 1) + 32 * l + 16 * (v & 1); }
+BZPF_HD inline int xcore_b_stage(int kb) { return kb * 4096; }
+BZPF_HD inline int xcore_m_stage(int kb, int64_t mask_sk) { return (int)(kb * XCORE_BK * mask_sk * 4); }
+BZPF_HD inline int64_t xcore_k_extent(int64_t N, int C) { return N * C * 4; }
+BZPF_HD inline int64_t xcore_v_extent(int64_t ldk, int C) { return C * ldk * 4; }
+BZPF_HD inline int64_t xcore_b_extent(int64_t ldk) { return ldk / 64 * 8192; }
+
 // ---- the fp16 contraction (bzpf_trimul.hip): per channel, rows of ld fp16 values; a load's lane offset holds the
 // row (rows of a 256-row tile, past N reading as zero) and its 16-byte chunk, the scalar offset the 64-element stage.
 BZPF_HD inline int64_t contract_extent(int64_t N, int64_t ld) { return N * ld * 2; }

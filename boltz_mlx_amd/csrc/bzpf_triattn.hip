@@ -243,8 +243,11 @@ hipError_t launch_seq_attention(const void* q, const void* k, const void* v, con
   return hipSuccess;
 }
 
-// Core dispatch (impl mirrors the reference's scalar / mma choice, boltz_mlx/kernels.py:902-945): 0 = MFMA for
-// fp16 with C = 32, else the VALU kernel; 1 = the VALU kernel; 2 = MFMA (fp16, C = 32 only).
+// Core dispatch (impl mirrors the reference's scalar / mma choice, boltz_mlx/kernels.py:902-945): 0 = the matrix cores
+// for C = 32 (fp16, or fp32 as split operands), else the VALU kernel; 1 = the VALU kernel; 2 = MFMA (fp16, C = 32
+// only). The fp32 matrix-core kernel takes every N and mask stride that its 32-bit buffer offsets hold; at every size
+// measured it is the faster one (VALU -> matrix cores: N = 29 26 -> 18 us, 128 137 -> 15, 400 2,410 -> 285,
+// 640 8,980 -> 832).
 hipError_t launch_triattn_core(const void* qkg, const void* vt, const void* tb, const float* mask, int64_t mask_si,
                                int64_t mask_sk, float inf, void* out, int dt, int64_t N, int64_t ldk, int H, int C,
                                int impl, hipStream_t st) {
@@ -252,6 +255,8 @@ hipError_t launch_triattn_core(const void* qkg, const void* vt, const void* tb, 
   if (impl == 2 && !mfma_ok) return hipErrorInvalidValue;
   if ((impl == 0 && mfma_ok) || impl == 2)
     return launch_triattn_core_f16_mfma(qkg, vt, tb, mask, mask_si, mask_sk, inf, out, N, ldk, H, C, st);
+  if (impl == 0 && dt == DT_F32 && core_shape_ok(N, ldk, C, mask_sk))
+    return launch_triattn_core_f32_x3(qkg, vt, tb, mask, mask_si, mask_sk, inf, out, N, ldk, H, st);
   return launch_triattn_core_simple(qkg, vt, tb, mask, mask_si, mask_sk, inf, out, dt, N, ldk, H, C, st);
 }
 

@@ -19,12 +19,19 @@ struct Pair3 {
 __device__ __forceinline__ uint32_t cvt_pair(float a, float b) {
   return __builtin_bit_cast(uint32_t, bf16x2{(__bf16)a, (__bf16)b});
 }
+// The packed part is opaque to the compiler, which otherwise rounds each value a second time for its residual (five
+// conversions a pair instead of three).
+__device__ __forceinline__ uint32_t opaque_pair(float a, float b) {
+  uint32_t p = cvt_pair(a, b);
+  asm("" : "+v"(p));
+  return p;
+}
 __device__ __forceinline__ Pair3 split3_pair(float x0, float x1) {
 #pragma clang fp contract(off)  // the parts are of the rounded x0, x1 (no product of the caller fused in)
   Pair3 o;
-  o.p[0] = cvt_pair(x0, x1);
+  o.p[0] = opaque_pair(x0, x1);
   const float r0 = x0 - __uint_as_float(o.p[0] << 16), r1 = x1 - __uint_as_float(o.p[0] & 0xffff0000u);  // exact
-  o.p[1] = cvt_pair(r0, r1);
+  o.p[1] = opaque_pair(r0, r1);
   // exact: at most 8 significant bits are left
   o.p[2] = cvt_pair(r0 - __uint_as_float(o.p[1] << 16), r1 - __uint_as_float(o.p[1] & 0xffff0000u));
   return o;

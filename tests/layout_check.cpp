@@ -152,6 +152,34 @@ extern "C" int lc_check(char* out, int cap) {
     }
     rep.line(!core_shape_ok(32768, row_pitch(32768), 32, 1), "core refuses N=32768");
   }
+  // The fp32 core on split operands, behind the same limits: its stages' ranges, and its bias loads against tb_offset.
+  for (int64_t N : {1, 64, 1000, 32767}) {
+    const int64_t ldk = row_pitch(N);
+    const int kb = (int)((N + XCORE_BK - 1) / XCORE_BK) - 1;
+    int64_t k_lane = 0, v_lane = 0, b_lane = 0;
+    for (int t = 0; t < 256; t++) {
+      k_lane = std::max<int64_t>(k_lane, xcore_k_lane(t, 32));
+      v_lane = std::max<int64_t>(v_lane, xcore_v_lane(t, ldk));
+    }
+    for (int v = 0; v < 4; v++)
+      for (int l = 0; l < 64; l++) b_lane = std::max<int64_t>(b_lane, xcore_b_lane(v, l));
+    const BufRange ranges[4] = {{xcore_k_extent(N, 32), k_lane + xcore_k_stage(kb, 32)},
+                                {xcore_v_extent(ldk, 32), v_lane + xcore_v_stage(kb)},
+                                {xcore_b_extent(ldk), b_lane + xcore_b_stage(kb)},
+                                {core_m_extent(N, 1), core_m_lane(31, 1) + xcore_m_stage(kb, 1)}};
+    for (int i = 0; i < 4; i++)
+      rep.line(fits_int(ranges[i]) && (i == 0 || i == 3 || ranges[i].max_offset + 16 <= ranges[i].extent),
+               "fp32 core N=" + std::to_string(N) + ": " + range_str(ranges[i]));
+    rep.line((31 * ldk + 28) * 4 == v_lane && (31 * 32 + 28) * 4 == k_lane, "fp32 core staging covers its rows");
+    bool same = true;  // element e of load v, lane 32 hl + q: query q, key 32 kb + 8 (v) + 4 hl + e of the stage
+    for (int l = 0; l < 64; l++)
+      for (int v = 0; v < 4; v++)
+        for (int e = 0; e < 4; e++)
+          for (int64_t st = 0; st < ldk / XCORE_BK; st += std::max<int64_t>(1, ldk / XCORE_BK - 1))
+            same = same && xcore_b_stage((int)st) + xcore_b_lane(v, l) + 4 * e ==
+                               4 * tb_offset(0, l & 31, 32 * st + 8 * v + 4 * (l >> 5) + e, N, ldk);
+    rep.line(same, "fp32 core bias loads follow tb_offset N=" + std::to_string(N));
+  }
   // The contraction: the largest N its launcher accepts, and one past it.
   {
     int64_t nmax = 0;
