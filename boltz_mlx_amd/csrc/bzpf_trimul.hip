@@ -8,111 +8,114 @@
 #include "bzpf_common.h"
 #include "bzpf_kernels.h"
 #include "bzpf_rowgemm.h"
+#include "bzpf_x3.h"
 
 namespace bzpf {
 
-// ---------------------------------------------------------------- per-channel contraction
-// o[c][i][j] = sum_{k < ld} a[c][i][k] * b[c][j][k], a = ab[c], b = ab[D + c] (k >= N is zero padding).
-// Workgroup: a 128 x 128 tile (i, j) of one channel, 4 waves in 2 x 2, each 64 x 64 = 4 x 4 MFMA blocks. The tile is
-// computed transposed, o^T = b a^T (A operand = rows of b, B operand = rows of a), so each lane holds 4 consecutive
-// j of one i and stores them as one vector. K advances BK elements per stage through a double-buffered LDS tile;
-// the next stage is loaded into registers while the current one computes. Lane group g of a wave reads the
-// contiguous k range [g*BK/4, (g+1)*BK/4) of each stage (a permutation of the k sum shared by A and B).
+// ---------------------------------------------------------------- per-channel contraction, fp32
+// o[c][i][j] = sum_{k < kl} a[c][i][k] * b[c][j][k], a = ab[c], b = ab[D + c] (k >= N is zero padding), as split operands
+// on the bf16 matrix cores (bzpf_x3.h: three exact bf16 parts a value, six part products, fp32 sums).
+// Workgroup: a (32 MB WM) x (32 NB WN) tile (i, j) of one channel, WM x WN waves of MB x NB blocks of 32 x 32. K advances
+// KS = 16 per stage: the threads load the next stage's fp32 rows into registers while the current one computes, then
+// split them into the three part planes of the other LDS buffer (one barrier a stage: a buffer is written two stages
+// after it was last read). A block's lane holds one j and 16 i, so a store covers 128 contiguous bytes of two rows.
 // Tiles are ordered (channel, tile) and dealt to the XCDs in contiguous ranges, so one channel's a and b stay in
 // one XCD's L2.
-template <typename T>
-__global__ __launch_bounds__(256, 2) void trimul_contract_kernel(const T* __restrict__ ab, T* __restrict__ o,
-                                                                 int64_t N, int64_t ld, int D, int64_t tiles1,
-                                                                 int64_t units, int64_t per_xcd, int nst) {
-  constexpr int BT = 128;
-  constexpr int BK = sizeof(T) == 2 ? 64 : 32;      // k per stage: 128 bytes of a row
-  constexpr int KG = BK / 4;                        // contiguous k per lane group
-  constexpr int KP = Mfma<T>::KP;
-  constexpr int STEPS = KG / KP;
-  constexpr int LDT = BK + 16 / (int)sizeof(T);     // LDS row pitch (elements)
-  constexpr int VE = 16 / (int)sizeof(T);           // elements per 16-byte vector
-  constexpr int VPR = BK / VE;                      // vectors per row per stage (8)
-  constexpr int LOADS = 2 * BT * VPR / 256;         // 16-byte vectors per thread per stage (8)
-  __shared__ LDS_ALIGN T As[2][BT * LDT];           // rows of a (i)
-  __shared__ LDS_ALIGN T Bs[2][BT * LDT];           // rows of b (j)
+// Bound by the matrix cores and the split beside them (a stage of a 64 x 64 wave tile is 768 MFMA cycles and 88 VALU
+// instructions): N = 640 402 us (167 TFLOP/s, 0.4 of the bf16 peak in part products), N = 513 276, N = 333 79, against
+// 626, 555 and 160 us for the fp32 MFMA kernel this replaces; error against float64 3.8e-7 -> 3.2e-7 (N = 513).
+// Element k of row r of a part plane: rows of KS = 16 values, their two 16-byte halves exchanged in every other group of
+// eight rows, so the fragment reads (16 lanes on 16 rows at one half) meet 16 distinct bank groups without padding.
+__device__ __forceinline__ int x3_at(int r, int k) { return r * KS + (k ^ (r & 8)); }
+
+template <int WM, int WN, int MB, int NB>
+__global__ __launch_bounds__(64 * WM * WN, 2) void trimul_contract_x3_k(const float* __restrict__ ab,
+                                                                        float* __restrict__ o, int64_t N, int64_t ld,
+                                                                        int D, int tiles_i, int tiles_j, int64_t units,
+                                                                        int64_t per_xcd, int nst) {
+  constexpr int BI = 32 * MB * WM, BJ = 32 * NB * WN, T = 64 * WM * WN;
+  constexpr int LOADS = (BI + BJ) * (KS / 4) / T;  // 16-byte vectors per thread and stage
+  constexpr int ROWS = T / (KS / 4);               // rows a pass of all threads covers
+  static_assert((BI + BJ) * (KS / 4) % T == 0 && BI % ROWS == 0, "staging covers whole passes of a, then of b");
+  constexpr int PL = (BI + BJ) * KS;               // one part plane: the a rows, then the b rows
+  __shared__ LDS_ALIGN __bf16 P[2][3 * PL];
 
   const int64_t u = (int64_t)(blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-  if (u >= units) return;
-  const int64_t c = u / (tiles1 * tiles1);
-  const int64_t tt = u - c * tiles1 * tiles1;
-  const int64_t i0 = (tt / tiles1) * BT, j0 = (tt % tiles1) * BT;
-  const T* a = ab + c * N * ld;
-  const T* b = ab + ((int64_t)D + c) * N * ld;
-  const int t = threadIdx.x, wave = t >> 6, l = t & 63, g = l >> 4;
-  const int wi = wave >> 1, wj = wave & 1;
+  if (u >= units) return;  // whole workgroup
+  const int tiles = tiles_i * tiles_j;
+  const int64_t c = u / tiles;
+  const int tt = (int)(u - c * tiles);
+  const int i0 = (tt / tiles_j) * BI, j0 = (tt % tiles_j) * BJ;
+  const float* a = ab + c * N * ld;
+  const float* b = ab + ((int64_t)D + c) * N * ld;
+  const int t = threadIdx.x, l = t & 63, r32 = l & 31, hl = l >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wi = wave / WN, wj = wave % WN;
 
-  // stage loads: vector v of thread t covers row (v*256 + t) / VPR of [a rows | b rows], column ((..) % VPR) * VE
-  u32x4_t reg[LOADS];
-  auto gload = [&](int64_t k0) {
+  // vector v of thread t: row v * ROWS + t / 4 of [a rows | b rows] (rows past N repeat the last one; their outputs are
+  // not stored), k = 4 (t % 4) of the stage
+  const float* src[LOADS];
 #pragma unroll
-    for (int v = 0; v < LOADS; v++) {
-      const int e = v * 256 + t, r = e / VPR, col = (e % VPR) * VE;
-      const bool isb = r >= BT;
-      int64_t row = (isb ? j0 : i0) + (isb ? r - BT : r);
-      if (row >= N) row = N - 1;
-      reg[v] = *reinterpret_cast<const u32x4_t*>((isb ? b : a) + row * ld + k0 + col);
-    }
-  };
-  auto lstore = [&](int buf) {
+  for (int v = 0; v < LOADS; v++) {
+    const int row = v * ROWS + (t >> 2);
+    const int64_t g = v * ROWS < BI ? min((int64_t)(i0 + row), N - 1) : min((int64_t)(j0 + row - BI), N - 1);
+    src[v] = (v * ROWS < BI ? a : b) + g * ld + 4 * (t & 3);
+  }
+  f4 reg[LOADS];
+  auto gload = [&](int st) {
 #pragma unroll
-    for (int v = 0; v < LOADS; v++) {
-      const int e = v * 256 + t, r = e / VPR, col = (e % VPR) * VE;
-      T* dst = r >= BT ? Bs[buf] + (r - BT) * LDT : As[buf] + r * LDT;
-      *reinterpret_cast<u32x4_t*>(dst + col) = reg[v];
-    }
+    for (int v = 0; v < LOADS; v++) reg[v] = *reinterpret_cast<const f4*>(src[v] + st * KS);
   };
-
-  f4 acc[4][4];  // acc[jb][ib]: o^T block (j = 64*wj + 16*jb .., i = 64*wi + 16*ib ..)
-  zero_acc(acc);
+  f16x acc[MB][NB];
+#pragma unroll
+  for (int m = 0; m < MB; m++)
+#pragma unroll
+    for (int n = 0; n < NB; n++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) acc[m][n][e] = 0.f;
   gload(0);
-  lstore(0);
-  __syncthreads();
   for (int st = 0; st < nst; st++) {
-    const int buf = st & 1;
-    if (st + 1 < nst) gload((int64_t)(st + 1) * BK);
-    const T* Ab = As[buf];
-    const T* Bb = Bs[buf];
+    __bf16* pl = P[st & 1];
 #pragma unroll
-    for (int s = 0; s < STEPS; s++) {
-      typename Mfma<T>::frag fa[4], fb[4];
+    for (int v = 0; v < LOADS; v++) {
+      const Pair3 lo = split3_pair(reg[v][0], reg[v][1]), hi = split3_pair(reg[v][2], reg[v][3]);
 #pragma unroll
-      for (int ib = 0; ib < 4; ib++)
-        fa[ib] = Mfma<T>::load(Ab + (64 * wi + 16 * ib + (l & 15)) * LDT + KG * g + KP * s);
-#pragma unroll
-      for (int jb = 0; jb < 4; jb++)
-        fb[jb] = Mfma<T>::load(Bb + (64 * wj + 16 * jb + (l & 15)) * LDT + KG * g + KP * s);
-#pragma unroll
-      for (int jb = 0; jb < 4; jb++)
-#pragma unroll
-        for (int ib = 0; ib < 4; ib++) acc[jb][ib] = Mfma<T>::run(fb[jb], fa[ib], acc[jb][ib]);
+      for (int q = 0; q < 3; q++)
+        *reinterpret_cast<uint2*>(pl + q * PL + x3_at(v * ROWS + (t >> 2), 4 * (t & 3))) = uint2{lo.p[q], hi.p[q]};
     }
-    if (st + 1 < nst) lstore(buf ^ 1);
     __syncthreads();
+    if (st + 1 < nst) gload(st + 1);
+    bf16x8 fa[MB][3], fb[NB][3];
+#pragma unroll
+    for (int m = 0; m < MB; m++)
+#pragma unroll
+      for (int q = 0; q < 3; q++)
+        fa[m][q] = *reinterpret_cast<const bf16x8*>(pl + q * PL + x3_at(32 * (MB * wi + m) + r32, 8 * hl));
+#pragma unroll
+    for (int n = 0; n < NB; n++)
+#pragma unroll
+      for (int q = 0; q < 3; q++)
+        fb[n][q] = *reinterpret_cast<const bf16x8*>(pl + q * PL + x3_at(BI + 32 * (NB * wj + n) + r32, 8 * hl));
+#pragma unroll
+    for (int m = 0; m < MB; m++)
+#pragma unroll
+      for (int n = 0; n < NB; n++) acc[m][n] = mfma_parts6(fa[m], fb[n], acc[m][n]);
   }
-  // acc[jb][ib][e] = o[i = i0 + 64 wi + 16 ib + (l & 15)][j = j0 + 64 wj + 16 jb + 4 g + e]
-  T* oc = o + c * N * ld;
+  // acc[m][n][4 q + e] = o[i0 + 32 MB wi + 32 m + 8 q + 4 hl + e][j0 + 32 NB wj + 32 n + r32]
+  float* oc = o + c * N * ld;
 #pragma unroll
-  for (int ib = 0; ib < 4; ib++) {
-    const int64_t i = i0 + 64 * wi + 16 * ib + (l & 15);
-    if (i >= N) continue;
+  for (int m = 0; m < MB; m++)
 #pragma unroll
-    for (int jb = 0; jb < 4; jb++) {
-      const int64_t j = j0 + 64 * wj + 16 * jb + 4 * g;
+    for (int n = 0; n < NB; n++) {
+      const int64_t j = j0 + 32 * NB * wj + 32 * n + r32;
       if (j >= ld) continue;
-      T* dst = oc + i * ld + j;
-      if constexpr (sizeof(T) == 2) {
-        *reinterpret_cast<half4*>(dst) =
-            half4{(half_t)acc[jb][ib][0], (half_t)acc[jb][ib][1], (half_t)acc[jb][ib][2], (half_t)acc[jb][ib][3]};
-      } else {
-        *reinterpret_cast<f4*>(dst) = acc[jb][ib];
-      }
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int64_t i = i0 + 32 * MB * wi + 32 * m + 8 * q + 4 * hl + e;
+          if (i < N) oc[i * ld + j] = acc[m][n][4 * q + e];
+        }
     }
-  }
 }
 
 // fp16 form, persistent and LDS-direct. One 512-thread workgroup per CU walks its tiles (256 x 256 of one channel) as
@@ -298,26 +301,34 @@ __global__ __launch_bounds__(512, 1) void trimul_contract_f16_k(const half_t* __
   __builtin_amdgcn_s_waitcnt(0);  // no LDS write of a trailing (unused) stage load outlives the workgroup
 }
 
-// kl: the k range contracted (a multiple of the stage width, <= ld); columns past it are zero in a and b.
-template <typename T>
-static hipError_t contract_t(const void* ab, void* o, int64_t N, int64_t ld, int64_t kl, int D, hipStream_t st) {
-  const int BT = sizeof(T) == 2 ? 256 : 128;
-  const int64_t tiles1 = (N + BT - 1) / BT;
-  const int64_t units = (int64_t)D * tiles1 * tiles1;
-  const int64_t per_xcd = (units + 7) / 8;
-  const dim3 grid((unsigned)(per_xcd * 8));
-  if constexpr (sizeof(T) == 2) {
-    static int cache[kMaxDevices] = {};
-    const int resident = resident_grid(trimul_contract_f16_k<64, 2>, 512, cache);
-    if (resident < 8) return hipErrorInvalidConfiguration;
-    const int wpx = (int)(resident / 8 < per_xcd ? resident / 8 : per_xcd);
-    trimul_contract_f16_k<64, 2><<<dim3(8 * wpx), 512, 0, st>>>(static_cast<const half_t*>(ab), static_cast<half_t*>(o),
-                                                               N, ld, D, tiles1, units, per_xcd, wpx, (int)(kl / 64));
-  } else {
-    trimul_contract_kernel<T><<<grid, 256, 0, st>>>(static_cast<const T*>(ab), static_cast<T*>(o), N, ld, D, tiles1,
-                                                    units, per_xcd, (int)(kl / 32));
-  }
+// kl: the k range contracted (a multiple of 64, <= ld); columns past it are zero in a and b.
+static hipError_t contract_f16(const half_t* ab, half_t* o, int64_t N, int64_t ld, int64_t kl, int D, hipStream_t st) {
+  const int64_t tiles1 = (N + 255) / 256, units = (int64_t)D * tiles1 * tiles1, per_xcd = (units + 7) / 8;
+  static int cache[kMaxDevices] = {};
+  const int resident = resident_grid(trimul_contract_f16_k<64, 2>, 512, cache);
+  if (resident < 8) return hipErrorInvalidConfiguration;
+  const int wpx = (int)(resident / 8 < per_xcd ? resident / 8 : per_xcd);
+  trimul_contract_f16_k<64, 2>
+      <<<dim3(8 * wpx), 512, 0, st>>>(ab, o, N, ld, D, tiles1, units, per_xcd, wpx, (int)(kl / 64));
   return hipGetLastError();
+}
+
+template <int WM, int WN, int MB, int NB>
+static hipError_t contract_x3(const float* ab, float* o, int64_t N, int64_t ld, int64_t kl, int D, hipStream_t st) {
+  constexpr int BI = 32 * MB * WM, BJ = 32 * NB * WN;
+  const int64_t ti = (N + BI - 1) / BI, tj = (N + BJ - 1) / BJ, units = (int64_t)D * ti * tj, per_xcd = (units + 7) / 8;
+  trimul_contract_x3_k<WM, WN, MB, NB><<<dim3((unsigned)(per_xcd * 8)), 64 * WM * WN, 0, st>>>(
+      ab, o, N, ld, D, (int)ti, (int)tj, units, per_xcd, (int)(kl / KS));
+  return hipGetLastError();
+}
+
+// 192 x 192 tiles (3 x 3 blocks a wave: half again the products per LDS read of 2 x 2) where their padded area is not much
+// larger than that of 128 x 128 tiles: they measure 0.83-0.85 ns per 1,000 padded outputs and channel against 0.98
+// (N = 513: 276 against 359 us; N = 333, equal areas: 79 against 93; N = 400: 226 against 186; N = 640: 502 against 402).
+static hipError_t contract_f32(const float* ab, float* o, int64_t N, int64_t ld, int64_t kl, int D, hipStream_t st) {
+  const int64_t t128 = (N + 127) / 128 * 128, t192 = (N + 191) / 192 * 192;
+  return 7 * t192 * t192 <= 8 * t128 * t128 ? contract_x3<2, 2, 3, 3>(ab, o, N, ld, kl, D, st)
+                                            : contract_x3<2, 2, 2, 2>(ab, o, N, ld, kl, D, st);
 }
 
 hipError_t launch_trimul_contract(const void* ab, void* o, int dt, int64_t N, int64_t ld, int64_t k_len, int D,
@@ -325,7 +336,8 @@ hipError_t launch_trimul_contract(const void* ab, void* o, int dt, int64_t N, in
   if (dt == DT_F16 && !contract_shape_ok(N, ld)) return hipErrorInvalidValue;  // 32-bit buffer offsets per channel
   // contract over k < k_len rounded up to 64 (a whole number of stages of either kernel); 0 or >= N: every k
   const int64_t kl = k_len <= 0 || k_len >= N ? ld : (k_len + 63) / 64 * 64;
-  return dt == DT_F16 ? contract_t<half_t>(ab, o, N, ld, kl, D, st) : contract_t<float>(ab, o, N, ld, kl, D, st);
+  return dt == DT_F16 ? contract_f16(static_cast<const half_t*>(ab), static_cast<half_t*>(o), N, ld, kl, D, st)
+                      : contract_f32(static_cast<const float*>(ab), static_cast<float*>(o), N, ld, kl, D, st);
 }
 
 }  // namespace bzpf

@@ -74,3 +74,17 @@ def test_triattn_core_f32(N, pad, holes, trans, inf):
         got, valu, ref = (t.view(N, N, H * C)[live] for t in (got, valu, ref))
     assert _rel(got, ref) <= 1e-6
     assert _rel(got, valu.double()) <= 2e-6
+
+
+# tile edges of the two tile shapes (128 and 192), the k extent, one token
+@pytest.mark.parametrize("N,k_len", [(1, 0), (29, 0), (64, 40), (128, 0), (129, 0), (192, 100), (193, 0), (333, 320)])
+def test_trimul_contract_f32(N, k_len):
+    from boltz_mlx_amd import kernels as K
+
+    D, ld = 16, K.row_pitch(N)
+    g = torch.Generator(device="cuda").manual_seed(N)
+    ab = torch.zeros((2 * D, N, ld), device="cuda")
+    ab[:, :, :k_len or N] = torch.randn((2 * D, N, k_len or N), generator=g, device="cuda")
+    o = K.trimul_contract(ab, N, k_len)
+    ref = ab[:D].double() @ ab[D:].double().transpose(1, 2).contiguous()
+    assert _rel(o[:, :, :N], ref) <= 1e-6
