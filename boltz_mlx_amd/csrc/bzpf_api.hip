@@ -90,7 +90,7 @@ int bzpf_trimul_proj(const void* xn, const void* w_pg, const float* pair_mask, f
   REQUIRE(D == 128, "bzpf_trimul_proj: D must be 128 (got %d)", D);
   REQUIRE(N >= 1 && ld == bzpf_row_pitch(N), "bzpf_trimul_proj: N=%lld ld=%lld (ld must be bzpf_row_pitch(N))",
           (long long)N, (long long)ld);
-  return done(bzpf::launch_trimul_proj(xn, w_pg, pair_mask, scale, incoming, ab, dt, N, ld, S(stream)),
+  return done(bzpf::launch_trimul_proj(xn, w_pg, pair_mask, scale, incoming, ab, dt, N, ld, D, S(stream)),
               "bzpf_trimul_proj");
 }
 
@@ -120,7 +120,7 @@ int bzpf_trimul_tail(const void* o, const float* norm_out_w, const float* norm_o
   REQUIRE(D == 128, "bzpf_trimul_tail: D must be 128 (got %d)", D);
   REQUIRE(N >= 1 && ld == bzpf_row_pitch(N), "bzpf_trimul_tail: N=%lld ld=%lld", (long long)N, (long long)ld);
   return done(bzpf::launch_trimul_tail(o, norm_out_w, norm_out_b, eps_out, w_po, xn, w_go, z, accumulate, next_w,
-                                       next_b, next_eps, xn_next, dt, N, ld, S(stream)),
+                                       next_b, next_eps, xn_next, dt, N, ld, D, S(stream)),
               "bzpf_trimul_tail");
 }
 
@@ -135,7 +135,7 @@ int bzpf_triattn_proj(const void* xn, const void* w, int trans, float q_scale, f
           "bzpf_triattn_proj: need D = H*C = 128, C in {16,32,64} (D=%d H=%d C=%d)", D, H, C);
   REQUIRE(N >= 1 && ldk == bzpf_row_pitch(N), "bzpf_triattn_proj: N=%lld ldk=%lld (ldk must be bzpf_row_pitch(N))",
           (long long)N, (long long)ldk);
-  return done(bzpf::launch_triattn_proj(xn, w, trans, q_scale, bias_scale, qkg, vt, tri_bias, dt, N, ldk, H, C,
+  return done(bzpf::launch_triattn_proj(xn, w, trans, q_scale, bias_scale, qkg, vt, tri_bias, dt, N, ldk, D, H, C,
                                         S(stream)),
               "bzpf_triattn_proj");
 }
@@ -170,8 +170,69 @@ int bzpf_linear_resid_ln(const void* x, const void* w, int trans, float* z, int 
   REQUIRE(D == 128, "bzpf_linear_resid_ln: D must be 128 (got %d)", D);
   REQUIRE(N >= 1, "bzpf_linear_resid_ln: N < 1");
   return done(bzpf::launch_linear_resid_ln(x, w, trans, z, accumulate, next_w, next_b, next_eps, xn_next, dt, N,
-                                           S(stream)),
+                                           D, S(stream)),
               "bzpf_linear_resid_ln");
+}
+
+// The 64-channel forms: the same checks, N and pitch included.
+int bzpf_trimul_proj64(const void* xn, const void* w_pg, const float* pair_mask, float scale, int incoming, void* ab,
+                       int dt, int64_t N, int64_t ld, void* stream) {
+  REQUIRE_PTR(xn);
+  REQUIRE_PTR(w_pg);
+  REQUIRE_PTR(ab);
+  REQUIRE(pair_mask != nullptr, "bzpf_trimul_proj64: pair_mask is NULL");
+  REQUIRE(dt_ok(dt), "bzpf_trimul_proj64: bad dtype %d", dt);
+  REQUIRE(N >= 1 && ld == bzpf_row_pitch(N), "bzpf_trimul_proj64: N=%lld ld=%lld", (long long)N, (long long)ld);
+  return done(bzpf::launch_trimul_proj(xn, w_pg, pair_mask, scale, incoming, ab, dt, N, ld, 64, S(stream)),
+              "bzpf_trimul_proj64");
+}
+
+int bzpf_trimul_tail64(const void* o, const float* norm_out_w, const float* norm_out_b, float eps_out,
+                       const void* w_po, const void* xn, const void* w_go, float* z, int accumulate,
+                       const float* next_w, const float* next_b, float next_eps, void* xn_next, int dt, int64_t N,
+                       int64_t ld, void* stream) {
+  REQUIRE_PTR(o);
+  REQUIRE_PTR(w_po);
+  REQUIRE_PTR(xn);
+  REQUIRE_PTR(w_go);
+  REQUIRE_PTR(z);
+  REQUIRE(norm_out_w && norm_out_b, "bzpf_trimul_tail64: norm_out weight/bias required");
+  REQUIRE(next_w == nullptr || (next_b != nullptr && xn_next != nullptr),
+          "bzpf_trimul_tail64: next LN needs next_b and xn_next");
+  REQUIRE(dt_ok(dt), "bzpf_trimul_tail64: bad dtype %d", dt);
+  REQUIRE(N >= 1 && ld == bzpf_row_pitch(N), "bzpf_trimul_tail64: N=%lld ld=%lld", (long long)N, (long long)ld);
+  return done(bzpf::launch_trimul_tail(o, norm_out_w, norm_out_b, eps_out, w_po, xn, w_go, z, accumulate, next_w,
+                                       next_b, next_eps, xn_next, dt, N, ld, 64, S(stream)),
+              "bzpf_trimul_tail64");
+}
+
+int bzpf_triattn_proj64(const void* xn, const void* w, int trans, float q_scale, float bias_scale, void* qkg, void* vt,
+                        void* tri_bias, int dt, int64_t N, int64_t ldk, int H, int C, void* stream) {
+  REQUIRE_PTR(xn);
+  REQUIRE_PTR(w);
+  REQUIRE_PTR(qkg);
+  REQUIRE(vt != nullptr && tri_bias != nullptr, "bzpf_triattn_proj64: NULL pointer");
+  REQUIRE(dt_ok(dt), "bzpf_triattn_proj64: bad dtype %d", dt);
+  REQUIRE(H >= 1 && H * C == 128 && (C == 16 || C == 32 || C == 64),
+          "bzpf_triattn_proj64: need H*C = 128, C in {16,32,64} (H=%d C=%d)", H, C);
+  REQUIRE(N >= 1 && ldk == bzpf_row_pitch(N), "bzpf_triattn_proj64: N=%lld ldk=%lld", (long long)N, (long long)ldk);
+  return done(bzpf::launch_triattn_proj(xn, w, trans, q_scale, bias_scale, qkg, vt, tri_bias, dt, N, ldk, 64, H, C,
+                                        S(stream)),
+              "bzpf_triattn_proj64");
+}
+
+int bzpf_linear_resid_ln64(const void* x, const void* w, int trans, float* z, int accumulate, const float* next_w,
+                           const float* next_b, float next_eps, void* xn_next, int dt, int64_t N, void* stream) {
+  REQUIRE_PTR(x);
+  REQUIRE_PTR(w);
+  REQUIRE_PTR(z);
+  REQUIRE(next_w == nullptr || (next_b != nullptr && xn_next != nullptr),
+          "bzpf_linear_resid_ln64: next LN needs next_b and xn_next");
+  REQUIRE(dt_ok(dt), "bzpf_linear_resid_ln64: bad dtype %d", dt);
+  REQUIRE(N >= 1, "bzpf_linear_resid_ln64: N < 1");
+  return done(bzpf::launch_linear_resid_ln(x, w, trans, z, accumulate, next_w, next_b, next_eps, xn_next, dt, N, 64,
+                                           S(stream)),
+              "bzpf_linear_resid_ln64");
 }
 
 int bzpf_transition(const void* xn, const void* w12, const void* w3, float* z, int accumulate, const float* next_w,

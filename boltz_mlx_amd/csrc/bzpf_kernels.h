@@ -15,16 +15,17 @@ hipError_t launch_add_ln(float* z, const void* y, int y_dt, float scale, int tra
 hipError_t launch_count_nonfinite(const void* x, int dt, int64_t n, int* count, hipStream_t st);
 
 hipError_t launch_trimul_proj(const void* xn, const void* w, const float* mask, float scale, int incoming, void* ab,
-                              int dt, int64_t N, int64_t ld, hipStream_t st);
+                              int dt, int64_t N, int64_t ld, int dim, hipStream_t st);
 hipError_t launch_trimul_contract(const void* ab, void* o, int dt, int64_t N, int64_t ld, int64_t k_len, int D,
                                   hipStream_t st);
 hipError_t launch_trimul_tail(const void* o, const float* now, const float* nob, float eps_out, const void* w_po,
                               const void* xn, const void* w_go, float* z, int accumulate, const float* lnw,
                               const float* lnb, float eps_next, void* xn_next, int dt, int64_t N, int64_t ld,
-                              hipStream_t st);
+                              int dim, hipStream_t st);
 
 hipError_t launch_triattn_proj(const void* xn, const void* w, int trans, float q_scale, float b_scale, void* qkg,
-                               void* vt, void* tb, int dt, int64_t N, int64_t ldk, int H, int C, hipStream_t st);
+                               void* vt, void* tb, int dt, int64_t N, int64_t ldk, int dim, int H, int C,
+                               hipStream_t st);
 hipError_t launch_triattn_core(const void* qkg, const void* vt, const void* tb, const float* mask, int64_t mask_si,
                                int64_t mask_sk, float inf, void* out, int dt, int64_t N, int64_t ldk, int H, int C,
                                int impl, hipStream_t st);
@@ -39,7 +40,7 @@ hipError_t launch_triattn_core_simple(const void* qkg, const void* vt, const voi
                                       int64_t ldk, int H, int C, hipStream_t st);
 hipError_t launch_linear_resid_ln(const void* x, const void* w, int trans, float* z, int accumulate,
                                   const float* lnw, const float* lnb, float eps, void* xn_next, int dt, int64_t N,
-                                  hipStream_t st);
+                                  int dim, hipStream_t st);
 hipError_t launch_transition(const void* xn, const void* w12, const void* w3, float* z, int accumulate,
                              const float* lnw, const float* lnb, float eps, void* xn_next, int dt, int64_t rows,
                              int hidden, hipStream_t st);

@@ -9,6 +9,8 @@
 //   transition       : z (+)= fc3(silu(fc1 xn) * fc2 xn), then the next LayerNorm (transition.py:27-54, 148-154;
 //                      kernels_nax2.py:54-190, kernels_nax3.py:713-827).
 // Tiles are 64 * RB rows (positions) per workgroup of 4 waves, RB = 2 row blocks per wave for fp16 and 1 for fp32.
+#include <type_traits>
+
 #include "bzpf_common.h"
 #include "bzpf_kernels.h"
 #include "bzpf_rowgemm.h"
@@ -19,7 +21,7 @@ namespace {
 
 constexpr int D = 128;
 
-template <typename T> constexpr int ldw_of() { return D + Pad<T>::v; }
+template <typename T, int KIN = D> constexpr int ldw_of() { return KIN + Pad<T>::v; }
 
 // ---------------------------------------------------------------- triangle multiplication projection
 // Persistent, one 512-thread workgroup per CU (8 waves, up to 256 VGPRs each). The launch covers output channels
@@ -31,16 +33,17 @@ template <typename T> constexpr int ldw_of() { return D + Pad<T>::v; }
 // values are loaded while the current tile computes (8 waves with the prefetch measured 3-4% faster than 12
 // without). HV = 1 (half tiles) is taken when it balances the last round of tiles better: at N = 400 (2,800 full
 // tiles on 2,048 waves) 0.041-0.045 against 0.050 ms; at N = 1000 full tiles are faster (0.23 against 0.26 ms).
-template <typename T> constexpr int proj_ch() { return sizeof(T) == 2 ? 256 : 128; }
+template <typename T, int KIN = D> constexpr int proj_ch() { return sizeof(T) == 2 ? 2 * KIN : 128; }
 constexpr int PROJ_WAVES = 8;
 
-template <typename T, int HV>
+template <typename T, int HV, int KIN>
 __global__ __launch_bounds__(64 * PROJ_WAVES) void trimul_proj_k(const T* __restrict__ xn, const T* __restrict__ w,
                                                                  const float* __restrict__ mask, float scale,
                                                                  int incoming, T* __restrict__ ab, int64_t N,
                                                                  int64_t ld, int c_lo) {
   using RT = RunTile<T>;
-  constexpr int RB = RT::RB, TW = RT::TW, STEPS = RG<T>::STEPS, LDW = ldw_of<T>(), PCH = proj_ch<T>();
+  constexpr int D = KIN;
+  constexpr int RB = RT::RB, TW = RT::TW, STEPS = RG<T, D>::STEPS, LDW = ldw_of<T, D>(), PCH = proj_ch<T, D>();
   __shared__ LDS_ALIGN T Ws[2 * PCH * LDW];  // rows [0, PCH): projections, [PCH, 2 PCH): gates
   lds_rows<T>(Ws, LDW, 2 * PCH, D,
               [&](int r) { return w + (int64_t)(r < PCH ? c_lo + r : 2 * D + c_lo + r - PCH) * D; });
@@ -50,7 +53,7 @@ __global__ __launch_bounds__(64 * PROJ_WAVES) void trimul_proj_k(const T* __rest
   int t = grid_wave(PROJ_WAVES);
   if (t >= ntiles) return;
 
-  typedef typename RG<T>::frag Frag;
+  typedef typename RG<T, D>::frag Frag;
   Frag x[HV][RB][STEPS];
   // mask values of the rows this lane loads, raw (at the clamped position): scaled, and zeroed past N (padding columns
   // are written as 0), where they are used. Any arithmetic on them at the load would wait for the prefetch there.
@@ -63,7 +66,7 @@ __global__ __launch_bounds__(64 * PROJ_WAVES) void trimul_proj_k(const T* __rest
       for (int rb = 0; rb < RB; rb++) {
         const int64_t k = k0 + hh * TW + RT::pos(rb, r), kc = k < N ? k : N - 1;
         const int64_t src = incoming ? kc * N + i : (int64_t)i * N + kc;
-        RG<T>::load_row(xx[hh][rb], xn + src * D, g);
+        RG<T, D>::load_row(xx[hh][rb], xn + src * D, g);
         mm[hh][rb] = mask[src];
       }
   };
@@ -89,8 +92,8 @@ __global__ __launch_bounds__(64 * PROJ_WAVES) void trimul_proj_k(const T* __rest
         f4 pa[RB][1], ga[RB][1];
         zero_acc(pa);
         zero_acc(ga);
-        mma_rows<T, RB, 1, true>(pa, x[hh], Ws + 16 * cb * LDW, LDW);
-        mma_rows<T, RB, 1, true>(ga, x[hh], Ws + (PCH + 16 * cb) * LDW, LDW);
+        mma_rows<T, RB, 1, true, D>(pa, x[hh], Ws + 16 * cb * LDW, LDW);
+        mma_rows<T, RB, 1, true, D>(ga, x[hh], Ws + (PCH + 16 * cb) * LDW, LDW);
         float v[RT::RUN];
 #pragma unroll
         for (int rb = 0; rb < RB; rb++)
@@ -113,14 +116,15 @@ __global__ __launch_bounds__(64 * PROJ_WAVES) void trimul_proj_k(const T* __rest
 
 // ---------------------------------------------------------------- triangle multiplication tail
 // grid: N * tiles_per_row over the padded rows (positions (i, j0 .. j0+TM)).
-template <typename T>
+template <typename T, int KIN>
 __global__ __launch_bounds__(256) void trimul_tail_k(const T* __restrict__ o, const float* __restrict__ now,
                                                      const float* __restrict__ nob, float eps_out,
                                                      const T* __restrict__ w_po, const T* __restrict__ xn,
                                                      const T* __restrict__ w_go, float* __restrict__ z, int accumulate,
                                                      const float* __restrict__ lnw, const float* __restrict__ lnb,
                                                      float eps_next, T* __restrict__ xn_next, int64_t N, int64_t ld) {
-  constexpr int RB = RowBlocks<T>::v, TM = 64 * RB, STEPS = RG<T>::STEPS, LDW = ldw_of<T>();
+  constexpr int D = KIN, NC = D / 64, QC = D / 4;  // 64-channel chunks, channels per LayerNorm thread
+  constexpr int RB = RowBlocks<T>::v, TM = 64 * RB, STEPS = RG<T, D>::STEPS, LDW = ldw_of<T, D>();
   __shared__ LDS_ALIGN T Ts[TM * LDW];  // o tile transposed to [position][channel], then LN_out of it
   __shared__ LDS_ALIGN T Ws[64 * LDW];
   const int64_t tpr = (ld + TM - 1) / TM;
@@ -144,37 +148,37 @@ __global__ __launch_bounds__(256) void trimul_tail_k(const T* __restrict__ o, co
   // LN_out over the 128 channels of each position (4 threads per row, two-pass fp32 statistics)
   for (int r = threadIdx.x >> 2; r < TM; r += 64) {
     const int q = threadIdx.x & 3;
-    T* tr = Ts + r * LDW + q * 32;
-    float v[32];
+    T* tr = Ts + r * LDW + q * QC;
+    float v[QC];
     float s = 0.f;
 #pragma unroll
-    for (int c = 0; c < 32; c++) { v[c] = to_f(tr[c]); s += v[c]; }
+    for (int c = 0; c < QC; c++) { v[c] = to_f(tr[c]); s += v[c]; }
     const float mean = group_sum<4>(s) * (1.0f / D);
     float ss = 0.f;
 #pragma unroll
-    for (int c = 0; c < 32; c++) { const float d = v[c] - mean; ss += d * d; }
+    for (int c = 0; c < QC; c++) { const float d = v[c] - mean; ss += d * d; }
     const float rstd = 1.0f / sqrtf(group_sum<4>(ss) * (1.0f / D) + eps_out);
 #pragma unroll
-    for (int c = 0; c < 32; c++) tr[c] = from_f<T>((v[c] - mean) * rstd * now[q * 32 + c] + nob[q * 32 + c]);
+    for (int c = 0; c < QC; c++) tr[c] = from_f<T>((v[c] - mean) * rstd * now[q * QC + c] + nob[q * QC + c]);
   }
   int64_t jpos[RB];
-  typename RG<T>::frag x[RB][STEPS];
+  typename RG<T, D>::frag x[RB][STEPS];
 #pragma unroll
   for (int rb = 0; rb < RB; rb++) {
     jpos[rb] = j0 + wave * 16 * RB + 16 * rb + (l & 15);
     const int64_t jc = jpos[rb] < N ? jpos[rb] : N - 1;
-    RG<T>::load_row(x[rb], xn + (i * N + jc) * D, g);
+    RG<T, D>::load_row(x[rb], xn + (i * N + jc) * D, g);
   }
-  // gates sigmoid(xn W_go^T), two 64-channel chunks
-  f4 gate[RB][8];
+  // gates sigmoid(xn W_go^T), 64-channel chunks
+  f4 gate[RB][4 * NC];
 #pragma unroll
-  for (int cc = 0; cc < 2; cc++) {
+  for (int cc = 0; cc < NC; cc++) {
     __syncthreads();
     lds_rows<T>(Ws, LDW, 64, D, [&](int r) { return w_go + (int64_t)(64 * cc + r) * D; });
     __syncthreads();
     f4 acc[RB][4];
     zero_acc(acc);
-    mma_rows<T, RB, 4>(acc, x, Ws, LDW);
+    mma_rows<T, RB, 4, false, D>(acc, x, Ws, LDW);
 #pragma unroll
     for (int rb = 0; rb < RB; rb++)
 #pragma unroll
@@ -184,16 +188,16 @@ __global__ __launch_bounds__(256) void trimul_tail_k(const T* __restrict__ o, co
   }
   // LN_out rows as the B operand, p_out chunks
 #pragma unroll
-  for (int rb = 0; rb < RB; rb++) RG<T>::load_row(x[rb], Ts + (wave * 16 * RB + 16 * rb + (l & 15)) * LDW, g);
-  f4 y[RB][8];
+  for (int rb = 0; rb < RB; rb++) RG<T, D>::load_row(x[rb], Ts + (wave * 16 * RB + 16 * rb + (l & 15)) * LDW, g);
+  f4 y[RB][4 * NC];
 #pragma unroll
-  for (int cc = 0; cc < 2; cc++) {
+  for (int cc = 0; cc < NC; cc++) {
     __syncthreads();
     lds_rows<T>(Ws, LDW, 64, D, [&](int r) { return w_po + (int64_t)(64 * cc + r) * D; });
     __syncthreads();
     f4 acc[RB][4];
     zero_acc(acc);
-    mma_rows<T, RB, 4>(acc, x, Ws, LDW);
+    mma_rows<T, RB, 4, false, D>(acc, x, Ws, LDW);
 #pragma unroll
     for (int rb = 0; rb < RB; rb++)
 #pragma unroll
@@ -218,13 +222,16 @@ __global__ __launch_bounds__(256) void trimul_tail_k(const T* __restrict__ o, co
 constexpr int TAIL_WAVES = 12;
 __host__ __device__ constexpr int64_t tail_tiles_per_row(int64_t N) { return (N + 63) / 64 * 4; }
 
+template <int KIN>
 __global__ __launch_bounds__(64 * TAIL_WAVES) void trimul_tail_f16_k(
     const half_t* __restrict__ o, const float* __restrict__ now, const float* __restrict__ nob, float eps_out,
     const half_t* __restrict__ w_po, const half_t* __restrict__ xn, const half_t* __restrict__ w_go,
     float* __restrict__ z, int accumulate, const float* __restrict__ lnw, const float* __restrict__ lnb,
     float eps_next, half_t* __restrict__ xn_next, int64_t N, int64_t ld) {
   using T = half_t;
-  constexpr int STEPS = RG<T>::STEPS, LDW = ldw_of<T>(), LDT = D + Pad<T>::v;
+  constexpr int D = KIN, CB = D / 16, PP = D / 16;  // column blocks; positions of o a lane loads (of 4 channels)
+  constexpr int STEPS = RG<T, D>::STEPS, LDW = ldw_of<T, D>(), LDT = D + Pad<T>::v;
+  typedef half_t OVec __attribute__((ext_vector_type(PP)));
   __shared__ LDS_ALIGN T Wg[D * LDW];
   __shared__ LDS_ALIGN T Wp[D * LDW];  // p_out with gamma_out folded into its columns
   __shared__ LDS_ALIGN float Bp[D];    // p_out . beta_out
@@ -232,7 +239,7 @@ __global__ __launch_bounds__(64 * TAIL_WAVES) void trimul_tail_f16_k(
   __shared__ LDS_ALIGN T Ts[TAIL_WAVES][16 * LDT];
   lds_rows<T>(Wg, LDW, D, D, [&](int r) { return w_go + (int64_t)r * D; });
   for (int e = threadIdx.x; e < D * D / 8; e += blockDim.x) {
-    const int r = e >> 4, c = (e & 15) * 8;
+    const int r = e / (D / 8), c = e % (D / 8) * 8;
     const half8 wv = *reinterpret_cast<const half8*>(w_po + (int64_t)r * D + c);
     half8 sv;
 #pragma unroll
@@ -243,14 +250,14 @@ __global__ __launch_bounds__(64 * TAIL_WAVES) void trimul_tail_f16_k(
     Lw[threadIdx.x] = lnw[threadIdx.x];
     Lb[threadIdx.x] = lnb[threadIdx.x];
   }
-  if (threadIdx.x < 4 * D) {  // 4 lanes per output channel, 32 inputs each
+  if (threadIdx.x < 4 * D) {  // 4 lanes per output channel, D / 4 inputs each
     const int c = threadIdx.x >> 2, q = threadIdx.x & 3;
     float acc = 0.f;
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const half8 wv = *reinterpret_cast<const half8*>(w_po + (int64_t)c * D + 32 * q + 8 * v);
+    for (int v = 0; v < D / 32; v++) {
+      const half8 wv = *reinterpret_cast<const half8*>(w_po + (int64_t)c * D + D / 4 * q + 8 * v);
 #pragma unroll
-      for (int u = 0; u < 8; u++) acc += (float)wv[u] * nob[32 * q + 8 * v + u];
+      for (int u = 0; u < 8; u++) acc += (float)wv[u] * nob[D / 4 * q + 8 * v + u];
     }
     acc += __shfl_xor(acc, 1, 64);
     acc += __shfl_xor(acc, 2, 64);
@@ -267,19 +274,19 @@ __global__ __launch_bounds__(64 * TAIL_WAVES) void trimul_tail_f16_k(
   int tb = blockIdx.x * TAIL_WAVES;
   if (tb >= ntiles) return;  // whole workgroup
   int t = min(tb + wave, ntiles - 1);
-  const int ocg = l >> 1, opc = l & 1;
+  const int ocg = l / (16 / PP), opc = l % (16 / PP);
   // o element offsets are 32-bit (the launcher checks D * N * ld < 2^31): channel rows of this lane, one apart
   const uint32_t ochan = (uint32_t)(4 * ocg) * (uint32_t)N * (uint32_t)ld, orow = (uint32_t)N * (uint32_t)ld;
-  const auto load = [&](int tt, half8 (&ob)[4], typename RG<T>::frag (&xf)[1][STEPS]) {
+  const auto load = [&](int tt, OVec (&ob)[4], typename RG<T, D>::frag (&xf)[1][STEPS]) {
     const int i = tt / tpr, j0 = (tt - i * tpr) * 16;
-    const uint32_t oo = ochan + (uint32_t)i * (uint32_t)ld + (uint32_t)(j0 + 8 * opc);
+    const uint32_t oo = ochan + (uint32_t)i * (uint32_t)ld + (uint32_t)(j0 + PP * opc);
 #pragma unroll
-    for (int u = 0; u < 4; u++) ob[u] = *reinterpret_cast<const half8*>(o + (oo + u * orow));
+    for (int u = 0; u < 4; u++) ob[u] = *reinterpret_cast<const OVec*>(o + (oo + u * orow));
     const int64_t jc = j0 + r < N ? j0 + r : N - 1;
-    RG<T>::load_row(xf[0], xn + ((int64_t)i * N + jc) * D, g);
+    RG<T, D>::load_row(xf[0], xn + ((int64_t)i * N + jc) * D, g);
   };
-  half8 ob[4];
-  typename RG<T>::frag xf[1][STEPS];
+  OVec ob[4];
+  typename RG<T, D>::frag xf[1][STEPS];
   load(t, ob, xf);
   for (; tb < ntiles; tb += stride) {
     const bool live = tb + wave < ntiles;
@@ -290,29 +297,31 @@ __global__ __launch_bounds__(64 * TAIL_WAVES) void trimul_tail_f16_k(
     const auto zrow = [&](int) { return zr; };
     float* zt = opaque_ptr(z);
     half_t* xnt = opaque_ptr(xn_next);
-    f4 zv[1][8];
+    f4 zv[1][CB];
     load_z_rows<1>(zv, zrow, zt, accumulate);
     // o block -> [position][channel] rows of the wave's tile
 #pragma unroll
-    for (int v = 0; v < 8; v++)
-      *reinterpret_cast<half4*>(ts + (8 * opc + v) * LDT + 4 * ocg) = half4{ob[0][v], ob[1][v], ob[2][v], ob[3][v]};
-    half8 obn[4];
-    typename RG<T>::frag xfn[1][STEPS];
+    for (int v = 0; v < PP; v++)
+      *reinterpret_cast<half4*>(ts + (PP * opc + v) * LDT + 4 * ocg) = half4{ob[0][v], ob[1][v], ob[2][v], ob[3][v]};
+    OVec obn[4];
+    typename RG<T, D>::frag xfn[1][STEPS];
     load(min(t + stride, ntiles - 1), obn, xfn);
-    // gates first (their inputs are free afterwards), kept as fp16
-    half4 gate[8];
+    // gates first (their inputs are free afterwards), kept as fp16 at 128 channels and in fp32 at 64
+    typedef typename std::conditional<D == 128, half4, f4>::type Gate;
+    typedef typename std::conditional<D == 128, half_t, float>::type GateT;
+    Gate gate[CB];
     {
-      f4 ga[1][8];
+      f4 ga[1][CB];
       zero_acc(ga);
-      mma_rows_grouped<T, 1, 8, 1>(ga, xf, Wg, LDW);
+      mma_rows_grouped<T, 1, CB, 1, false, D>(ga, xf, Wg, LDW);
 #pragma unroll
-      for (int cb = 0; cb < 8; cb++)
-        gate[cb] = half4{(half_t)sigmoidf_(ga[0][cb][0]), (half_t)sigmoidf_(ga[0][cb][1]),
-                         (half_t)sigmoidf_(ga[0][cb][2]), (half_t)sigmoidf_(ga[0][cb][3])};
+      for (int cb = 0; cb < CB; cb++)
+        gate[cb] = Gate{(GateT)sigmoidf_(ga[0][cb][0]), (GateT)sigmoidf_(ga[0][cb][1]),
+                        (GateT)sigmoidf_(ga[0][cb][2]), (GateT)sigmoidf_(ga[0][cb][3])};
     }
-    // LN_out of this lane's position (channels 32 g .. 32 g + 31 here, the rest in lanes l ^ 16, l ^ 32, l ^ 48)
-    typename RG<T>::frag of[1][STEPS];
-    RG<T>::load_row(of[0], ts + r * LDT, g);
+    // LN_out of this lane's position (channels D/4 g .. + D/4 - 1 here, the rest in lanes l ^ 16, l ^ 32, l ^ 48)
+    typename RG<T, D>::frag of[1][STEPS];
+    RG<T, D>::load_row(of[0], ts + r * LDT, g);
     float sum = 0.f;
 #pragma unroll
     for (int s2 = 0; s2 < STEPS; s2++)
@@ -332,11 +341,11 @@ __global__ __launch_bounds__(64 * TAIL_WAVES) void trimul_tail_f16_k(
     for (int s2 = 0; s2 < STEPS; s2++)
 #pragma unroll
       for (int u = 0; u < 8; u++) of[0][s2][u] = (half_t)(((float)of[0][s2][u] - mean) * rstd);
-    f4 y[1][8];
+    f4 y[1][CB];
     zero_acc(y);
-    mma_rows_grouped<T, 1, 8, 1>(y, of, Wp, LDW);
+    mma_rows_grouped<T, 1, CB, 1, false, D>(y, of, Wp, LDW);
 #pragma unroll
-    for (int cb = 0; cb < 8; cb++) {
+    for (int cb = 0; cb < CB; cb++) {
       const f4 bp = *reinterpret_cast<const f4*>(Bp + 16 * cb + 4 * g);
 #pragma unroll
       for (int e = 0; e < 4; e++) y[0][cb][e] = (y[0][cb][e] + bp[e]) * (float)gate[cb][e];
@@ -359,7 +368,7 @@ __global__ __launch_bounds__(64 * TAIL_WAVES) void trimul_tail_f16_k(
 //             one 16-byte run of qkg[plane][i N + j][:] (q scaled by q_scale);
 //   v       : ROWS orientation, 16-byte runs of keys of vt[h][i][d][:] (zeros past N);
 //   bias    : ROWS orientation, runs of 4 keys of the fragment-ordered bias (scaled by b_scale, zeros past N).
-template <typename T> constexpr int attn_rows() { return sizeof(T) == 2 ? 4 * D + 16 : 2 * D + 16; }
+template <typename T, int KIN> constexpr int attn_rows() { return sizeof(T) == 2 || KIN == 64 ? 4 * D + 16 : 2 * D + 16; }
 
 __device__ __forceinline__ void st8(half_t* p, const float (&v)[8]) { st_run(p, v); }
 __device__ __forceinline__ void st8(float* p, const float (&v)[8]) {
@@ -371,7 +380,7 @@ __device__ __forceinline__ void st8(float* p, const float (&v)[8]) {
 // of the three output layouts do not fit the 128 VGPRs of 4 waves per SIMD.
 constexpr int ATTN_PROJ_WAVES = 12;
 
-template <typename T>
+template <typename T, int KIN>
 __global__ __launch_bounds__(64 * ATTN_PROJ_WAVES) void triattn_proj_k(const T* __restrict__ xn,
                                                                         const T* __restrict__ w, int trans,
                                                                         float q_scale, float b_scale,
@@ -379,14 +388,14 @@ __global__ __launch_bounds__(64 * ATTN_PROJ_WAVES) void triattn_proj_k(const T* 
                                                                         T* __restrict__ tb, int64_t N, int64_t ldk,
                                                                         int H, int C, int r_lo, int r_hi) {
   using RT = RunTile<T>;
-  constexpr int RB = RT::RB, TW = RT::TW, STEPS = RG<T>::STEPS, LDW = ldw_of<T>();
-  __shared__ LDS_ALIGN T Ws[attn_rows<T>() * LDW];
-  lds_rows<T>(Ws, LDW, r_hi - r_lo, D, [&](int lr) -> const T* {
+  constexpr int RB = RT::RB, TW = RT::TW, STEPS = RG<T, KIN>::STEPS, LDW = ldw_of<T, KIN>();
+  __shared__ LDS_ALIGN T Ws[attn_rows<T, KIN>() * LDW];
+  lds_rows<T>(Ws, LDW, r_hi - r_lo, KIN, [&](int lr) -> const T* {
     const int R = r_lo + lr;
-    if (R >= 4 * D) return R - 4 * D < H ? w + (int64_t)R * D : nullptr;
-    if (R >= 2 * D && R < 3 * D) return w + (int64_t)R * D;
+    if (R >= 4 * D) return R - 4 * D < H ? w + (int64_t)R * KIN : nullptr;
+    if (R >= 2 * D && R < 3 * D) return w + (int64_t)R * KIN;
     const int q = R & 31, rr = q & 15;
-    return w + (int64_t)((R & ~31) + 8 * (rr >> 2) + 4 * (q >> 4) + (rr & 3)) * D;
+    return w + (int64_t)((R & ~31) + 8 * (rr >> 2) + 4 * (q >> 4) + (rr & 3)) * KIN;
   });
   __syncthreads();
   const int l = threadIdx.x & 63, g = l >> 4, r = l & 15;
@@ -395,19 +404,19 @@ __global__ __launch_bounds__(64 * ATTN_PROJ_WAVES) void triattn_proj_k(const T* 
   int t = grid_wave(ATTN_PROJ_WAVES);
   if (t >= ntiles) return;
 
-  typename RG<T>::frag x[RB][STEPS];
-  const auto load = [&](int tt, typename RG<T>::frag (&xx)[RB][STEPS]) {
+  typename RG<T, KIN>::frag x[RB][STEPS];
+  const auto load = [&](int tt, typename RG<T, KIN>::frag (&xx)[RB][STEPS]) {
     const int i = tt / tpr, j0 = (tt - i * tpr) * TW;
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
       const int64_t j = j0 + RT::pos(rb, r), jc = j < N ? j : N - 1;
-      RG<T>::load_row(xx[rb], xn + (trans ? jc * N + i : (int64_t)i * N + jc) * D, g);
+      RG<T, KIN>::load_row(xx[rb], xn + (trans ? jc * N + i : (int64_t)i * N + jc) * KIN, g);
     }
   };
   load(t, x);
   for (; t < ntiles; t += stride) {
     const int i = t / tpr, j0 = (t - i * tpr) * TW;
-    typename RG<T>::frag xnext[RB][STEPS];
+    typename RG<T, KIN>::frag xnext[RB][STEPS];
     load(min(t + stride, ntiles - 1), xnext);
     // ROWS orientation: key j0 + RUN g + 4 rb + e is inside the row
     const auto valid = [&](int rb, int e) { return j0 + RT::RUN * g + 4 * rb + e < N ? 1.0f : 0.0f; };
@@ -417,7 +426,7 @@ __global__ __launch_bounds__(64 * ATTN_PROJ_WAVES) void triattn_proj_k(const T* 
       if (R >= 4 * D) {  // triangle bias (16-row block, H valid rows)
         f4 acc[RB][1];
         zero_acc(acc);
-        mma_rows<T, RB, 1, true>(acc, x, wb, LDW);
+        mma_rows<T, RB, 1, true, KIN>(acc, x, wb, LDW);
         if (r < H) {
 #pragma unroll
           for (int rb = 0; rb < RB; rb++) {
@@ -429,7 +438,7 @@ __global__ __launch_bounds__(64 * ATTN_PROJ_WAVES) void triattn_proj_k(const T* 
       } else if (R >= 2 * D && R < 3 * D) {  // v
         f4 acc[RB][2];
         zero_acc(acc);
-        mma_rows_grouped<T, RB, 2, 1, true>(acc, x, wb, LDW);
+        mma_rows_grouped<T, RB, 2, 1, true, KIN>(acc, x, wb, LDW);
 #pragma unroll
         for (int c = 0; c < 2; c++) {
           const int ch = R - 2 * D + 16 * c + r, h = ch / C, d = ch - h * C;
@@ -443,7 +452,7 @@ __global__ __launch_bounds__(64 * ATTN_PROJ_WAVES) void triattn_proj_k(const T* 
       } else {  // q, k, g
         f4 acc[RB][2];
         zero_acc(acc);
-        mma_rows_grouped<T, RB, 2, 1, false>(acc, x, wb, LDW);
+        mma_rows_grouped<T, RB, 2, 1, false, KIN>(acc, x, wb, LDW);
         const int P = R / D, within = R - P * D + 8 * g, h = within / C, d = within - h * C;
         const int64_t plane = (int64_t)(P == 3 ? 2 : P) * H + h;
         const float sc = P == 0 ? q_scale : 1.0f;
@@ -470,7 +479,7 @@ __global__ __launch_bounds__(64 * ATTN_PROJ_WAVES) void triattn_proj_k(const T* 
 // barriers. The rows and residual rows of the wave's next tile are loaded a whole tile ahead (one HBM round trip is
 // longer than the compute of the waves sharing a SIMD). On a wave's last tile the clamped "next" tile may be another
 // wave's; those loads are never used.
-template <typename T>
+template <typename T, int DO>
 __global__ __launch_bounds__(256, sizeof(T) == 2 ? 3 : 2) void linear_resid_ln_k(const T* __restrict__ x_in,
                                                                                 const T* __restrict__ w, int trans,
                                                                                 float* __restrict__ z, int accumulate,
@@ -478,11 +487,11 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 3 : 2) void linear_resid_ln_k
                                                                                 const float* __restrict__ lnb,
                                                                                 float eps, T* __restrict__ xn_next,
                                                                                 int64_t N) {
-  constexpr int STEPS = RG<T>::STEPS, LDW = ldw_of<T>();
-  __shared__ LDS_ALIGN T Ws[D * LDW];
+  constexpr int STEPS = RG<T>::STEPS, LDW = ldw_of<T>(), CB = DO / 16;
+  __shared__ LDS_ALIGN T Ws[DO * LDW];
   __shared__ LnLds lns;
-  lds_rows<T>(Ws, LDW, D, D, [&](int r) { return w + (int64_t)r * D; });
-  stage_ln(lns, lnw, lnb);
+  lds_rows<T>(Ws, LDW, DO, D, [&](int r) { return w + (int64_t)r * D; });
+  stage_ln(lns, lnw, lnb, DO);
   __syncthreads();
   const float* lw = lnw != nullptr ? lns.w : nullptr;
   const int64_t NN = N * N;
@@ -496,27 +505,27 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 3 : 2) void linear_resid_ln_k
     if (trans) { const int64_t a = p / N; p = (p - a * N) * N + a; }
     return p;
   };
-  const auto load = [&](int tt, typename RG<T>::frag (&xx)[1][STEPS], f4 (&zz)[1][8]) {
+  const auto load = [&](int tt, typename RG<T>::frag (&xx)[1][STEPS], f4 (&zz)[1][CB]) {
     RG<T>::load_row(xx[0], x_in + min((int64_t)tt * 16 + (l & 15), NN - 1) * D, g);
     const int64_t zr = zrow_of(tt);
     load_z_rows<1>(zz, [&](int) { return zr; }, z, accumulate);
   };
   typename RG<T>::frag x[1][STEPS];
-  f4 zv[1][8];
+  f4 zv[1][CB];
   load(t, x, zv);
   for (; t < ntiles; t += stride) {
     typename RG<T>::frag xnext[1][STEPS];
-    f4 znext[1][8];
+    f4 znext[1][CB];
     load(min(t + stride, ntiles - 1), xnext, znext);
-    f4 y[1][8];
+    f4 y[1][CB];
     zero_acc(y);
-    mma_rows_grouped<T, 1, 8, 2>(y, x, Ws, LDW);
+    mma_rows_grouped<T, 1, CB, 2>(y, x, Ws, LDW);
     const int64_t zr = zrow_of(t);
     resid_ln_apply<T, 1>(y, zv, [&](int) { return zr; }, z, lw, lns.b, eps, xn_next);
 #pragma unroll
     for (int s = 0; s < STEPS; s++) x[0][s] = xnext[0][s];
 #pragma unroll
-    for (int cb = 0; cb < 8; cb++) zv[0][cb] = znext[0][cb];
+    for (int cb = 0; cb < CB; cb++) zv[0][cb] = znext[0][cb];
   }
 }
 
@@ -852,14 +861,14 @@ __global__ __launch_bounds__(64 * TRW, 8 / TRW) void transition_f16_k(const half
 
 // ---------------------------------------------------------------- launchers
 
-template <typename T, int HV>
+template <typename T, int HV, int KIN>
 static hipError_t tm_proj_hv(const void* xn, const void* w, const float* mask, float scale, int incoming, void* ab,
                              int64_t N, int64_t ld, int resident, hipStream_t st) {
   const int64_t ntiles = N * (ld / (HV * RunTile<T>::TW));  // ld is a multiple of 64
   if (ntiles >= (1LL << 30)) return hipErrorInvalidValue;  // tile indices are 32-bit in the kernel
   const dim3 grid((unsigned)std::min<int64_t>(resident, (ntiles + PROJ_WAVES - 1) / PROJ_WAVES));
-  for (int c_lo = 0; c_lo < 2 * D; c_lo += proj_ch<T>()) {
-    trimul_proj_k<T, HV><<<grid, 64 * PROJ_WAVES, 0, st>>>(static_cast<const T*>(xn), static_cast<const T*>(w), mask,
+  for (int c_lo = 0; c_lo < 2 * KIN; c_lo += proj_ch<T, KIN>()) {
+    trimul_proj_k<T, HV, KIN><<<grid, 64 * PROJ_WAVES, 0, st>>>(static_cast<const T*>(xn), static_cast<const T*>(w), mask,
                                                           scale, incoming, static_cast<T*>(ab), N, ld, c_lo);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -867,80 +876,95 @@ static hipError_t tm_proj_hv(const void* xn, const void* w, const float* mask, f
   return hipSuccess;
 }
 
-template <typename T>
+template <typename T, int KIN>
 static hipError_t tm_proj(const void* xn, const void* w, const float* mask, float scale, int incoming, void* ab,
                           int64_t N, int64_t ld, hipStream_t st) {
   static int cache[kMaxDevices];
   // both tile forms have the same resources (the LDS weights and 8 waves set the occupancy)
-  const int resident = resident_grid(trimul_proj_k<T, 2>, 64 * PROJ_WAVES, cache);
+  const int resident = resident_grid(trimul_proj_k<T, 2, KIN>, 64 * PROJ_WAVES, cache);
   if (resident <= 0) return hipErrorInvalidDevice;
   // rounds of full tiles on the resident waves, against rounds of half tiles (counted in full tiles, with 10% for
   // the half tile's own overhead)
   const int64_t waves = (int64_t)resident * PROJ_WAVES, full = N * (ld / (2 * RunTile<T>::TW));
   const int64_t r2 = (full + waves - 1) / waves, r1x2 = (2 * full + waves - 1) / waves;
-  return 10 * r1x2 < 18 * r2 ? tm_proj_hv<T, 1>(xn, w, mask, scale, incoming, ab, N, ld, resident, st)
-                             : tm_proj_hv<T, 2>(xn, w, mask, scale, incoming, ab, N, ld, resident, st);
+  return 10 * r1x2 < 18 * r2 ? tm_proj_hv<T, 1, KIN>(xn, w, mask, scale, incoming, ab, N, ld, resident, st)
+                             : tm_proj_hv<T, 2, KIN>(xn, w, mask, scale, incoming, ab, N, ld, resident, st);
 }
 
 hipError_t launch_trimul_proj(const void* xn, const void* w, const float* mask, float scale, int incoming, void* ab,
-                              int dt, int64_t N, int64_t ld, hipStream_t st) {
-  return dt == DT_F16 ? tm_proj<half_t>(xn, w, mask, scale, incoming, ab, N, ld, st)
-                      : tm_proj<float>(xn, w, mask, scale, incoming, ab, N, ld, st);
+                              int dt, int64_t N, int64_t ld, int dim, hipStream_t st) {
+  if (dim == 64)
+    return dt == DT_F16 ? tm_proj<half_t, 64>(xn, w, mask, scale, incoming, ab, N, ld, st)
+                        : tm_proj<float, 64>(xn, w, mask, scale, incoming, ab, N, ld, st);
+  return dt == DT_F16 ? tm_proj<half_t, D>(xn, w, mask, scale, incoming, ab, N, ld, st)
+                      : tm_proj<float, D>(xn, w, mask, scale, incoming, ab, N, ld, st);
 }
 
-template <typename T>
+template <typename T, int KIN>
 static hipError_t tm_tail(const void* o, const float* now, const float* nob, float eps_out, const void* w_po,
                           const void* xn, const void* w_go, float* z, int accumulate, const float* lnw,
                           const float* lnb, float eps_next, void* xn_next, int64_t N, int64_t ld, hipStream_t st) {
   constexpr int TM = 64 * RowBlocks<T>::v;
   const dim3 grid((unsigned)(N * ((ld + TM - 1) / TM)));
-  trimul_tail_k<T><<<grid, 256, 0, st>>>(static_cast<const T*>(o), now, nob, eps_out, static_cast<const T*>(w_po),
+  trimul_tail_k<T, KIN><<<grid, 256, 0, st>>>(static_cast<const T*>(o), now, nob, eps_out, static_cast<const T*>(w_po),
                                          static_cast<const T*>(xn), static_cast<const T*>(w_go), z, accumulate, lnw,
                                          lnb, eps_next, static_cast<T*>(xn_next), N, ld);
   return hipGetLastError();
 }
 
+template <int KIN>
 static hipError_t tm_tail_f16(const void* o, const float* now, const float* nob, float eps_out, const void* w_po,
                               const void* xn, const void* w_go, float* z, int accumulate, const float* lnw,
                               const float* lnb, float eps_next, void* xn_next, int64_t N, int64_t ld, hipStream_t st) {
   static int cache[kMaxDevices];
-  const int resident = resident_grid(trimul_tail_f16_k, 64 * TAIL_WAVES, cache);
+  const int resident = resident_grid(trimul_tail_f16_k<KIN>, 64 * TAIL_WAVES, cache);
   if (resident <= 0) return hipErrorInvalidDevice;
   const int64_t ntiles = N * tail_tiles_per_row(N);  // the last tile of a row ends at ld (ld = N rounded up to 64)
   if (ntiles >= (1LL << 30)) return hipErrorInvalidValue;  // tile indices are 32-bit in the kernel
   const dim3 grid((unsigned)std::min<int64_t>(resident, (ntiles + TAIL_WAVES - 1) / TAIL_WAVES));
-  trimul_tail_f16_k<<<grid, 64 * TAIL_WAVES, 0, st>>>(static_cast<const half_t*>(o), now, nob, eps_out,
+  trimul_tail_f16_k<KIN><<<grid, 64 * TAIL_WAVES, 0, st>>>(static_cast<const half_t*>(o), now, nob, eps_out,
                                                       static_cast<const half_t*>(w_po), static_cast<const half_t*>(xn),
                                                       static_cast<const half_t*>(w_go), z, accumulate, lnw, lnb,
                                                       eps_next, static_cast<half_t*>(xn_next), N, ld);
   return hipGetLastError();
 }
 
-hipError_t launch_trimul_tail(const void* o, const float* now, const float* nob, float eps_out, const void* w_po,
-                              const void* xn, const void* w_go, float* z, int accumulate, const float* lnw,
-                              const float* lnb, float eps_next, void* xn_next, int dt, int64_t N, int64_t ld,
-                              hipStream_t st) {
-  if (dt == DT_F16 && (int64_t)D * N * ld < (1LL << 31))
-    return tm_tail_f16(o, now, nob, eps_out, w_po, xn, w_go, z, accumulate, lnw, lnb, eps_next, xn_next, N, ld, st);
-  return dt == DT_F16 ? tm_tail<half_t>(o, now, nob, eps_out, w_po, xn, w_go, z, accumulate, lnw, lnb, eps_next,
-                                        xn_next, N, ld, st)
-                      : tm_tail<float>(o, now, nob, eps_out, w_po, xn, w_go, z, accumulate, lnw, lnb, eps_next,
-                                       xn_next, N, ld, st);
+template <int KIN>
+static hipError_t tm_tail_c(const void* o, const float* now, const float* nob, float eps_out, const void* w_po,
+                            const void* xn, const void* w_go, float* z, int accumulate, const float* lnw,
+                            const float* lnb, float eps_next, void* xn_next, int dt, int64_t N, int64_t ld,
+                            hipStream_t st) {
+  if (dt == DT_F16 && (int64_t)KIN * N * ld < (1LL << 31))
+    return tm_tail_f16<KIN>(o, now, nob, eps_out, w_po, xn, w_go, z, accumulate, lnw, lnb, eps_next, xn_next, N, ld,
+                            st);
+  return dt == DT_F16 ? tm_tail<half_t, KIN>(o, now, nob, eps_out, w_po, xn, w_go, z, accumulate, lnw, lnb, eps_next,
+                                             xn_next, N, ld, st)
+                      : tm_tail<float, KIN>(o, now, nob, eps_out, w_po, xn, w_go, z, accumulate, lnw, lnb, eps_next,
+                                            xn_next, N, ld, st);
 }
 
-template <typename T>
+hipError_t launch_trimul_tail(const void* o, const float* now, const float* nob, float eps_out, const void* w_po,
+                              const void* xn, const void* w_go, float* z, int accumulate, const float* lnw,
+                              const float* lnb, float eps_next, void* xn_next, int dt, int64_t N, int64_t ld, int dim,
+                              hipStream_t st) {
+  return (dim == 64 ? tm_tail_c<64> : tm_tail_c<D>)(o, now, nob, eps_out, w_po, xn, w_go, z, accumulate, lnw, lnb,
+                                                    eps_next, xn_next, dt, N, ld, st);
+}
+
+template <typename T, int KIN>
 static hipError_t ta_proj(const void* xn, const void* w, int trans, float q_scale, float b_scale, void* qkg, void* vt,
                           void* tb, int64_t N, int64_t ldk, int H, int C, hipStream_t st) {
   if (H * C != D || H > 16 || C % 8) return hipErrorInvalidValue;
   static int cache[kMaxDevices];
-  const int resident = resident_grid(triattn_proj_k<T>, 64 * ATTN_PROJ_WAVES, cache);
+  const int resident = resident_grid(triattn_proj_k<T, KIN>, 64 * ATTN_PROJ_WAVES, cache);
   if (resident <= 0) return hipErrorInvalidDevice;
   const int64_t ntiles = N * (ldk / RunTile<T>::TW);  // ldk is a multiple of 64
   if (ntiles >= (1LL << 30)) return hipErrorInvalidValue;  // tile indices are 32-bit in the kernel
   const dim3 grid((unsigned)std::min<int64_t>(resident, (ntiles + ATTN_PROJ_WAVES - 1) / ATTN_PROJ_WAVES));
-  const int bounds[3] = {0, sizeof(T) == 2 ? 4 * D + 16 : 2 * D, 4 * D + 16};
-  for (int p = 0; p < (sizeof(T) == 2 ? 1 : 2); p++) {
-    triattn_proj_k<T><<<grid, 64 * ATTN_PROJ_WAVES, 0, st>>>(
+  constexpr bool ONE = attn_rows<T, KIN>() == 4 * D + 16;  // every row staged in one launch
+  const int bounds[3] = {0, ONE ? 4 * D + 16 : 2 * D, 4 * D + 16};
+  for (int p = 0; p < (ONE ? 1 : 2); p++) {
+    triattn_proj_k<T, KIN><<<grid, 64 * ATTN_PROJ_WAVES, 0, st>>>(
         static_cast<const T*>(xn), static_cast<const T*>(w), trans, q_scale, b_scale, static_cast<T*>(qkg),
         static_cast<T*>(vt), static_cast<T*>(tb), N, ldk, H, C, bounds[p], bounds[p + 1]);
     const hipError_t e = hipGetLastError();
@@ -950,30 +974,37 @@ static hipError_t ta_proj(const void* xn, const void* w, int trans, float q_scal
 }
 
 hipError_t launch_triattn_proj(const void* xn, const void* w, int trans, float q_scale, float b_scale, void* qkg,
-                               void* vt, void* tb, int dt, int64_t N, int64_t ldk, int H, int C, hipStream_t st) {
-  return dt == DT_F16 ? ta_proj<half_t>(xn, w, trans, q_scale, b_scale, qkg, vt, tb, N, ldk, H, C, st)
-                      : ta_proj<float>(xn, w, trans, q_scale, b_scale, qkg, vt, tb, N, ldk, H, C, st);
+                               void* vt, void* tb, int dt, int64_t N, int64_t ldk, int dim, int H, int C,
+                               hipStream_t st) {
+  if (dim == 64)
+    return dt == DT_F16 ? ta_proj<half_t, 64>(xn, w, trans, q_scale, b_scale, qkg, vt, tb, N, ldk, H, C, st)
+                        : ta_proj<float, 64>(xn, w, trans, q_scale, b_scale, qkg, vt, tb, N, ldk, H, C, st);
+  return dt == DT_F16 ? ta_proj<half_t, D>(xn, w, trans, q_scale, b_scale, qkg, vt, tb, N, ldk, H, C, st)
+                      : ta_proj<float, D>(xn, w, trans, q_scale, b_scale, qkg, vt, tb, N, ldk, H, C, st);
 }
 
-template <typename T>
+template <typename T, int DO>
 static hipError_t lrl(const void* x, const void* w, int trans, float* z, int accumulate, const float* lnw,
                       const float* lnb, float eps, void* xn_next, int64_t N, hipStream_t st) {
   static int cache[kMaxDevices];
-  const int resident = resident_grid(linear_resid_ln_k<T>, 256, cache);
+  const int resident = resident_grid(linear_resid_ln_k<T, DO>, 256, cache);
   if (resident <= 0) return hipErrorInvalidDevice;
   const int64_t waves = (N * N + 15) / 16;
   if (waves >= (1LL << 30)) return hipErrorInvalidValue;  // tile indices are 32-bit in the kernel
   const dim3 grid((unsigned)std::min<int64_t>(resident, (waves + 3) / 4));
-  linear_resid_ln_k<T><<<grid, 256, 0, st>>>(static_cast<const T*>(x), static_cast<const T*>(w), trans, z, accumulate,
+  linear_resid_ln_k<T, DO><<<grid, 256, 0, st>>>(static_cast<const T*>(x), static_cast<const T*>(w), trans, z, accumulate,
                                              lnw, lnb, eps, static_cast<T*>(xn_next), N);
   return hipGetLastError();
 }
 
 hipError_t launch_linear_resid_ln(const void* x, const void* w, int trans, float* z, int accumulate,
                                   const float* lnw, const float* lnb, float eps, void* xn_next, int dt, int64_t N,
-                                  hipStream_t st) {
-  return dt == DT_F16 ? lrl<half_t>(x, w, trans, z, accumulate, lnw, lnb, eps, xn_next, N, st)
-                      : lrl<float>(x, w, trans, z, accumulate, lnw, lnb, eps, xn_next, N, st);
+                                  int dim, hipStream_t st) {
+  if (dim == 64)
+    return dt == DT_F16 ? lrl<half_t, 64>(x, w, trans, z, accumulate, lnw, lnb, eps, xn_next, N, st)
+                        : lrl<float, 64>(x, w, trans, z, accumulate, lnw, lnb, eps, xn_next, N, st);
+  return dt == DT_F16 ? lrl<half_t, D>(x, w, trans, z, accumulate, lnw, lnb, eps, xn_next, N, st)
+                      : lrl<float, D>(x, w, trans, z, accumulate, lnw, lnb, eps, xn_next, N, st);
 }
 
 template <typename T, int HCH>

@@ -1,46 +1,37 @@
-// Transposed row-tile GEMM building blocks for the pair kernels (K = 128 input channels per row).
+// Transposed row-tile GEMM building blocks for the pair kernels (K = 128 or 64 input channels per row).
 //
 // The kernels compute Y^T = W X^T on MFMA: A = a 16-row block of the weight W (output channels, K-contiguous, staged
 // in LDS), B = X^T for 16 rows of X (positions, K-contiguous, loaded once per tile straight from global memory into
 // registers). The accumulator then holds, per lane l, row l % 16 of X and the 4 consecutive output channels
 // 16*cb + 4*(l/16) + e, e = 0..3: every row lives in 4 lanes (l, l^16, l^32, l^48), so row-wise epilogues (residual
 // add, LayerNorm) need two cross-lane steps, and each lane writes 4 contiguous outputs.
-// K is split in lane-group blocks: MFMA step s of lane group g = l/16 takes k = 32*g + s*KP + t (t < KP), which is a
-// permutation of the sum over k shared by A and B, so a lane reads 32 contiguous channels of its row.
+// K is split in lane-group blocks: MFMA step s of lane group g = l/16 takes k = (K/4)*g + s*KP + t (t < KP), which is a
+// permutation of the sum over k shared by A and B, so a lane reads K/4 contiguous channels of its row.
 #pragma once
 
 #include "bzpf_common.h"
 
 namespace bzpf {
 
-template <typename T> struct RG;
-template <> struct RG<half_t> {
-  static constexpr int STEPS = 4;  // MFMA steps over K = 128
+// KIN input channels per row (128, or 64: the template stack), lane group g reading the KIN / 4 from (KIN / 4) g on.
+template <typename T, int KIN = 128> struct RG;
+template <int KIN> struct RG<half_t, KIN> {
+  static constexpr int STEPS = KIN / 32;  // MFMA steps over K
   typedef half8 frag;
   __device__ static __forceinline__ void load_row(frag (&f)[STEPS], const half_t* p, int g) {
 #pragma unroll
-    for (int s = 0; s < STEPS; s++) f[s] = *reinterpret_cast<const half8*>(p + 32 * g + 8 * s);
-  }
-  __device__ static __forceinline__ void zero(frag (&f)[STEPS]) {
-#pragma unroll
-    for (int s = 0; s < STEPS; s++)
-#pragma unroll
-      for (int t = 0; t < 8; t++) f[s][t] = (half_t)0.0f;
+    for (int s = 0; s < STEPS; s++) f[s] = *reinterpret_cast<const half8*>(p + KIN / 4 * g + 8 * s);
   }
 };
-template <> struct RG<float> {
-  static constexpr int STEPS = 32;
+template <int KIN> struct RG<float, KIN> {
+  static constexpr int STEPS = KIN / 4;
   typedef float frag;
   __device__ static __forceinline__ void load_row(frag (&f)[STEPS], const float* p, int g) {
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const f4 v = *reinterpret_cast<const f4*>(p + 32 * g + 4 * j);
+    for (int j = 0; j < KIN / 16; j++) {
+      const f4 v = *reinterpret_cast<const f4*>(p + KIN / 4 * g + 4 * j);
       f[4 * j] = v[0]; f[4 * j + 1] = v[1]; f[4 * j + 2] = v[2]; f[4 * j + 3] = v[3];
     }
-  }
-  __device__ static __forceinline__ void zero(frag (&f)[STEPS]) {
-#pragma unroll
-    for (int s = 0; s < STEPS; s++) f[s] = 0.0f;
   }
 };
 
@@ -52,16 +43,16 @@ template <typename T> struct RowBlocks { static constexpr int v = sizeof(T) == 2
 // layouts of the MFMA are mirror images (lane l holds 8 k-consecutive elements of row/column l % 16), so swapping
 // the operands swaps the accumulator layout. Then lane l holds rows (positions) 4 (l/16) + e of block rb and output
 // channel 16 cb + l % 16: position-contiguous runs, for outputs stored channel-major.
-template <typename T, int RB, int CB, bool ROWS = false>
-__device__ __forceinline__ void mma_rows(f4 (&acc)[RB][CB], const typename RG<T>::frag (&x)[RB][RG<T>::STEPS],
+template <typename T, int RB, int CB, bool ROWS = false, int KIN = 128>
+__device__ __forceinline__ void mma_rows(f4 (&acc)[RB][CB], const typename RG<T, KIN>::frag (&x)[RB][RG<T, KIN>::STEPS],
                                          const T* Ws, int ldw) {
   const int l = threadIdx.x & 63, g = l >> 4;
 #pragma unroll
   for (int cb = 0; cb < CB; cb++) {
-    const T* wp = Ws + (16 * cb + (l & 15)) * ldw + 32 * g;
+    const T* wp = Ws + (16 * cb + (l & 15)) * ldw + KIN / 4 * g;
     if constexpr (sizeof(T) == 2) {
 #pragma unroll
-      for (int s = 0; s < 4; s++) {
+      for (int s = 0; s < KIN / 32; s++) {
         const half8 a = *reinterpret_cast<const half8*>(wp + 8 * s);
 #pragma unroll
         for (int rb = 0; rb < RB; rb++)
@@ -70,7 +61,7 @@ __device__ __forceinline__ void mma_rows(f4 (&acc)[RB][CB], const typename RG<T>
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
+      for (int j = 0; j < KIN / 16; j++) {
         const f4 a = *reinterpret_cast<const f4*>(wp + 4 * j);
 #pragma unroll
         for (int t = 0; t < 4; t++)
@@ -116,8 +107,9 @@ __device__ __forceinline__ void st_run_cached(float* p, const float (&v)[4]) {
 
 // mma_rows over CB column blocks in groups of G with a scheduling barrier between groups: the compiler otherwise
 // hoists every LDS weight read ahead of the MFMAs (CB * 4 fragments live at once), which spills at 4 waves/SIMD.
-template <typename T, int RB, int CB, int G, bool ROWS = false>
-__device__ __forceinline__ void mma_rows_grouped(f4 (&acc)[RB][CB], const typename RG<T>::frag (&x)[RB][RG<T>::STEPS],
+template <typename T, int RB, int CB, int G, bool ROWS = false, int KIN = 128>
+__device__ __forceinline__ void mma_rows_grouped(f4 (&acc)[RB][CB],
+                                                 const typename RG<T, KIN>::frag (&x)[RB][RG<T, KIN>::STEPS],
                                                  const T* Ws, int ldw) {
   static_assert(CB % G == 0, "column blocks must split into groups");
 #pragma unroll
@@ -127,7 +119,7 @@ __device__ __forceinline__ void mma_rows_grouped(f4 (&acc)[RB][CB], const typena
     for (int rb = 0; rb < RB; rb++)
 #pragma unroll
       for (int c = 0; c < G; c++) part[rb][c] = acc[rb][G * q + c];
-    mma_rows<T, RB, G, ROWS>(part, x, Ws + 16 * G * q * ldw, ldw);
+    mma_rows<T, RB, G, ROWS, KIN>(part, x, Ws + 16 * G * q * ldw, ldw);
 #pragma unroll
     for (int rb = 0; rb < RB; rb++)
 #pragma unroll
@@ -161,9 +153,10 @@ struct LnLds {
   float w[128];
   float b[128];
 };
-__device__ __forceinline__ void stage_ln(LnLds& s, const float* __restrict__ w, const float* __restrict__ b) {
+__device__ __forceinline__ void stage_ln(LnLds& s, const float* __restrict__ w, const float* __restrict__ b,
+                                         int n = 128) {
   if (w == nullptr) return;
-  for (int c = threadIdx.x; c < 128; c += blockDim.x) {
+  for (int c = threadIdx.x; c < n; c += blockDim.x) {
     s.w[c] = w[c];
     s.b[c] = b[c];
   }
@@ -184,28 +177,28 @@ __device__ __forceinline__ void st4(half_t* p, f4 v) {
 // row); zeros where accumulate == 0. A lane with no row (zrow < 0) loads row 0 instead: its values only enter the
 // reductions of its own row, which is never stored, and the loads stay unconditional (no per-lane branches).
 // Issued ahead of the MFMAs so the loads overlap them.
-template <int RB, typename ZRow>
-__device__ __forceinline__ void load_z_rows(f4 (&zv)[RB][8], ZRow zrow, const float* __restrict__ z, int accumulate) {
-  constexpr int D = 128;
+template <int RB, typename ZRow, int CB>
+__device__ __forceinline__ void load_z_rows(f4 (&zv)[RB][CB], ZRow zrow, const float* __restrict__ z, int accumulate) {
+  constexpr int D = 16 * CB;
   const int g = (threadIdx.x & 63) >> 4;
 #pragma unroll
   for (int rb = 0; rb < RB; rb++) {
     const int64_t zr = zrow(rb);
     const float* zp = z + (zr >= 0 ? zr : 0) * D + 4 * g;  // one row base; column blocks are immediate offsets
 #pragma unroll
-    for (int cb = 0; cb < 8; cb++) zv[rb][cb] = accumulate ? ld4(zp + 16 * cb) : f4{0.f, 0.f, 0.f, 0.f};
+    for (int cb = 0; cb < CB; cb++) zv[rb][cb] = accumulate ? ld4(zp + 16 * cb) : f4{0.f, 0.f, 0.f, 0.f};
   }
 }
 
-// Residual + LayerNorm epilogue on the transposed accumulator of 8 column blocks (D = 128 channels): for each of the
+// Residual + LayerNorm epilogue on the transposed accumulator of CB column blocks (D = 16 CB channels): for each of the
 // lane's rows, z[zr] = zv + y, then xn_next[zr] = LN(z[zr]) when lnw != nullptr. zrow(rb) returns the z row of the
 // lane's row in block rb (< 0: no row; the lane still joins the cross-lane reductions, which only mix the 4 lanes
 // of one row, and stores nothing).
-template <typename TO, int RB, typename ZRow>
-__device__ __forceinline__ void resid_ln_apply(const f4 (&y)[RB][8], const f4 (&zv)[RB][8], ZRow zrow,
+template <typename TO, int RB, typename ZRow, int CB>
+__device__ __forceinline__ void resid_ln_apply(const f4 (&y)[RB][CB], const f4 (&zv)[RB][CB], ZRow zrow,
                                                float* __restrict__ z, const float* __restrict__ lnw,
                                                const float* __restrict__ lnb, float eps, TO* __restrict__ xn_next) {
-  constexpr int D = 128;
+  constexpr int D = 16 * CB;
   const int l = threadIdx.x & 63, g = l >> 4;
 #pragma unroll
   for (int rb = 0; rb < RB; rb++) {
@@ -213,22 +206,22 @@ __device__ __forceinline__ void resid_ln_apply(const f4 (&y)[RB][8], const f4 (&
     // one row base per pointer; the column blocks 16 cb are immediate offsets (no per-block 64-bit addresses)
     const int64_t rowoff = (zr >= 0 ? zr : 0) * D + 4 * g;
     float* zp = z + rowoff;
-    f4 v[8];
+    f4 v[CB];
     float s = 0.f;
 #pragma unroll
-    for (int cb = 0; cb < 8; cb++) {
+    for (int cb = 0; cb < CB; cb++) {
       v[cb] = y[rb][cb] + zv[rb][cb];
       s += v[cb][0] + v[cb][1] + v[cb][2] + v[cb][3];
     }
     if (zr >= 0) {
 #pragma unroll
-      for (int cb = 0; cb < 8; cb++) __builtin_nontemporal_store(v[cb], reinterpret_cast<f4*>(zp + 16 * cb));
+      for (int cb = 0; cb < CB; cb++) __builtin_nontemporal_store(v[cb], reinterpret_cast<f4*>(zp + 16 * cb));
     }
     if (lnw == nullptr) continue;
     const float mean = xgroups_sum(s) * (1.0f / D);
     float ss = 0.f;
 #pragma unroll
-    for (int cb = 0; cb < 8; cb++) {
+    for (int cb = 0; cb < CB; cb++) {
       const f4 d = v[cb] - mean;
       ss += d[0] * d[0] + d[1] * d[1] + d[2] * d[2] + d[3] * d[3];
     }
@@ -236,7 +229,7 @@ __device__ __forceinline__ void resid_ln_apply(const f4 (&y)[RB][8], const f4 (&
     if (zr < 0) continue;
     TO* xp = xn_next + rowoff;
 #pragma unroll
-    for (int cb = 0; cb < 8; cb++) {
+    for (int cb = 0; cb < CB; cb++) {
       const int c = 16 * cb + 4 * g;
       st4(xp + 16 * cb, (v[cb] - mean) * rstd * ld4(lnw + c) + ld4(lnb + c));
     }
@@ -244,11 +237,11 @@ __device__ __forceinline__ void resid_ln_apply(const f4 (&y)[RB][8], const f4 (&
 }
 
 // z[zr] = (accumulate ? z[zr] : 0) + y, then the next LayerNorm (resid_ln_apply with the residual loaded in place).
-template <typename TO, int RB, typename ZRow>
-__device__ __forceinline__ void resid_ln_rows(const f4 (&y)[RB][8], ZRow zrow, float* __restrict__ z, int accumulate,
+template <typename TO, int RB, typename ZRow, int CB>
+__device__ __forceinline__ void resid_ln_rows(const f4 (&y)[RB][CB], ZRow zrow, float* __restrict__ z, int accumulate,
                                               const float* __restrict__ lnw, const float* __restrict__ lnb, float eps,
                                               TO* __restrict__ xn_next) {
-  f4 zv[RB][8];
+  f4 zv[RB][CB];
   load_z_rows<RB>(zv, zrow, z, accumulate);
   resid_ln_apply<TO, RB>(y, zv, zrow, z, lnw, lnb, eps, xn_next);
 }

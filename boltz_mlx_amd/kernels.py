@@ -229,6 +229,67 @@ def trimul_proj(xn, w_pg, mask, scale: float, incoming: bool, N: int) -> torch.T
     return ab
 
 
+def trimul_proj64(xn, w_pg, mask, scale: float, incoming: bool, N: int) -> torch.Tensor:
+    """trimul_proj for 64 channels: xn [N*N, 64], w_pg [256, 64] -> ab [128, N, ld]."""
+    _dev(xn, w_pg, mask)
+    if mask.dtype != torch.float32 or mask.numel() != N * N or w_pg.shape != (256, 64) or w_pg.dtype != xn.dtype \
+            or xn.numel() != N * N * 64:
+        raise ValueError("trimul_proj64: need xn [N*N, 64], w_pg [256, 64] of one dtype and an fp32 mask [N, N]")
+    ld = row_pitch(N)
+    ab = torch.empty((128, N, ld), dtype=xn.dtype, device=xn.device)
+    call("bzpf_trimul_proj64", _p(xn), _p(w_pg), _p(mask), float(scale), int(incoming), _p(ab), _dt(xn), N, ld,
+         _stream())
+    return ab
+
+
+def trimul_tail64(o, norm_out, eps_out: float, w_po, xn, w_go, z, accumulate: bool, next_ln=None, N: int = 0):
+    """trimul_tail for 64 channels: o [64, N, ld], w_po and w_go [64, 64], xn [N*N, 64], z [N, N, 64]."""
+    _dev(o, w_po, xn, w_go, z)
+    ld = row_pitch(N)
+    if z.dtype != torch.float32 or z.numel() != N * N * 64 or o.shape != (64, N, ld) or xn.numel() != N * N * 64 \
+            or w_po.shape != (64, 64) or w_go.shape != (64, 64) \
+            or not (o.dtype == w_po.dtype == w_go.dtype == xn.dtype):
+        raise ValueError("trimul_tail64: shape/dtype mismatch")
+    nxt = nw = nb = None
+    neps = 1e-5
+    if next_ln is not None:
+        nxt = torch.empty((N * N, 64), dtype=xn.dtype, device=xn.device)
+        nw, nb, neps = f32c(next_ln.weight), f32c(next_ln.bias), next_ln.eps
+    call("bzpf_trimul_tail64", _p(o), _p(f32c(norm_out.weight)), _p(f32c(norm_out.bias)), float(eps_out), _p(w_po),
+         _p(xn), _p(w_go), _p(z), int(accumulate), _p(nw), _p(nb), float(neps), _p(nxt), _dt(xn), N, ld, _stream())
+    return nxt
+
+
+def triattn_proj64(xn, w, trans: bool, N: int, H: int, C: int):
+    """triattn_proj for 64 input channels (H * C = 128): xn [N*N, 64], w [4HC + H, 64]."""
+    _dev(xn, w)
+    if H * C != 128 or w.shape != (4 * H * C + H, 64) or w.dtype != xn.dtype or xn.numel() != N * N * 64:
+        raise ValueError("triattn_proj64: need xn [N*N, 64] and w [4HC + H, 64] of one dtype with H * C = 128")
+    ldk = row_pitch(N)
+    qkg = torch.empty((3 * H, N * N, C), dtype=xn.dtype, device=xn.device)
+    vt = torch.empty((H, N, C, ldk), dtype=xn.dtype, device=xn.device)
+    tb = torch.empty((tri_bias_numel(N, H),), dtype=xn.dtype, device=xn.device)
+    call("bzpf_triattn_proj64", _p(xn), _p(w), int(trans), LOG2E / C ** 0.5, LOG2E, _p(qkg), _p(vt), _p(tb), _dt(xn),
+         N, ldk, H, C, _stream())
+    return qkg, vt, tb
+
+
+def linear_resid_ln64(x, w, trans: bool, z, accumulate: bool, next_ln=None, N: int = 0):
+    """linear_resid_ln into 64 channels: x [N*N, 128], w [64, 128], z [N, N, 64]."""
+    _dev(x, w, z)
+    if z.dtype != torch.float32 or z.numel() != N * N * 64 or x.numel() != N * N * 128 or w.shape != (64, 128) \
+            or w.dtype != x.dtype:
+        raise ValueError("linear_resid_ln64: shape/dtype mismatch")
+    nxt = nw = nb = None
+    neps = 1e-5
+    if next_ln is not None:
+        nxt = torch.empty((N * N, 64), dtype=x.dtype, device=x.device)
+        nw, nb, neps = f32c(next_ln.weight), f32c(next_ln.bias), next_ln.eps
+    call("bzpf_linear_resid_ln64", _p(x), _p(w), int(trans), _p(z), int(accumulate), _p(nw), _p(nb), float(neps),
+         _p(nxt), _dt(x), N, _stream())
+    return nxt
+
+
 def trimul_pack(P: torch.Tensor, mask: torch.Tensor, scale: float, incoming: bool, N: int) -> torch.Tensor:
     """ab [2D, N, ld] from P = xn [p_in; g_in]^T ([N*N, 4D]) at any D (the fused trimul_proj is built for 128)."""
     _dev(P, mask)

@@ -72,7 +72,14 @@ class TriangleAttention(torch.nn.Module):
         # the projection reads xn at the attention frame's position: transposed for the ending node unless the
         # caller already transposed it
         proj_trans = trans and not xn_transposed
-        if D != 128 or H * C != D:  # the fused projection / output kernels are built for 128 = H * C channels:
+        if D == 64 and H * C == 128:  # the template stack's widths
+            qkg, vt, tb = K.triattn_proj64(xn, w, proj_trans, N, H, C)
+            if before_core is not None:
+                before_core()
+            core = K.triattn_core(qkg, vt, tb, mask, trans, self.inf, N, H, C)
+            del qkg, vt, tb
+            return K.linear_resid_ln64(core, w_o, trans, z, accumulate, next_ln, N)
+        if D != 128 or H * C != D:  # the fused projection / output kernels are built for H * C = 128 channels:
             # otherwise GEMMs plus layout kernels (the core takes C = 16, 32 or 64)
             qkg, vt, tb = K.triattn_pack(K.linear(xn, w), proj_trans, N, H, C)
             if before_core is not None:

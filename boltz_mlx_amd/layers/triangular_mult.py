@@ -52,7 +52,11 @@ class _TriangleMultiplication(torch.nn.Module):
         N, D = z.shape[0], z.shape[-1]
         kexp = K.TRIMULT_K if K.f16() else 0
         w_pg, w_po, w_go = self.prepare()
-        if D != 128:  # the projection and tail kernels are built for 128 channels: GEMMs plus layout kernels
+        if D == 64:  # the template stack's width
+            o = K.trimul_contract(K.trimul_proj64(xn, w_pg, mask, 2.0 ** -kexp, not self.outgoing, N), N)
+            return K.trimul_tail64(o, self.norm_out, self.norm_out.eps * 2.0 ** (-4 * kexp), w_po, xn, w_go, z,
+                                   accumulate, next_ln, N)
+        if D != 128:  # the projection and tail kernels are built for 128 and 64 channels: GEMMs plus layout kernels
             ab = K.trimul_pack(K.linear(xn, w_pg), mask, 2.0 ** -kexp, not self.outgoing, N)
             o = K.trimul_contract(ab, N)
             del ab

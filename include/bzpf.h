@@ -220,6 +220,22 @@ int bzpf_seq_attention_batched(const void* q, const void* k, const void* v, cons
 int bzpf_trimul_pack(const void* P, const float* mask, float scale, int incoming, void* ab, int dt, int64_t N,
                      int64_t ld, int D, void* stream);
 
+/* The fused pair kernels at 64 channels (the template stack): bzpf_trimul_proj, bzpf_trimul_tail, bzpf_triattn_proj and
+ * bzpf_linear_resid_ln with 64 for D in every operand but the attention's H*C = 128 (bzpf_triattn_proj64 reads xn
+ * [N*N, 64] and w [4*H*C + H, 64]; bzpf_linear_resid_ln64 takes x [N*N, 128] and w [64, 128]); the fp16 tail keeps its
+ * gates in fp32. Same reference lines as the 128-channel forms (boltz_mlx/layers/triangular_mult.py:40-118,
+ * triangular_attention/attention.py:49-104). */
+int bzpf_trimul_proj64(const void* xn, const void* w_pg, const float* pair_mask, float scale, int incoming, void* ab,
+                       int dt, int64_t N, int64_t ld, void* stream);
+int bzpf_trimul_tail64(const void* o, const float* norm_out_w, const float* norm_out_b, float eps_out,
+                       const void* w_po, const void* xn, const void* w_go, float* z, int accumulate,
+                       const float* next_w, const float* next_b, float next_eps, void* xn_next, int dt, int64_t N,
+                       int64_t ld, void* stream);
+int bzpf_triattn_proj64(const void* xn, const void* w, int trans, float q_scale, float bias_scale, void* qkg, void* vt,
+                        void* tri_bias, int dt, int64_t N, int64_t ldk, int H, int C, void* stream);
+int bzpf_linear_resid_ln64(const void* x, const void* w, int trans, float* z, int accumulate, const float* next_w,
+                           const float* next_b, float next_eps, void* xn_next, int dt, int64_t N, void* stream);
+
 /* bzpf_channels_to_rows: out[i*N + j][c] = o[c][i][j] for o [D][N][ld] (the contraction output) -> out [N*N, D]
  * (dtypes independent), the operand of norm_out (boltz_mlx/layers/triangular_mult.py:93-98). D <= 252. */
 int bzpf_channels_to_rows(const void* o, int o_dt, void* out, int out_dt, int64_t N, int64_t ld, int D,
