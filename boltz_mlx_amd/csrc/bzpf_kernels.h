@@ -16,6 +16,22 @@ hipError_t launch_count_nonfinite(const void* x, int dt, int64_t n, int* count, 
 
 hipError_t launch_trimul_proj(const void* xn, const void* w, const float* mask, float scale, int incoming, void* ab,
                               int dt, int64_t N, int64_t ld, int dim, hipStream_t st);
+// The fp32 forms of the pair row kernels (bzpf_pair_x3.hip).
+hipError_t launch_trimul_proj_x3(const float* xn, const float* w, const float* mask, float scale, int incoming,
+                                 float* ab, int64_t N, int64_t ld, int dim, hipStream_t st);
+hipError_t launch_trimul_tail_x3(const float* o, const float* now, const float* nob, float eps_out, const float* w_po,
+                                 const float* xn, const float* w_go, float* z, int accumulate, const float* lnw,
+                                 const float* lnb, float eps_next, float* xn_next, int64_t N, int64_t ld, int dim,
+                                 hipStream_t st);
+hipError_t launch_triattn_proj_x3(const float* xn, const float* w, int trans, float q_scale, float b_scale, float* qkg,
+                                  float* vt, float* tb, int64_t N, int64_t ldk, int dim, int H, int C,
+                                  hipStream_t st);
+hipError_t launch_linear_resid_ln_x3(const float* x, const float* w, int trans, float* z, int accumulate,
+                                     const float* lnw, const float* lnb, float eps, float* xn_next, int64_t N, int dim,
+                                     hipStream_t st);
+hipError_t launch_transition_x3(const float* xn, const float* w12, const float* w3, float* z, int accumulate,
+                                const float* lnw, const float* lnb, float eps, float* xn_next, int64_t rows,
+                                int hidden, hipStream_t st);
 hipError_t launch_trimul_contract(const void* ab, void* o, int dt, int64_t N, int64_t ld, int64_t k_len, int D,
                                   hipStream_t st);
 hipError_t launch_trimul_tail(const void* o, const float* now, const float* nob, float eps_out, const void* w_po,

@@ -8,7 +8,7 @@
 //   linear_resid_ln  : z (+)= x W_o^T at the (transposed) position, then the next LayerNorm (kernels_nax3.py:176-198);
 //   transition       : z (+)= fc3(silu(fc1 xn) * fc2 xn), then the next LayerNorm (transition.py:27-54, 148-154;
 //                      kernels_nax2.py:54-190, kernels_nax3.py:713-827).
-// Tiles are 64 * RB rows (positions) per workgroup of 4 waves, RB = 2 row blocks per wave for fp16 and 1 for fp32.
+// These are the fp16 forms (two 16-row blocks per wave); the fp32 ones are in bzpf_pair_x3.hip.
 #include <type_traits>
 
 #include "bzpf_common.h"
@@ -24,29 +24,26 @@ constexpr int D = 128;
 template <typename T, int KIN = D> constexpr int ldw_of() { return KIN + Pad<T>::v; }
 
 // ---------------------------------------------------------------- triangle multiplication projection
-// Persistent, one 512-thread workgroup per CU (8 waves, up to 256 VGPRs each). The launch covers output channels
-// [c_lo, c_lo + PCH): the projection rows c_lo.. and gate rows 2D + c_lo.. of w (PCH = 256 in fp16: all of them;
-// 128 in fp32, two launches) are staged in LDS once; each wave then streams tiles of HV TW positions
+// Persistent, one 512-thread workgroup per CU (8 waves, up to 256 VGPRs each). The 2D projection and 2D gate rows of w
+// are staged in LDS once; each wave then streams tiles of HV TW positions
 // (i, k0 .. k0 + HV TW) over the padded rows of length ld as HV halves of TW, computing (ROWS orientation) one
 // 16-byte run per channel and half: with HV = 2 a whole 128-byte line of ab[c][i][k] (fp16) per channel row and
 // tile, written by one wave with two adjacent stores (incoming: xn read at (k, i)). The next tile's rows and mask
 // values are loaded while the current tile computes (8 waves with the prefetch measured 3-4% faster than 12
 // without). HV = 1 (half tiles) is taken when it balances the last round of tiles better: at N = 400 (2,800 full
 // tiles on 2,048 waves) 0.041-0.045 against 0.050 ms; at N = 1000 full tiles are faster (0.23 against 0.26 ms).
-template <typename T, int KIN = D> constexpr int proj_ch() { return sizeof(T) == 2 ? 2 * KIN : 128; }
 constexpr int PROJ_WAVES = 8;
 
 template <typename T, int HV, int KIN>
 __global__ __launch_bounds__(64 * PROJ_WAVES) void trimul_proj_k(const T* __restrict__ xn, const T* __restrict__ w,
                                                                  const float* __restrict__ mask, float scale,
                                                                  int incoming, T* __restrict__ ab, int64_t N,
-                                                                 int64_t ld, int c_lo) {
+                                                                 int64_t ld) {
   using RT = RunTile<T>;
   constexpr int D = KIN;
-  constexpr int RB = RT::RB, TW = RT::TW, STEPS = RG<T, D>::STEPS, LDW = ldw_of<T, D>(), PCH = proj_ch<T, D>();
+  constexpr int RB = RT::RB, TW = RT::TW, STEPS = RG<T, D>::STEPS, LDW = ldw_of<T, D>(), PCH = 2 * D;
   __shared__ LDS_ALIGN T Ws[2 * PCH * LDW];  // rows [0, PCH): projections, [PCH, 2 PCH): gates
-  lds_rows<T>(Ws, LDW, 2 * PCH, D,
-              [&](int r) { return w + (int64_t)(r < PCH ? c_lo + r : 2 * D + c_lo + r - PCH) * D; });
+  lds_rows<T>(Ws, LDW, 2 * PCH, D, [&](int r) { return w + (int64_t)r * D; });
   __syncthreads();
   const int l = threadIdx.x & 63, g = l >> 4, r = l & 15;
   const int tpr = (int)(ld / (HV * TW)), ntiles = (int)N * tpr, stride = gridDim.x * PROJ_WAVES;
@@ -85,7 +82,7 @@ __global__ __launch_bounds__(64 * PROJ_WAVES) void trimul_proj_k(const T* __rest
 #pragma unroll
         for (int e = 0; e < 4; e++) mo[hh][rb][e] = __shfl(mv, 4 * g + e);
       }
-    T* dst = ab + ((int64_t)(c_lo + r) * N + i) * ld + k0 + RT::RUN * g;
+    T* dst = ab + ((int64_t)r * N + i) * ld + k0 + RT::RUN * g;
     for (int cb = 0; cb < PCH / 16; cb++) {
 #pragma unroll
       for (int hh = 0; hh < HV; hh++) {
@@ -124,7 +121,7 @@ __global__ __launch_bounds__(256) void trimul_tail_k(const T* __restrict__ o, co
                                                      const float* __restrict__ lnw, const float* __restrict__ lnb,
                                                      float eps_next, T* __restrict__ xn_next, int64_t N, int64_t ld) {
   constexpr int D = KIN, NC = D / 64, QC = D / 4;  // 64-channel chunks, channels per LayerNorm thread
-  constexpr int RB = RowBlocks<T>::v, TM = 64 * RB, STEPS = RG<T, D>::STEPS, LDW = ldw_of<T, D>();
+  constexpr int RB = 2, TM = 64 * RB, STEPS = RG<T, D>::STEPS, LDW = ldw_of<T, D>();
   __shared__ LDS_ALIGN T Ts[TM * LDW];  // o tile transposed to [position][channel], then LN_out of it
   __shared__ LDS_ALIGN T Ws[64 * LDW];
   const int64_t tpr = (ld + TM - 1) / TM;
@@ -360,21 +357,14 @@ __global__ __launch_bounds__(64 * TAIL_WAVES) void trimul_tail_f16_k(
 
 // ---------------------------------------------------------------- triangle attention projection
 // Persistent like trimul_proj. Rows of w: q [0, D), k [D, 2D), v [2D, 3D), g [3D, 4D), triangle bias [4D, 4D + H)
-// (H * C = D). A launch stages the rows [r_lo, r_hi) of that list with the bias block padded to 16 zero rows
-// (fp16: all 4D + 16 rows; fp32: [0, 2D) and [2D, 4D + 16) in two launches). Each wave streams tiles of TW positions
+// (H * C = D), staged with the bias block padded to 16 rows by zeros. Each wave streams tiles of TW positions
 // (i, j0 .. j0 + TW) of the padded rows (length ldk), position (i, j) reading xn at (i, j) (trans: (j, i)):
 //   q, k, g : transposed orientation; the staging permutes each 32-row group (LDS row 32 m + 16 c + rr holds channel
 //             32 m + 8 (rr / 4) + 4 c + rr % 4), so the lane of group g holds channels 8 g .. 8 g + 7 of its position:
 //             one 16-byte run of qkg[plane][i N + j][:] (q scaled by q_scale);
 //   v       : ROWS orientation, 16-byte runs of keys of vt[h][i][d][:] (zeros past N);
 //   bias    : ROWS orientation, runs of 4 keys of the fragment-ordered bias (scaled by b_scale, zeros past N).
-template <typename T, int KIN> constexpr int attn_rows() { return sizeof(T) == 2 || KIN == 64 ? 4 * D + 16 : 2 * D + 16; }
-
-__device__ __forceinline__ void st8(half_t* p, const float (&v)[8]) { st_run(p, v); }
-__device__ __forceinline__ void st8(float* p, const float (&v)[8]) {
-  *reinterpret_cast<f4*>(p) = f4{v[0], v[1], v[2], v[3]};
-  *reinterpret_cast<f4*>(p + 4) = f4{v[4], v[5], v[6], v[7]};
-}
+constexpr int ATTN_ROWS = 4 * D + 16;
 
 // 12 waves (3 per SIMD, up to 168 VGPRs): the two row sets (current and prefetched) plus the per-lane store addresses
 // of the three output layouts do not fit the 128 VGPRs of 4 waves per SIMD.
@@ -386,12 +376,11 @@ __global__ __launch_bounds__(64 * ATTN_PROJ_WAVES) void triattn_proj_k(const T* 
                                                                         float q_scale, float b_scale,
                                                                         T* __restrict__ qkg, T* __restrict__ vt,
                                                                         T* __restrict__ tb, int64_t N, int64_t ldk,
-                                                                        int H, int C, int r_lo, int r_hi) {
+                                                                        int H, int C) {
   using RT = RunTile<T>;
   constexpr int RB = RT::RB, TW = RT::TW, STEPS = RG<T, KIN>::STEPS, LDW = ldw_of<T, KIN>();
-  __shared__ LDS_ALIGN T Ws[attn_rows<T, KIN>() * LDW];
-  lds_rows<T>(Ws, LDW, r_hi - r_lo, KIN, [&](int lr) -> const T* {
-    const int R = r_lo + lr;
+  __shared__ LDS_ALIGN T Ws[ATTN_ROWS * LDW];
+  lds_rows<T>(Ws, LDW, ATTN_ROWS, KIN, [&](int R) -> const T* {
     if (R >= 4 * D) return R - 4 * D < H ? w + (int64_t)R * KIN : nullptr;
     if (R >= 2 * D && R < 3 * D) return w + (int64_t)R * KIN;
     const int q = R & 31, rr = q & 15;
@@ -420,9 +409,8 @@ __global__ __launch_bounds__(64 * ATTN_PROJ_WAVES) void triattn_proj_k(const T* 
     load(min(t + stride, ntiles - 1), xnext);
     // ROWS orientation: key j0 + RUN g + 4 rb + e is inside the row
     const auto valid = [&](int rb, int e) { return j0 + RT::RUN * g + 4 * rb + e < N ? 1.0f : 0.0f; };
-    for (int m = 0; m < r_hi - r_lo; m += 32) {
-      const int R = r_lo + m;
-      const T* wb = Ws + m * LDW;
+    for (int R = 0; R < ATTN_ROWS; R += 32) {
+      const T* wb = Ws + R * LDW;
       if (R >= 4 * D) {  // triangle bias (16-row block, H valid rows)
         f4 acc[RB][1];
         zero_acc(acc);
@@ -462,7 +450,7 @@ __global__ __launch_bounds__(64 * ATTN_PROJ_WAVES) void triattn_proj_k(const T* 
           if (j >= N) continue;
           const float v[8] = {acc[rb][0][0] * sc, acc[rb][0][1] * sc, acc[rb][0][2] * sc, acc[rb][0][3] * sc,
                               acc[rb][1][0] * sc, acc[rb][1][1] * sc, acc[rb][1][2] * sc, acc[rb][1][3] * sc};
-          st8(qkg + (plane * NN + (int64_t)i * N + j) * C + d, v);
+          st_run(qkg + (plane * NN + (int64_t)i * N + j) * C + d, v);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -480,7 +468,7 @@ __global__ __launch_bounds__(64 * ATTN_PROJ_WAVES) void triattn_proj_k(const T* 
 // longer than the compute of the waves sharing a SIMD). On a wave's last tile the clamped "next" tile may be another
 // wave's; those loads are never used.
 template <typename T, int DO>
-__global__ __launch_bounds__(256, sizeof(T) == 2 ? 3 : 2) void linear_resid_ln_k(const T* __restrict__ x_in,
+__global__ __launch_bounds__(256, 3) void linear_resid_ln_k(const T* __restrict__ x_in,
                                                                                 const T* __restrict__ w, int trans,
                                                                                 float* __restrict__ z, int accumulate,
                                                                                 const float* __restrict__ lnw,
@@ -532,14 +520,14 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 3 : 2) void linear_resid_ln_k
 // ---------------------------------------------------------------- transition
 // Hidden chunks of HCH units: h1^T, h2^T = fc1/fc2 chunk . xn^T (16-unit blocks), a = silu(h1) * h2 stays in the
 // accumulator layout, which is already the B operand layout of out^T += fc3[:, chunk] . a^T (keys of the fp16 MFMA
-// permuted as {4g .. 4g+3} u {16+4g .. 16+4g+3} within each 32-unit slice; fp32 steps take unit 4g + s).
+// permuted as {4g .. 4g+3} u {16+4g .. 16+4g+3} within each 32-unit slice).
 template <typename T, int HCH>
 __global__ __launch_bounds__(256) void transition_k(const T* __restrict__ xn, const T* __restrict__ w12,
                                                     const T* __restrict__ w3, float* __restrict__ z, int accumulate,
                                                     const float* __restrict__ lnw, const float* __restrict__ lnb,
                                                     float eps, T* __restrict__ xn_next, int64_t rows_total,
                                                     int hidden) {
-  constexpr int RB = RowBlocks<T>::v, TM = 64 * RB, STEPS = RG<T>::STEPS, LDW = ldw_of<T>();
+  constexpr int RB = 2, TM = 64 * RB, STEPS = RG<T>::STEPS, LDW = ldw_of<T>();
   constexpr int LDH = HCH + Pad<T>::v;
   constexpr int HB = HCH / 16;
   __shared__ LDS_ALIGN T W1s[HCH * LDW];
@@ -575,40 +563,26 @@ __global__ __launch_bounds__(256) void transition_k(const T* __restrict__ xn, co
 #pragma unroll
         for (int e = 0; e < 4; e++) a[rb][hb][e] = siluf_(h1[rb][0][e]) * h2[rb][0][e];
     }
-    if constexpr (sizeof(T) == 2) {
 #pragma unroll
-      for (int m = 0; m < HB / 2; m++) {
-        half8 bf[RB];
+    for (int m = 0; m < HB / 2; m++) {
+      half8 bf[RB];
+#pragma unroll
+      for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          bf[rb][e] = (half_t)a[rb][2 * m][e];
+          bf[rb][4 + e] = (half_t)a[rb][2 * m + 1][e];
+        }
+#pragma unroll
+      for (int ob = 0; ob < 8; ob++) {
+        const T* wr = W3s + (16 * ob + (l & 15)) * LDH + 32 * m + 4 * g;
+        const half4 lo = *reinterpret_cast<const half4*>(wr);
+        const half4 hi = *reinterpret_cast<const half4*>(wr + 16);
+        const half8 af = half8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 #pragma unroll
         for (int rb = 0; rb < RB; rb++)
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            bf[rb][e] = (half_t)a[rb][2 * m][e];
-            bf[rb][4 + e] = (half_t)a[rb][2 * m + 1][e];
-          }
-#pragma unroll
-        for (int ob = 0; ob < 8; ob++) {
-          const T* wr = W3s + (16 * ob + (l & 15)) * LDH + 32 * m + 4 * g;
-          const half4 lo = *reinterpret_cast<const half4*>(wr);
-          const half4 hi = *reinterpret_cast<const half4*>(wr + 16);
-          const half8 af = half8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-#pragma unroll
-          for (int rb = 0; rb < RB; rb++)
-            out[rb][ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf[rb], out[rb][ob], 0, 0, 0);
-        }
+          out[rb][ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf[rb], out[rb][ob], 0, 0, 0);
       }
-    } else {
-#pragma unroll
-      for (int hb = 0; hb < HB; hb++)
-#pragma unroll
-        for (int s = 0; s < 4; s++)
-#pragma unroll
-          for (int ob = 0; ob < 8; ob++) {
-            const float af = to_f(W3s[(16 * ob + (l & 15)) * LDH + 16 * hb + 4 * g + s]);
-#pragma unroll
-            for (int rb = 0; rb < RB; rb++)
-              out[rb][ob] = __builtin_amdgcn_mfma_f32_16x16x4f32(af, a[rb][hb][s], out[rb][ob], 0, 0, 0);
-          }
     }
   }
   resid_ln_rows<T, RB>(out, [&](int rb) -> int64_t { return row[rb] < rows_total ? row[rb] : -1; }, z, accumulate, lnw,
@@ -861,22 +835,18 @@ __global__ __launch_bounds__(64 * TRW, 8 / TRW) void transition_f16_k(const half
 
 // ---------------------------------------------------------------- launchers
 
-template <typename T, int HV, int KIN>
+template <int HV, int KIN, typename T = half_t>
 static hipError_t tm_proj_hv(const void* xn, const void* w, const float* mask, float scale, int incoming, void* ab,
                              int64_t N, int64_t ld, int resident, hipStream_t st) {
   const int64_t ntiles = N * (ld / (HV * RunTile<T>::TW));  // ld is a multiple of 64
   if (ntiles >= (1LL << 30)) return hipErrorInvalidValue;  // tile indices are 32-bit in the kernel
   const dim3 grid((unsigned)std::min<int64_t>(resident, (ntiles + PROJ_WAVES - 1) / PROJ_WAVES));
-  for (int c_lo = 0; c_lo < 2 * KIN; c_lo += proj_ch<T, KIN>()) {
-    trimul_proj_k<T, HV, KIN><<<grid, 64 * PROJ_WAVES, 0, st>>>(static_cast<const T*>(xn), static_cast<const T*>(w), mask,
-                                                          scale, incoming, static_cast<T*>(ab), N, ld, c_lo);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
+  trimul_proj_k<T, HV, KIN><<<grid, 64 * PROJ_WAVES, 0, st>>>(static_cast<const T*>(xn), static_cast<const T*>(w), mask,
+                                                        scale, incoming, static_cast<T*>(ab), N, ld);
+  return hipGetLastError();
 }
 
-template <typename T, int KIN>
+template <int KIN, typename T = half_t>
 static hipError_t tm_proj(const void* xn, const void* w, const float* mask, float scale, int incoming, void* ab,
                           int64_t N, int64_t ld, hipStream_t st) {
   static int cache[kMaxDevices];
@@ -887,24 +857,23 @@ static hipError_t tm_proj(const void* xn, const void* w, const float* mask, floa
   // the half tile's own overhead)
   const int64_t waves = (int64_t)resident * PROJ_WAVES, full = N * (ld / (2 * RunTile<T>::TW));
   const int64_t r2 = (full + waves - 1) / waves, r1x2 = (2 * full + waves - 1) / waves;
-  return 10 * r1x2 < 18 * r2 ? tm_proj_hv<T, 1, KIN>(xn, w, mask, scale, incoming, ab, N, ld, resident, st)
-                             : tm_proj_hv<T, 2, KIN>(xn, w, mask, scale, incoming, ab, N, ld, resident, st);
+  return 10 * r1x2 < 18 * r2 ? tm_proj_hv<1, KIN>(xn, w, mask, scale, incoming, ab, N, ld, resident, st)
+                             : tm_proj_hv<2, KIN>(xn, w, mask, scale, incoming, ab, N, ld, resident, st);
 }
 
 hipError_t launch_trimul_proj(const void* xn, const void* w, const float* mask, float scale, int incoming, void* ab,
                               int dt, int64_t N, int64_t ld, int dim, hipStream_t st) {
-  if (dim == 64)
-    return dt == DT_F16 ? tm_proj<half_t, 64>(xn, w, mask, scale, incoming, ab, N, ld, st)
-                        : tm_proj<float, 64>(xn, w, mask, scale, incoming, ab, N, ld, st);
-  return dt == DT_F16 ? tm_proj<half_t, D>(xn, w, mask, scale, incoming, ab, N, ld, st)
-                      : tm_proj<float, D>(xn, w, mask, scale, incoming, ab, N, ld, st);
+  if (dt == DT_F32)
+    return launch_trimul_proj_x3(static_cast<const float*>(xn), static_cast<const float*>(w), mask, scale, incoming,
+                                 static_cast<float*>(ab), N, ld, dim, st);
+  return (dim == 64 ? tm_proj<64> : tm_proj<D>)(xn, w, mask, scale, incoming, ab, N, ld, st);
 }
 
-template <typename T, int KIN>
+template <int KIN, typename T = half_t>
 static hipError_t tm_tail(const void* o, const float* now, const float* nob, float eps_out, const void* w_po,
                           const void* xn, const void* w_go, float* z, int accumulate, const float* lnw,
                           const float* lnb, float eps_next, void* xn_next, int64_t N, int64_t ld, hipStream_t st) {
-  constexpr int TM = 64 * RowBlocks<T>::v;
+  constexpr int TM = 128;
   const dim3 grid((unsigned)(N * ((ld + TM - 1) / TM)));
   trimul_tail_k<T, KIN><<<grid, 256, 0, st>>>(static_cast<const T*>(o), now, nob, eps_out, static_cast<const T*>(w_po),
                                          static_cast<const T*>(xn), static_cast<const T*>(w_go), z, accumulate, lnw,
@@ -932,26 +901,24 @@ static hipError_t tm_tail_f16(const void* o, const float* now, const float* nob,
 template <int KIN>
 static hipError_t tm_tail_c(const void* o, const float* now, const float* nob, float eps_out, const void* w_po,
                             const void* xn, const void* w_go, float* z, int accumulate, const float* lnw,
-                            const float* lnb, float eps_next, void* xn_next, int dt, int64_t N, int64_t ld,
-                            hipStream_t st) {
-  if (dt == DT_F16 && (int64_t)KIN * N * ld < (1LL << 31))
-    return tm_tail_f16<KIN>(o, now, nob, eps_out, w_po, xn, w_go, z, accumulate, lnw, lnb, eps_next, xn_next, N, ld,
-                            st);
-  return dt == DT_F16 ? tm_tail<half_t, KIN>(o, now, nob, eps_out, w_po, xn, w_go, z, accumulate, lnw, lnb, eps_next,
-                                             xn_next, N, ld, st)
-                      : tm_tail<float, KIN>(o, now, nob, eps_out, w_po, xn, w_go, z, accumulate, lnw, lnb, eps_next,
-                                            xn_next, N, ld, st);
+                            const float* lnb, float eps_next, void* xn_next, int64_t N, int64_t ld, hipStream_t st) {
+  return ((int64_t)KIN * N * ld < (1LL << 31) ? tm_tail_f16<KIN> : tm_tail<KIN>)(
+      o, now, nob, eps_out, w_po, xn, w_go, z, accumulate, lnw, lnb, eps_next, xn_next, N, ld, st);
 }
 
 hipError_t launch_trimul_tail(const void* o, const float* now, const float* nob, float eps_out, const void* w_po,
                               const void* xn, const void* w_go, float* z, int accumulate, const float* lnw,
                               const float* lnb, float eps_next, void* xn_next, int dt, int64_t N, int64_t ld, int dim,
                               hipStream_t st) {
+  if (dt == DT_F32)
+    return launch_trimul_tail_x3(static_cast<const float*>(o), now, nob, eps_out, static_cast<const float*>(w_po),
+                                 static_cast<const float*>(xn), static_cast<const float*>(w_go), z, accumulate, lnw,
+                                 lnb, eps_next, static_cast<float*>(xn_next), N, ld, dim, st);
   return (dim == 64 ? tm_tail_c<64> : tm_tail_c<D>)(o, now, nob, eps_out, w_po, xn, w_go, z, accumulate, lnw, lnb,
-                                                    eps_next, xn_next, dt, N, ld, st);
+                                                    eps_next, xn_next, N, ld, st);
 }
 
-template <typename T, int KIN>
+template <int KIN, typename T = half_t>
 static hipError_t ta_proj(const void* xn, const void* w, int trans, float q_scale, float b_scale, void* qkg, void* vt,
                           void* tb, int64_t N, int64_t ldk, int H, int C, hipStream_t st) {
   if (H * C != D || H > 16 || C % 8) return hipErrorInvalidValue;
@@ -961,29 +928,23 @@ static hipError_t ta_proj(const void* xn, const void* w, int trans, float q_scal
   const int64_t ntiles = N * (ldk / RunTile<T>::TW);  // ldk is a multiple of 64
   if (ntiles >= (1LL << 30)) return hipErrorInvalidValue;  // tile indices are 32-bit in the kernel
   const dim3 grid((unsigned)std::min<int64_t>(resident, (ntiles + ATTN_PROJ_WAVES - 1) / ATTN_PROJ_WAVES));
-  constexpr bool ONE = attn_rows<T, KIN>() == 4 * D + 16;  // every row staged in one launch
-  const int bounds[3] = {0, ONE ? 4 * D + 16 : 2 * D, 4 * D + 16};
-  for (int p = 0; p < (ONE ? 1 : 2); p++) {
-    triattn_proj_k<T, KIN><<<grid, 64 * ATTN_PROJ_WAVES, 0, st>>>(
-        static_cast<const T*>(xn), static_cast<const T*>(w), trans, q_scale, b_scale, static_cast<T*>(qkg),
-        static_cast<T*>(vt), static_cast<T*>(tb), N, ldk, H, C, bounds[p], bounds[p + 1]);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
+  triattn_proj_k<T, KIN><<<grid, 64 * ATTN_PROJ_WAVES, 0, st>>>(
+      static_cast<const T*>(xn), static_cast<const T*>(w), trans, q_scale, b_scale, static_cast<T*>(qkg),
+      static_cast<T*>(vt), static_cast<T*>(tb), N, ldk, H, C);
+  return hipGetLastError();
 }
 
 hipError_t launch_triattn_proj(const void* xn, const void* w, int trans, float q_scale, float b_scale, void* qkg,
                                void* vt, void* tb, int dt, int64_t N, int64_t ldk, int dim, int H, int C,
                                hipStream_t st) {
-  if (dim == 64)
-    return dt == DT_F16 ? ta_proj<half_t, 64>(xn, w, trans, q_scale, b_scale, qkg, vt, tb, N, ldk, H, C, st)
-                        : ta_proj<float, 64>(xn, w, trans, q_scale, b_scale, qkg, vt, tb, N, ldk, H, C, st);
-  return dt == DT_F16 ? ta_proj<half_t, D>(xn, w, trans, q_scale, b_scale, qkg, vt, tb, N, ldk, H, C, st)
-                      : ta_proj<float, D>(xn, w, trans, q_scale, b_scale, qkg, vt, tb, N, ldk, H, C, st);
+  if (dt == DT_F32)
+    return launch_triattn_proj_x3(static_cast<const float*>(xn), static_cast<const float*>(w), trans, q_scale, b_scale,
+                                  static_cast<float*>(qkg), static_cast<float*>(vt), static_cast<float*>(tb), N, ldk,
+                                  dim, H, C, st);
+  return (dim == 64 ? ta_proj<64> : ta_proj<D>)(xn, w, trans, q_scale, b_scale, qkg, vt, tb, N, ldk, H, C, st);
 }
 
-template <typename T, int DO>
+template <int DO, typename T = half_t>
 static hipError_t lrl(const void* x, const void* w, int trans, float* z, int accumulate, const float* lnw,
                       const float* lnb, float eps, void* xn_next, int64_t N, hipStream_t st) {
   static int cache[kMaxDevices];
@@ -1000,18 +961,17 @@ static hipError_t lrl(const void* x, const void* w, int trans, float* z, int acc
 hipError_t launch_linear_resid_ln(const void* x, const void* w, int trans, float* z, int accumulate,
                                   const float* lnw, const float* lnb, float eps, void* xn_next, int dt, int64_t N,
                                   int dim, hipStream_t st) {
-  if (dim == 64)
-    return dt == DT_F16 ? lrl<half_t, 64>(x, w, trans, z, accumulate, lnw, lnb, eps, xn_next, N, st)
-                        : lrl<float, 64>(x, w, trans, z, accumulate, lnw, lnb, eps, xn_next, N, st);
-  return dt == DT_F16 ? lrl<half_t, D>(x, w, trans, z, accumulate, lnw, lnb, eps, xn_next, N, st)
-                      : lrl<float, D>(x, w, trans, z, accumulate, lnw, lnb, eps, xn_next, N, st);
+  if (dt == DT_F32)
+    return launch_linear_resid_ln_x3(static_cast<const float*>(x), static_cast<const float*>(w), trans, z, accumulate,
+                                     lnw, lnb, eps, static_cast<float*>(xn_next), N, dim, st);
+  return (dim == 64 ? lrl<64> : lrl<D>)(x, w, trans, z, accumulate, lnw, lnb, eps, xn_next, N, st);
 }
 
 template <typename T, int HCH>
 static hipError_t trans_t(const void* xn, const void* w12, const void* w3, float* z, int accumulate, const float* lnw,
                           const float* lnb, float eps, void* xn_next, int64_t rows, int hidden, hipStream_t st) {
   if (hidden % HCH) return hipErrorInvalidValue;
-  constexpr int TM = 64 * RowBlocks<T>::v;
+  constexpr int TM = 128;
   const dim3 grid((unsigned)((rows + TM - 1) / TM));
   transition_k<T, HCH><<<grid, 256, 0, st>>>(static_cast<const T*>(xn), static_cast<const T*>(w12),
                                              static_cast<const T*>(w3), z, accumulate, lnw, lnb, eps,
@@ -1056,11 +1016,14 @@ static hipError_t trans_f16(const void* xn, const void* w12, const void* w3, flo
 hipError_t launch_transition(const void* xn, const void* w12, const void* w3, float* z, int accumulate,
                              const float* lnw, const float* lnb, float eps, void* xn_next, int dt, int64_t rows,
                              int hidden, hipStream_t st) {
-  if (dt == DT_F16 && hidden % TR_HCH == 0 && (int64_t)2 * hidden * D < (1LL << 31))
+  if (dt == DT_F32)
+    return launch_transition_x3(static_cast<const float*>(xn), static_cast<const float*>(w12),
+                                static_cast<const float*>(w3), z, accumulate, lnw, lnb, eps,
+                                static_cast<float*>(xn_next), rows, hidden, st);
+  if (hidden % TR_HCH == 0 && (int64_t)2 * hidden * D < (1LL << 31))
     return trans_f16<false>(xn, w12, w3, z, accumulate, lnw, lnb, eps, xn_next, rows, hidden, nullptr, nullptr,
                             nullptr, 0.f, nullptr, 0, st);
-  return dt == DT_F16 ? trans_t<half_t, 64>(xn, w12, w3, z, accumulate, lnw, lnb, eps, xn_next, rows, hidden, st)
-                      : trans_t<float, 32>(xn, w12, w3, z, accumulate, lnw, lnb, eps, xn_next, rows, hidden, st);
+  return trans_t<half_t, 64>(xn, w12, w3, z, accumulate, lnw, lnb, eps, xn_next, rows, hidden, st);
 }
 
 // Transition + the s track's pair bias from the updated z: the fp16 kernel computes it in its epilogue; otherwise

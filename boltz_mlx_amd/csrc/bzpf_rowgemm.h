@@ -23,20 +23,6 @@ template <int KIN> struct RG<half_t, KIN> {
     for (int s = 0; s < STEPS; s++) f[s] = *reinterpret_cast<const half8*>(p + KIN / 4 * g + 8 * s);
   }
 };
-template <int KIN> struct RG<float, KIN> {
-  static constexpr int STEPS = KIN / 4;
-  typedef float frag;
-  __device__ static __forceinline__ void load_row(frag (&f)[STEPS], const float* p, int g) {
-#pragma unroll
-    for (int j = 0; j < KIN / 16; j++) {
-      const f4 v = *reinterpret_cast<const f4*>(p + KIN / 4 * g + 4 * j);
-      f[4 * j] = v[0]; f[4 * j + 1] = v[1]; f[4 * j + 2] = v[2]; f[4 * j + 3] = v[3];
-    }
-  }
-};
-
-// Row blocks per wave: fp16 tiles are 128 rows per workgroup (2 blocks per wave), fp32 tiles 64 rows.
-template <typename T> struct RowBlocks { static constexpr int v = sizeof(T) == 2 ? 2 : 1; };
 
 // acc[rb][cb] += W[16 cb .. +15][0:128] . X[rb]^T for CB column blocks of the LDS weight chunk Ws (pitch ldw).
 // ROWS = true computes the same block untransposed, acc[rb][cb] += X[rb] . W[16 cb .. +15]^T: the two operand
@@ -50,26 +36,13 @@ __device__ __forceinline__ void mma_rows(f4 (&acc)[RB][CB], const typename RG<T,
 #pragma unroll
   for (int cb = 0; cb < CB; cb++) {
     const T* wp = Ws + (16 * cb + (l & 15)) * ldw + KIN / 4 * g;
-    if constexpr (sizeof(T) == 2) {
 #pragma unroll
-      for (int s = 0; s < KIN / 32; s++) {
-        const half8 a = *reinterpret_cast<const half8*>(wp + 8 * s);
+    for (int s = 0; s < KIN / 32; s++) {
+      const half8 a = *reinterpret_cast<const half8*>(wp + 8 * s);
 #pragma unroll
-        for (int rb = 0; rb < RB; rb++)
-          acc[rb][cb] = ROWS ? __builtin_amdgcn_mfma_f32_16x16x32_f16(x[rb][s], a, acc[rb][cb], 0, 0, 0)
-                             : __builtin_amdgcn_mfma_f32_16x16x32_f16(a, x[rb][s], acc[rb][cb], 0, 0, 0);
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < KIN / 16; j++) {
-        const f4 a = *reinterpret_cast<const f4*>(wp + 4 * j);
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-          for (int rb = 0; rb < RB; rb++)
-            acc[rb][cb] = ROWS ? __builtin_amdgcn_mfma_f32_16x16x4f32(x[rb][4 * j + t], a[t], acc[rb][cb], 0, 0, 0)
-                               : __builtin_amdgcn_mfma_f32_16x16x4f32(a[t], x[rb][4 * j + t], acc[rb][cb], 0, 0, 0);
-      }
+      for (int rb = 0; rb < RB; rb++)
+        acc[rb][cb] = ROWS ? __builtin_amdgcn_mfma_f32_16x16x32_f16(x[rb][s], a, acc[rb][cb], 0, 0, 0)
+                           : __builtin_amdgcn_mfma_f32_16x16x32_f16(a, x[rb][s], acc[rb][cb], 0, 0, 0);
     }
   }
 }
@@ -78,7 +51,7 @@ __device__ __forceinline__ void mma_rows(f4 (&acc)[RB][CB], const typename RG<T,
 // lane r (= l % 16) loads for row block rb is position pos(rb, r) = 4 RB (r / 4) + 4 rb + r % 4. The accumulator
 // lane of group g then holds positions 4 RB g .. 4 RB g + 4 RB - 1 (index 4 rb + e) of one channel: 16 bytes of T.
 template <typename T> struct RunTile {
-  static constexpr int RB = sizeof(T) == 2 ? 2 : 1;
+  static constexpr int RB = 2;
   static constexpr int TW = 16 * RB;
   static constexpr int RUN = 4 * RB;
   __device__ static __forceinline__ int pos(int rb, int r) { return RUN * (r >> 2) + 4 * rb + (r & 3); }
@@ -92,17 +65,11 @@ __device__ __forceinline__ void st_run(half_t* p, const float (&v)[8]) {
                                     (half_t)v[5], (half_t)v[6], (half_t)v[7]},
                               reinterpret_cast<half8*>(p));
 }
-__device__ __forceinline__ void st_run(float* p, const float (&v)[4]) {
-  __builtin_nontemporal_store(f4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f4*>(p));
-}
 // The same runs through the default cache policy (the trimul projection: its half-line runs of one channel row
 // merge in L2 before they are written back; measured 7-10% faster there than non-temporal stores).
 __device__ __forceinline__ void st_run_cached(half_t* p, const float (&v)[8]) {
   *reinterpret_cast<half8*>(p) = half8{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3], (half_t)v[4],
                                        (half_t)v[5], (half_t)v[6], (half_t)v[7]};
-}
-__device__ __forceinline__ void st_run_cached(float* p, const float (&v)[4]) {
-  *reinterpret_cast<f4*>(p) = f4{v[0], v[1], v[2], v[3]};
 }
 
 // mma_rows over CB column blocks in groups of G with a scheduling barrier between groups: the compiler otherwise

@@ -1,0 +1,142 @@
+"""The fp32 row kernels of the pair track (split operands on the bf16 matrix cores) against float64, at the sizes where
+their tiles of 16, 32, 64 and 256 rows end, and at the row counts where the transition changes its form.
+
+Tolerance: fp32 sums over 128 to 512 terms err by 1e-7 .. 3e-7 of the result's norm; 1e-6 leaves a factor of three, and a
+dropped part product (2^-16 of the value) would show as 1e-5."""
+
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+LOG2E = 1.4426950408889634
+TOL = 1e-6
+
+
+@pytest.fixture(autouse=True)
+def _fp32():
+    from boltz_mlx_amd import kernels as K
+
+    before = K.PRECISION
+    K.set_precision("fp32")
+    yield
+    K.set_precision(before)
+
+
+def _rel(a, ref):
+    return ((a.double() - ref).norm() / ref.norm()).item()
+
+
+def _ln(x, ln):
+    return torch.nn.functional.layer_norm(x, x.shape[-1:], ln.weight.double(), ln.bias.double(), ln.eps)
+
+
+def _make(N, D, DO=None):
+    from boltz_mlx_amd.layers.norm import LayerNorm
+
+    g = torch.Generator(device="cuda").manual_seed(1000 * D + N)
+    randn = lambda *s: torch.randn(s, generator=g, device="cuda")
+    ln = LayerNorm(DO or D).cuda()
+    with torch.no_grad():
+        ln.weight.copy_(1 + 0.1 * randn(DO or D))
+        ln.bias.copy_(0.1 * randn(DO or D))
+    return randn, ln
+
+
+SIZES = [1, 5, 16, 33, 64, 95]
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("N", SIZES)
+def test_trimul_proj_and_tail(N, D):
+    from boltz_mlx_amd import kernels as K
+
+    randn, ln = _make(N, D)
+    proj, tail = (K.trimul_proj64, K.trimul_tail64) if D == 64 else (K.trimul_proj, K.trimul_tail)
+    xn, w = randn(N * N, D), randn(4 * D, D) * D ** -0.5
+    mask = (torch.rand((N, N), device="cuda") > 0.2).float()
+    p, gate = (xn.double() @ w.double().T).view(N, N, 4 * D).split(2 * D, -1)
+    ref = (p * torch.sigmoid(gate) * mask.double()[..., None]).permute(2, 0, 1)
+    for incoming in (False, True):
+        ab = proj(xn, w, mask, 0.5, incoming, N)
+        want = 0.5 * (ref.transpose(1, 2) if incoming else ref)
+        assert _rel(ab[..., :N], want) < TOL if want.norm() > 0 else not ab[..., :N].any()
+        assert not ab[..., N:].any()
+    with torch.no_grad():
+        norm_out = type(ln)(D).cuda()
+        norm_out.weight.copy_(1 + 0.1 * randn(D))
+        norm_out.bias.copy_(0.1 * randn(D))
+        o = torch.full((D, N, K.row_pitch(N)), float("nan"), device="cuda")  # columns past N may hold anything
+        o[..., :N] = randn(D, N, N) * 3 + 1
+        w_po, w_go, z0 = randn(D, D) * D ** -0.5, randn(D, D) * D ** -0.5, randn(N, N, D)
+        y = (_ln(o[..., :N].double().permute(1, 2, 0), norm_out) @ w_po.double().T) * torch.sigmoid(
+            xn.double() @ w_go.double().T).view(N, N, D)
+        for acc, nxt in ((False, None), (True, ln)):
+            z = z0.clone() if acc else torch.full_like(z0, float("nan"))
+            xo = tail(o, norm_out, norm_out.eps, w_po, xn, w_go, z, acc, nxt, N)
+            want = y + z0.double() if acc else y
+            assert _rel(z, want) < TOL
+            if nxt is not None:
+                assert _rel(xo.view(N, N, D), _ln(want, ln)) < TOL
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("N,H,C", [(1, 4, 32), (5, 8, 16), (16, 2, 64), (33, 4, 32), (64, 4, 32), (95, 4, 32)])
+def test_triattn_proj(N, H, C, D):
+    from boltz_mlx_amd import kernels as K
+
+    randn, _ = _make(N, D)
+    xn, w = randn(N * N, D), randn(4 * H * C + H, D) * D ** -0.5
+    for trans in (False, True):
+        qkg, vt, tb = (K.triattn_proj64 if D == 64 else K.triattn_proj)(xn, w, trans, N, H, C)
+        y = (xn.double() @ w.double().T).view(N, N, -1)
+        y = y.transpose(0, 1) if trans else y
+        q, k, v, g, b = y.split([H * C] * 4 + [H], -1)
+        heads = lambda t: t.reshape(N * N, H, C).transpose(0, 1)
+        want = torch.cat([heads(q) * LOG2E / C ** 0.5, heads(k), heads(g)])
+        assert _rel(qkg, want) < TOL
+        assert _rel(vt[..., :N], v.reshape(N, N, H, C).permute(2, 0, 3, 1)) < TOL and not vt[..., N:].any()
+        off = torch.from_numpy(K.tri_bias_offsets(N, H)).cuda()
+        assert _rel(tb[off], b.permute(2, 0, 1) * LOG2E) < TOL
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("N", SIZES)
+def test_linear_resid_ln(N, D):
+    from boltz_mlx_amd import kernels as K
+
+    randn, ln = _make(N, D)
+    x, w, z0 = randn(N * N, 128), randn(D, 128) * 128 ** -0.5, randn(N, N, D)
+    y = (x.double() @ w.double().T).view(N, N, D)
+    with torch.no_grad():
+        for trans, acc, nxt in ((False, True, ln), (True, True, ln), (True, False, None)):
+            z = z0.clone() if acc else torch.full_like(z0, float("nan"))
+            xo = (K.linear_resid_ln64 if D == 64 else K.linear_resid_ln)(x, w, trans, z, acc, nxt, N)
+            want = (y.transpose(0, 1) if trans else y) + (z0.double() if acc else 0.0)
+            assert _rel(z, want) < TOL
+            if nxt is not None:
+                assert _rel(xo.view(N, N, D), _ln(want, ln)) < TOL
+
+
+# rows: ends of the 16-, 32-, 128- and 256-row tiles, both sides of the row counts where the form changes, and whole
+# rounds of 65,536 rows with a remainder in each form
+@pytest.mark.parametrize("rows,hidden", [(1, 64), (15, 512), (17, 320), (4096, 512), (4097, 64), (16384, 64),
+                                         (16385, 512), (32768, 64), (32769, 512), (65536, 64), (65537, 192),
+                                         (70001, 64), (90000, 128), (100000, 64)])
+def test_transition(rows, hidden):
+    from boltz_mlx_amd import kernels as K
+
+    randn, ln = _make(rows, 128)
+    xn, z0 = randn(rows, 128), randn(rows, 1, 128)
+    w12, w3 = randn(2 * hidden, 128) * 128 ** -0.5, randn(128, hidden) * hidden ** -0.5
+    h1, h2 = (xn.double() @ w12.double().T).split(hidden, -1)
+    y = ((torch.nn.functional.silu(h1) * h2) @ w3.double().T).view(rows, 1, 128)
+    with torch.no_grad():
+        for acc, nxt in ((True, ln), (False, None)):
+            z = z0.clone() if acc else torch.full_like(z0, float("nan"))
+            xo = K.transition(xn, w12, w3, z, acc, nxt)
+            want = y + z0.double() if acc else y
+            assert _rel(z, want) < TOL
+            if nxt is not None:
+                assert _rel(xo.view(rows, 1, 128), _ln(want, ln)) < TOL
