@@ -120,6 +120,46 @@ def test_opm_ln_split(S, N):
     assert O.metrics(out, oref)["max_rel"] < 1e-5
 
 
+# tiles of 4 x 4 tokens, one and odd numbers of stages, ranges of rows; masks of 0 / 1, with values past 1 and with a token that is masked everywhere; rows of very large values
+@pytest.mark.parametrize("S,N,i_base,n_i,mscale,wscale", [(37, 5, 0, 5, 1.0, 1.0), (16, 130, 3, 126, 1.0, 1.0),
+                                                          (1, 9, 0, 9, 3.0, 1.0), (33, 181, 0, 181, 1.0, 1.0),
+                                                          (50, 190, 2, 177, 1.0, 300.0), (64, 37, 0, 37, 1e4, 1e-6)])
+def test_opm_outer2(S, N, i_base, n_i, mscale, wscale):
+    """The fp16 outer sum over two fp16 parts against float64: the error of the fp16 store, 2^-11 of the value, and the
+    sum's own, 2^-20 of the largest value (split parts: 2^-22 of a product)."""
+    from boltz_mlx_amd import kernels as K
+
+    rng = np.random.default_rng(S * N)
+    m = (rng.standard_normal((S, N, 64)) * 1.5 + 0.2).astype(np.float32)
+    m[0, 0] *= 1e6
+    mask = (mscale * (rng.random((S, N)) > 0.2)).astype(np.float32)
+    mask[:, N - 1] = 0
+    w_ab = (wscale * rng.standard_normal((64, 64)) / 8).astype(np.float32)
+
+    class LN:
+        weight = dev(1 + 0.1 * rng.standard_normal(64))
+        bias = dev(0.1 * rng.standard_normal(64))
+        eps = 1e-5
+
+    num = K.opm_counts(dev(mask))
+    planes, inv = K.opm_ln_split2(dev(m), LN, dev(w_ab), dev(mask), num)
+    assert torch.isfinite(planes).all()
+    got = K.opm_outer2(planes, inv, num, S, N, i_base, n_i).double()
+    mn = torch.nn.functional.layer_norm(dev(m).double(), (64,), LN.weight.double(), LN.bias.double(), 1e-5)
+    x = (mn @ dev(w_ab).double().T) * dev(mask).double()[..., None]
+    a, b = x[:, i_base:i_base + n_i, :32].reshape(S, -1), x[..., 32:].reshape(S, -1)
+    ref = (a.T.contiguous() @ b).view(n_i, 32, N, 32).transpose(1, 2).reshape(n_i * N, 1024)
+    md = dev(mask).double()
+    ref = ref / (md.T @ md)[i_base:i_base + n_i].clamp(min=1).reshape(-1, 1)
+    top = ref.abs().max()
+    if top < 6e4:  # fp16's range
+        assert ((got - ref).abs() <= ref.abs() * 2.0 ** -11 + top * 2.0 ** -20 + 2.0 ** -25).all()
+    else:
+        small = ref.abs() < 6e4
+        assert ((got - ref).abs()[small] <= ref.abs()[small] * 2.0 ** -11 + top * 2.0 ** -20).all()
+        assert torch.isinf(got[ref.abs() > 6.6e4]).all()
+
+
 def test_opm_outer_zero_count_pair():
     """Two tokens that never share an unmasked MSA row: their pair's count is 0, clamped to 1, and z is 0."""
     from boltz_mlx_amd import kernels as K
