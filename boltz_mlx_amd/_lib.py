@@ -99,7 +99,7 @@ def load(path: str | None = None):
 
 def call(name: str, *args) -> None:
     """Call an entry point; a non-zero status raises BzpfError with the library's message."""
-    rc = getattr(load(), name)(*args)
+    rc = getattr(_lib or load(), name)(*args)
     if rc != 0:
         msg = load().bzpf_last_error().decode()
         raise BzpfError(f"{name} failed ({rc}): {msg}")

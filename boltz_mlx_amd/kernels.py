@@ -14,6 +14,7 @@ multiplication operands a, b are pre-scaled by 2^-TRIMULT_K and norm_out's eps b
 from __future__ import annotations
 
 import contextlib
+import functools
 import os
 from typing import NamedTuple
 
@@ -95,7 +96,8 @@ def _dt(t: torch.Tensor) -> int:
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    # torch.cuda.current_stream().cuda_stream without the Stream object (6 us of a launch's 20 on the host)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _p(t):
@@ -133,11 +135,31 @@ def declared_weights(owner: torch.nn.Module) -> dict:
 
 def kernel_weight(owner: torch.nn.Module, name: str) -> torch.Tensor:
     """The declared kernel weight `name` of `owner` in its dtype, cached on the module (wcache)."""
-    kw = declared_weights(owner).get(name)
+    fn = getattr(owner, "kernel_weights", None)
+    kw = None if fn is None else next((k for k in fn() if k.name == name), None)
     if kw is None:
         raise KeyError(f"{type(owner).__name__} declares no kernel weight {name!r}")
-    params = [owner.get_parameter(p) for p in kw.srcs]
+    params = [_parameter(owner, p) for p in kw.srcs]
     return wcache(owner, name, *params, dtype=storage_dtype() if kw.half else torch.float32)
+
+
+@functools.lru_cache(maxsize=4096)
+def _path(path: str) -> tuple:
+    *modules, leaf = path.split(".")
+    return tuple(modules), leaf
+
+
+def _parameter(owner: torch.nn.Module, path: str) -> torch.Tensor:
+    """owner.get_parameter(path), straight from the modules' registries where every step is registered there (the
+    attribute walk costs the host as much as a launch)."""
+    modules, leaf = _path(path)
+    m = owner
+    for name in modules:
+        m = m._modules.get(name)
+        if m is None:
+            return owner.get_parameter(path)
+    p = m._parameters.get(leaf)
+    return owner.get_parameter(path) if p is None else p
 
 
 def _wkey(dtype, params) -> tuple:
@@ -167,6 +189,9 @@ def wcache(owner: torch.nn.Module, name: str, *params: torch.Tensor, dtype=None)
 
 
 def f32c(t: torch.Tensor) -> torch.Tensor:
+    """t in fp32, contiguous, for its data pointer (t itself where it is both already)."""
+    if t.dtype == torch.float32 and t.is_contiguous():
+        return t
     return t.detach().float().contiguous()
 
 

@@ -39,12 +39,14 @@ class AttentionPairBias(torch.nn.Module):
             self.proj_z = torch.nn.Sequential(LayerNorm(c_z), torch.nn.Linear(c_z, num_heads, bias=False))
         self.proj_o = torch.nn.Linear(c_s, c_s, bias=False)
 
+    _S_WEIGHTS = (K.KernelWeight("w_qkvg", ("proj_q.weight", "proj_k.weight", "proj_v.weight", "proj_g.weight"),
+                                 half=False),
+                  K.KernelWeight("w_o", ("proj_o.weight",), half=False))
+    _ALL_WEIGHTS = _S_WEIGHTS + (K.KernelWeight("w_z", ("proj_z.1.weight",)),)
+
     def kernel_weights(self):
         """[proj_q; proj_k; proj_v; proj_g] and proj_o in fp32 (both modes), proj_z's linear in the storage dtype."""
-        kws = (K.KernelWeight("w_qkvg", ("proj_q.weight", "proj_k.weight", "proj_v.weight", "proj_g.weight"),
-                              half=False),
-               K.KernelWeight("w_o", ("proj_o.weight",), half=False))
-        return kws + ((K.KernelWeight("w_z", ("proj_z.1.weight",)),) if self.compute_pair_bias else ())
+        return self._ALL_WEIGHTS if self.compute_pair_bias else self._S_WEIGHTS
 
     def qkvg_bias(self) -> torch.Tensor:
         """fp32 [4 c_s]: proj_q's bias, then zeros (the bias of the fused q | k | v | g GEMM), cached."""

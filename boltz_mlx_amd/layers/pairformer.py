@@ -119,7 +119,7 @@ class PairformerLayer(torch.nn.Module):
 
     def _pair_bias_args(self):
         """(LayerNorm, weight) of the attention's proj_z, for the transition's pair-bias epilogue."""
-        return self.attention.proj_z[0], self.attention.prepare()[3]
+        return self.attention.proj_z[0], K.kernel_weight(self.attention, "w_z")
 
     def prepare(self) -> None:
         """Cache every kernel weight of the layer in the storage dtype (a one-time conversion per precision; the

@@ -50,9 +50,11 @@ class Transition(torch.nn.Module):
             return out
         return self.unfused(xn)
 
+    _KERNEL_WEIGHTS = (K.KernelWeight("w12", ("fc1.weight", "fc2.weight")), K.KernelWeight("w3", ("fc3.weight",)))
+
     def kernel_weights(self):
         """[fc1; fc2] (the up-projection, SiLU branch first) and fc3, in the storage dtype."""
-        return K.KernelWeight("w12", ("fc1.weight", "fc2.weight")), K.KernelWeight("w3", ("fc3.weight",))
+        return self._KERNEL_WEIGHTS
 
     def prepare(self):
         """The kernel weights in the storage dtype ([fc1; fc2] and fc3), cached on the module. In f16 mode at 64

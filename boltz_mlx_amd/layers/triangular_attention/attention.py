@@ -91,7 +91,7 @@ class TriangleAttention(torch.nn.Module):
                 z.zero_()
             nxt = K.add_ln(z, y, ln=next_ln, trans_y=trans, out_dtype=K.storage_dtype())
             return None if nxt is None else nxt.view(N * N, D)
-        core = self._core_128(xn, mask, N, before_core, proj_trans)
+        core = self._core_128(xn, w, mask, N, before_core, proj_trans)
         return K.linear_resid_ln(core, w_o, trans, z, accumulate, next_ln, N)
 
     def fused_core(self, xn: torch.Tensor, mask: torch.Tensor, before_core=None):
@@ -101,11 +101,11 @@ class TriangleAttention(torch.nn.Module):
         N, D = mask.shape[0], xn.shape[-1]
         if D != 128 or self.no_heads * self.mha.c_hidden != D:
             return None
-        return self._core_128(xn, mask, N, before_core, not self.starting), self.prepare()[1]
+        w, w_o = self.prepare()
+        return self._core_128(xn, w, mask, N, before_core, not self.starting), w_o
 
-    def _core_128(self, xn, mask, N: int, before_core, proj_trans: bool):
+    def _core_128(self, xn, w, mask, N: int, before_core, proj_trans: bool):
         H, C = self.no_heads, self.mha.c_hidden
-        w = self.prepare()[0]
         qkg, vt, tb = K.triattn_proj(xn, w, proj_trans, N, H, C)
         if before_core is not None:
             before_core()
@@ -113,11 +113,13 @@ class TriangleAttention(torch.nn.Module):
         del qkg, vt, tb
         return core
 
+    _KERNEL_WEIGHTS = (K.KernelWeight("w_qkvgb", ("mha.linear_q.weight", "mha.linear_k.weight", "mha.linear_v.weight",
+                                                  "mha.linear_g.weight", "linear.weight")),
+                       K.KernelWeight("w_o", ("mha.linear_o.weight",)))
+
     def kernel_weights(self):
         """[q; k; v; g; triangle bias] (the projection's 4·H·C + H rows) and linear_o, in the storage dtype."""
-        return (K.KernelWeight("w_qkvgb", ("mha.linear_q.weight", "mha.linear_k.weight", "mha.linear_v.weight",
-                                           "mha.linear_g.weight", "linear.weight")),
-                K.KernelWeight("w_o", ("mha.linear_o.weight",)))
+        return self._KERNEL_WEIGHTS
 
     def prepare(self):
         """The kernel weights ([q; k; v; g; triangle bias] and linear_o), cached on the module."""

@@ -74,10 +74,12 @@ class _TriangleMultiplication(torch.nn.Module):
         return K.trimul_tail(o, self.norm_out, self.norm_out.eps * 2.0 ** (-4 * kexp), w_po, xn, w_go, z,
                              accumulate, next_ln, N)
 
+    _KERNEL_WEIGHTS = (K.KernelWeight("w_pg", ("p_in.weight", "g_in.weight")),
+                       K.KernelWeight("w_po", ("p_out.weight",)), K.KernelWeight("w_go", ("g_out.weight",)))
+
     def kernel_weights(self):
         """[p_in; g_in] (the projection kernel's 4·128 rows), p_out and g_out (the tail), all in the storage dtype."""
-        return (K.KernelWeight("w_pg", ("p_in.weight", "g_in.weight")), K.KernelWeight("w_po", ("p_out.weight",)),
-                K.KernelWeight("w_go", ("g_out.weight",)))
+        return self._KERNEL_WEIGHTS
 
     def prepare(self):
         """The kernel weights ([p_in; g_in], p_out, g_out), cached on the module."""
