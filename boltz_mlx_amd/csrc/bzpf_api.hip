@@ -101,7 +101,24 @@ int bzpf_trimul_contract(const void* ab, void* o, int dt, int64_t N, int64_t ld,
   REQUIRE(dt_ok(dt), "bzpf_trimul_contract: bad dtype %d", dt);
   REQUIRE(D >= 1 && D <= 65535, "bzpf_trimul_contract: bad D=%d", D);
   REQUIRE(N >= 1 && ld == bzpf_row_pitch(N), "bzpf_trimul_contract: N=%lld ld=%lld", (long long)N, (long long)ld);
-  return done(bzpf::launch_trimul_contract(ab, o, dt, N, ld, k_len, D, S(stream)), "bzpf_trimul_contract");
+  return done(bzpf::launch_trimul_contract(ab, o, dt, N, ld, k_len, nullptr, D, S(stream)), "bzpf_trimul_contract");
+}
+
+int bzpf_trimul_contract_ext(const void* ab, void* o, int dt, int64_t N, int64_t ld, int D, const int* ext,
+                             void* stream) {
+  REQUIRE_PTR(ab);
+  REQUIRE_PTR(o);
+  REQUIRE(ext != nullptr, "bzpf_trimul_contract_ext: ext is NULL");
+  REQUIRE(dt_ok(dt), "bzpf_trimul_contract_ext: bad dtype %d", dt);
+  REQUIRE(D >= 1 && D <= 65535, "bzpf_trimul_contract_ext: bad D=%d", D);
+  REQUIRE(N >= 1 && ld == bzpf_row_pitch(N), "bzpf_trimul_contract_ext: N=%lld ld=%lld", (long long)N, (long long)ld);
+  return done(bzpf::launch_trimul_contract(ab, o, dt, N, ld, 0, ext, D, S(stream)), "bzpf_trimul_contract_ext");
+}
+
+int bzpf_key_extents(const float* mask, int64_t N, int* ext, void* stream) {
+  REQUIRE(mask && ext, "bzpf_key_extents: NULL pointer");
+  REQUIRE(N >= 1 && N <= INT32_MAX, "bzpf_key_extents: N=%lld", (long long)N);
+  return done(bzpf::launch_key_extents(mask, N, ext, S(stream)), "bzpf_key_extents");
 }
 
 int bzpf_trimul_tail(const void* o, const float* norm_out_w, const float* norm_out_b, float eps_out,

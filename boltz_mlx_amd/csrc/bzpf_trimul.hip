@@ -24,6 +24,33 @@ namespace bzpf {
 // Bound by the matrix cores and the split beside them (a stage of a 64 x 64 wave tile is 768 MFMA cycles and 88 VALU
 // instructions): N = 640 402 us (167 TFLOP/s, 0.4 of the bf16 peak in part products), N = 513 276, N = 333 79, against
 // 626, 555 and 160 us for the fp32 MFMA kernel this replaces; error against float64 3.8e-7 -> 3.2e-7 (N = 513).
+// The stages of bk columns to contract: `all` of them, or those up to the extent the device holds (rounded up to 64
+// columns; 0 or >= N: all).
+__device__ __forceinline__ int contract_stages(int all, int bk, const int* ext, int64_t N) {
+  if (ext == nullptr) return all;
+  const int e = __builtin_amdgcn_readfirstlane(*ext);
+  return e <= 0 || e >= N ? all : min(all, (e + 63) / 64 * 64 / bk);
+}
+
+// ext[0] = 1 + the last column with a nonzero in any row of mask [N][N], ext[1] = 1 + the last row with a nonzero (both 0
+// before the launch). A wave takes a row and scans it from its end, so a mask of leading real tokens is read for its
+// padded part and one step more.
+__global__ __launch_bounds__(256) void key_extents_k(const float* __restrict__ mask, int64_t N, int* __restrict__ ext) {
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= N) return;  // whole wave
+  const int l = threadIdx.x & 63;
+  const float* m = mask + row * N;
+  for (int64_t k0 = (N - 1) / 64 * 64; k0 >= 0; k0 -= 64) {
+    const uint64_t live = __ballot(k0 + l < N && m[min(k0 + l, N - 1)] != 0.0f);
+    if (live == 0) continue;
+    if (l == 0) {
+      atomicMax(ext, (int)(k0 + 64 - __clzll((long long)live)));
+      atomicMax(ext + 1, (int)(row + 1));
+    }
+    return;
+  }
+}
+
 // Element k of row r of a part plane: rows of KS = 16 values, their two 16-byte halves exchanged in every other group of
 // eight rows, so the fragment reads (16 lanes on 16 rows at one half) meet 16 distinct bank groups without padding.
 __device__ __forceinline__ int x3_at(int r, int k) { return r * KS + (k ^ (r & 8)); }
@@ -32,7 +59,9 @@ template <int WM, int WN, int MB, int NB>
 __global__ __launch_bounds__(64 * WM * WN, 2) void trimul_contract_x3_k(const float* __restrict__ ab,
                                                                         float* __restrict__ o, int64_t N, int64_t ld,
                                                                         int D, int tiles_i, int tiles_j, int64_t units,
-                                                                        int64_t per_xcd, int nst) {
+                                                                        int64_t per_xcd, int nst,
+                                                                        const int* __restrict__ ext) {
+  nst = contract_stages(nst, KS, ext, N);
   constexpr int BI = 32 * MB * WM, BJ = 32 * NB * WN, T = 64 * WM * WN;
   constexpr int LOADS = (BI + BJ) * (KS / 4) / T;  // 16-byte vectors per thread and stage
   constexpr int ROWS = T / (KS / 4);               // rows a pass of all threads covers
@@ -136,7 +165,8 @@ template <int BK, int NS>
 __global__ __launch_bounds__(512, 1) void trimul_contract_f16_k(const half_t* __restrict__ ab, half_t* __restrict__ o,
                                                                 int64_t N, int64_t ld, int D, int64_t tiles1,
                                                                 int64_t units, int64_t per_xcd, int wg_per_xcd,
-                                                                int nst) {
+                                                                int nst, const int* __restrict__ ext) {
+  nst = contract_stages(nst, BK, ext, N);
   constexpr int BT = 256, NW = 8;
   constexpr int ROWB = BK * 2;               // bytes of a row per stage
   constexpr int CPR = ROWB / 16;             // 16-byte chunks per row
@@ -302,42 +332,52 @@ __global__ __launch_bounds__(512, 1) void trimul_contract_f16_k(const half_t* __
 }
 
 // kl: the k range contracted (a multiple of 64, <= ld); columns past it are zero in a and b.
-static hipError_t contract_f16(const half_t* ab, half_t* o, int64_t N, int64_t ld, int64_t kl, int D, hipStream_t st) {
+static hipError_t contract_f16(const half_t* ab, half_t* o, int64_t N, int64_t ld, int64_t kl, const int* ext, int D,
+                               hipStream_t st) {
   const int64_t tiles1 = (N + 255) / 256, units = (int64_t)D * tiles1 * tiles1, per_xcd = (units + 7) / 8;
   static int cache[kMaxDevices] = {};
   const int resident = resident_grid(trimul_contract_f16_k<64, 2>, 512, cache);
   if (resident < 8) return hipErrorInvalidConfiguration;
   const int wpx = (int)(resident / 8 < per_xcd ? resident / 8 : per_xcd);
   trimul_contract_f16_k<64, 2>
-      <<<dim3(8 * wpx), 512, 0, st>>>(ab, o, N, ld, D, tiles1, units, per_xcd, wpx, (int)(kl / 64));
+      <<<dim3(8 * wpx), 512, 0, st>>>(ab, o, N, ld, D, tiles1, units, per_xcd, wpx, (int)(kl / 64),
+                                       ext);
   return hipGetLastError();
 }
 
 template <int WM, int WN, int MB, int NB>
-static hipError_t contract_x3(const float* ab, float* o, int64_t N, int64_t ld, int64_t kl, int D, hipStream_t st) {
+static hipError_t contract_x3(const float* ab, float* o, int64_t N, int64_t ld, int64_t kl, const int* ext, int D,
+                              hipStream_t st) {
   constexpr int BI = 32 * MB * WM, BJ = 32 * NB * WN;
   const int64_t ti = (N + BI - 1) / BI, tj = (N + BJ - 1) / BJ, units = (int64_t)D * ti * tj, per_xcd = (units + 7) / 8;
   trimul_contract_x3_k<WM, WN, MB, NB><<<dim3((unsigned)(per_xcd * 8)), 64 * WM * WN, 0, st>>>(
-      ab, o, N, ld, D, (int)ti, (int)tj, units, per_xcd, (int)(kl / KS));
+      ab, o, N, ld, D, (int)ti, (int)tj, units, per_xcd, (int)(kl / KS), ext);
   return hipGetLastError();
 }
 
 // 192 x 192 tiles (3 x 3 blocks a wave: half again the products per LDS read of 2 x 2) where their padded area is not much
 // larger than that of 128 x 128 tiles: they measure 0.83-0.85 ns per 1,000 padded outputs and channel against 0.98
 // (N = 513: 276 against 359 us; N = 333, equal areas: 79 against 93; N = 400: 226 against 186; N = 640: 502 against 402).
-static hipError_t contract_f32(const float* ab, float* o, int64_t N, int64_t ld, int64_t kl, int D, hipStream_t st) {
+static hipError_t contract_f32(const float* ab, float* o, int64_t N, int64_t ld, int64_t kl, const int* ext, int D,
+                               hipStream_t st) {
   const int64_t t128 = (N + 127) / 128 * 128, t192 = (N + 191) / 192 * 192;
-  return 7 * t192 * t192 <= 8 * t128 * t128 ? contract_x3<2, 2, 3, 3>(ab, o, N, ld, kl, D, st)
-                                            : contract_x3<2, 2, 2, 2>(ab, o, N, ld, kl, D, st);
+  return 7 * t192 * t192 <= 8 * t128 * t128 ? contract_x3<2, 2, 3, 3>(ab, o, N, ld, kl, ext, D, st)
+                                            : contract_x3<2, 2, 2, 2>(ab, o, N, ld, kl, ext, D, st);
 }
 
-hipError_t launch_trimul_contract(const void* ab, void* o, int dt, int64_t N, int64_t ld, int64_t k_len, int D,
-                                  hipStream_t st) {
+hipError_t launch_trimul_contract(const void* ab, void* o, int dt, int64_t N, int64_t ld, int64_t k_len, const int* ext,
+                                  int D, hipStream_t st) {
   if (dt == DT_F16 && !contract_shape_ok(N, ld)) return hipErrorInvalidValue;  // 32-bit buffer offsets per channel
   // contract over k < k_len rounded up to 64 (a whole number of stages of either kernel); 0 or >= N: every k
   const int64_t kl = k_len <= 0 || k_len >= N ? ld : (k_len + 63) / 64 * 64;
-  return dt == DT_F16 ? contract_f16(static_cast<const half_t*>(ab), static_cast<half_t*>(o), N, ld, kl, D, st)
-                      : contract_f32(static_cast<const float*>(ab), static_cast<float*>(o), N, ld, kl, D, st);
+  return dt == DT_F16 ? contract_f16(static_cast<const half_t*>(ab), static_cast<half_t*>(o), N, ld, kl, ext, D, st)
+                      : contract_f32(static_cast<const float*>(ab), static_cast<float*>(o), N, ld, kl, ext, D, st);
+}
+
+hipError_t launch_key_extents(const float* mask, int64_t N, int* ext, hipStream_t st) {
+  if (N < 1 || (N + 3) / 4 > INT32_MAX) return hipErrorInvalidValue;
+  key_extents_k<<<(unsigned)((N + 3) / 4), 256, 0, st>>>(mask, N, ext);
+  return hipGetLastError();
 }
 
 }  // namespace bzpf

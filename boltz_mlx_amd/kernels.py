@@ -353,16 +353,23 @@ def triattn_pack(P: torch.Tensor, trans: bool, N: int, H: int, C: int):
     return qkg, vt, tb
 
 
-def trimul_contract(ab: torch.Tensor, N: int, k_len: int = 0) -> torch.Tensor:
+def trimul_contract(ab: torch.Tensor, N: int, k_len=0) -> torch.Tensor:
     """o [D, N, ld] = per-channel a b^T; k_len > 0: columns k >= k_len of ab are zero and the sum stops there (the
-    trailing padded tokens; key_extent gives it for a pair mask)."""
+    trailing padded tokens; key_extent gives it for a pair mask). k_len may be an int32 tensor [1] on the device
+    (key_extent_device), which the kernel reads: the host need not know it."""
     _dev(ab)
     D = ab.shape[0] // 2
     ld = row_pitch(N)
     if ab.shape != (2 * D, N, ld):
         raise ValueError("trimul_contract: ab must be [2D, N, ld]")
     o = torch.empty((D, N, ld), dtype=ab.dtype, device=ab.device)
-    call("bzpf_trimul_contract", _p(ab), _p(o), _dt(ab), N, ld, D, int(k_len), _stream())
+    if isinstance(k_len, torch.Tensor):
+        _dev(k_len)
+        if k_len.dtype != torch.int32 or k_len.numel() != 1:
+            raise ValueError("trimul_contract: k_len must be an int or an int32 tensor of one element")
+        call("bzpf_trimul_contract_ext", _p(ab), _p(o), _dt(ab), N, ld, D, _p(k_len), _stream())
+    else:
+        call("bzpf_trimul_contract", _p(ab), _p(o), _dt(ab), N, ld, D, int(k_len), _stream())
     return o
 
 
@@ -414,6 +421,21 @@ def key_extent(mask: torch.Tensor, N: int, incoming: bool) -> int:
         idx = torch.nonzero(live)
         ent[("ext", incoming)] = int(idx[-1, 0].item()) + 1 if idx.numel() else N
     return ent[("ext", incoming)]
+
+
+def key_extent_device(mask: torch.Tensor, N: int, incoming: bool):
+    """key_extent as an int32 tensor [1] on the device (0 for a mask without a nonzero, which the contraction takes as
+    every key), so that a module run neither waits for the mask nor launches torch's reductions: inside pair_mask_scope
+    one kernel finds both directions' extents once per mask; 0 (every key) outside."""
+    ent = _mask_entry(mask)
+    if ent is None:
+        return 0
+    if "dev" not in ent:
+        _dev(mask)
+        ext = torch.zeros((2,), dtype=torch.int32, device=mask.device)
+        call("bzpf_key_extents", _p(mask), N, _p(ext), _stream())
+        ent["dev"] = ext
+    return ent["dev"][int(incoming):int(incoming) + 1]
 
 
 def trimul_tail(o, norm_out, eps_out: float, w_po, xn, w_go, z, accumulate: bool, next_ln=None, N: int = 0):

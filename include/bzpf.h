@@ -74,6 +74,14 @@ int bzpf_trimul_proj(const void* xn, const void* w_pg, const float* pair_mask, f
  * (boltz_mlx/kernels_nax2.py:315-407). */
 int bzpf_trimul_contract(const void* ab, void* o, int dt, int64_t N, int64_t ld, int D, int64_t k_len, void* stream);
 
+/* The same with k_len read from device memory by the kernel (one int: 0 or >= N for every k), and the extents of a pair
+ * mask fp32 [N][N] for it: bzpf_key_extents raises ext[0] (zeroed by the caller) to 1 + the last column with a nonzero
+ * (the outgoing direction's k_len) and ext[1] to 1 + the last row with one (incoming), so no host wait stands between a
+ * mask and the contraction (boltz_mlx/layers/triangular_mult.py:90-93, 172-175). */
+int bzpf_trimul_contract_ext(const void* ab, void* o, int dt, int64_t N, int64_t ld, int D, const int* ext,
+                             void* stream);
+int bzpf_key_extents(const float* mask, int64_t N, int* ext, void* stream);
+
 /* Triangle-multiplication tail: at each position p = (i, j),
  *   y = (LN_out(o[:, i, j]; eps_out) . W_po^T) * sigmoid(xn[p] . W_go^T);  z[p] = (accumulate ? z[p] : 0) + y;
  *   and, when next_w != NULL, xn_next[p] = LN_next(z[p]).

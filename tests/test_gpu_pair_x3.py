@@ -119,6 +119,28 @@ def test_linear_resid_ln(N, D):
                 assert _rel(xo.view(N, N, D), _ln(want, ln)) < TOL
 
 
+# masks whose last live column and row fall inside, at and past a 64-lane step; no live entry; one live entry
+@pytest.mark.parametrize("N,rows,cols", [(1, 1, 1), (5, 0, 0), (64, 40, 64), (65, 65, 1), (130, 64, 65), (200, 129, 70)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_key_extent_device(N, rows, cols, dtype):
+    """The extents against the host's, and the contraction that reads one against the same contraction told it."""
+    from boltz_mlx_amd import kernels as K
+
+    mask = torch.zeros((N, N), device="cuda")
+    if rows and cols:
+        mask[rows - 1, 0] = mask[0, cols - 1] = 1.0
+    ab = torch.randn((16, N, K.row_pitch(N)), device="cuda", dtype=dtype)
+    with K.pair_mask_scope():
+        for incoming, want in ((False, cols), (True, rows)):
+            ext = K.key_extent_device(mask, N, incoming)
+            assert int(ext.item()) == want and K.key_extent(mask, N, incoming) == (want or N)
+            masked = ab.clone()
+            masked[:, :, want or N:] = 0
+            got, ref = K.trimul_contract(masked, N, ext), K.trimul_contract(masked, N, want or N)
+            assert torch.equal(got[..., :N], ref[..., :N])
+    assert K.key_extent_device(mask, N, False) == 0
+
+
 # rows: ends of the 16-, 32-, 128- and 256-row tiles, both sides of the row counts where the form changes, and whole
 # rounds of 65,536 rows with a remainder in each form
 @pytest.mark.parametrize("rows,hidden", [(1, 64), (15, 512), (17, 320), (4096, 512), (4097, 64), (16384, 64),
