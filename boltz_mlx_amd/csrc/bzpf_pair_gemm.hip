@@ -9,6 +9,7 @@
 //   transition       : z (+)= fc3(silu(fc1 xn) * fc2 xn), then the next LayerNorm (transition.py:27-54, 148-154;
 //                      kernels_nax2.py:54-190, kernels_nax3.py:713-827).
 // These are the fp16 forms (two 16-row blocks per wave); the fp32 ones are in bzpf_pair_x3.hip.
+#include <algorithm>
 #include <type_traits>
 
 #include "bzpf_common.h"
@@ -32,22 +33,28 @@ template <typename T, int KIN = D> constexpr int ldw_of() { return KIN + Pad<T>:
 // values are loaded while the current tile computes (8 waves with the prefetch measured 3-4% faster than 12
 // without). HV = 1 (half tiles) is taken when it balances the last round of tiles better: at N = 400 (2,800 full
 // tiles on 2,048 waves) 0.041-0.045 against 0.050 ms; at N = 1000 full tiles are faster (0.23 against 0.26 ms).
+// NG > 1: the weight rows are dealt to NG groups of workgroups (all reading the same xn), for inputs of less than one
+// round of tiles: a wave's chain of channel blocks and a workgroup's staging are then 1 / NG as long.
 constexpr int PROJ_WAVES = 8;
 
-template <typename T, int HV, int KIN>
+template <typename T, int HV, int KIN, int NG>
 __global__ __launch_bounds__(64 * PROJ_WAVES) void trimul_proj_k(const T* __restrict__ xn, const T* __restrict__ w,
                                                                  const float* __restrict__ mask, float scale,
                                                                  int incoming, T* __restrict__ ab, int64_t N,
                                                                  int64_t ld) {
   using RT = RunTile<T>;
   constexpr int D = KIN;
-  constexpr int RB = RT::RB, TW = RT::TW, STEPS = RG<T, D>::STEPS, LDW = ldw_of<T, D>(), PCH = 2 * D;
+  constexpr int RB = RT::RB, TW = RT::TW, STEPS = RG<T, D>::STEPS, LDW = ldw_of<T, D>(), PCH = 2 * D / NG;
   __shared__ LDS_ALIGN T Ws[2 * PCH * LDW];  // rows [0, PCH): projections, [PCH, 2 PCH): gates
-  lds_rows<T>(Ws, LDW, 2 * PCH, D, [&](int r) { return w + (int64_t)r * D; });
+  int grp, wg;
+  weight_group<NG>(grp, wg);
+  const int c_lo = grp * PCH;
+  lds_rows<T>(Ws, LDW, 2 * PCH, D,
+              [&](int r) { return w + (int64_t)(r < PCH ? c_lo + r : 2 * D + c_lo + r - PCH) * D; });
   __syncthreads();
   const int l = threadIdx.x & 63, g = l >> 4, r = l & 15;
-  const int tpr = (int)(ld / (HV * TW)), ntiles = (int)N * tpr, stride = gridDim.x * PROJ_WAVES;
-  int t = grid_wave(PROJ_WAVES);
+  const int tpr = (int)(ld / (HV * TW)), ntiles = (int)N * tpr, stride = (int)(gridDim.x / NG) * PROJ_WAVES;
+  int t = __builtin_amdgcn_readfirstlane(wg * PROJ_WAVES + (int)(threadIdx.x >> 6));
   if (t >= ntiles) return;
 
   typedef typename RG<T, D>::frag Frag;
@@ -82,7 +89,7 @@ __global__ __launch_bounds__(64 * PROJ_WAVES) void trimul_proj_k(const T* __rest
 #pragma unroll
         for (int e = 0; e < 4; e++) mo[hh][rb][e] = __shfl(mv, 4 * g + e);
       }
-    T* dst = ab + ((int64_t)r * N + i) * ld + k0 + RT::RUN * g;
+    T* dst = ab + ((int64_t)(c_lo + r) * N + i) * ld + k0 + RT::RUN * g;
     for (int cb = 0; cb < PCH / 16; cb++) {
 #pragma unroll
       for (int hh = 0; hh < HV; hh++) {
@@ -217,14 +224,13 @@ __global__ __launch_bounds__(256) void trimul_tail_k(const T* __restrict__ o, co
 // keeps its waves in step: the four loads of a line reach L2 together and it is read from HBM once. Without the
 // barrier the waves drift apart by more than the L2 residency of a line and o is read about 2.3 times.
 constexpr int TAIL_WAVES = 12;
-__host__ __device__ constexpr int64_t tail_tiles_per_row(int64_t N) { return (N + 63) / 64 * 4; }
 
 template <int KIN>
 __global__ __launch_bounds__(64 * TAIL_WAVES) void trimul_tail_f16_k(
     const half_t* __restrict__ o, const float* __restrict__ now, const float* __restrict__ nob, float eps_out,
     const half_t* __restrict__ w_po, const half_t* __restrict__ xn, const half_t* __restrict__ w_go,
     float* __restrict__ z, int accumulate, const float* __restrict__ lnw, const float* __restrict__ lnb,
-    float eps_next, half_t* __restrict__ xn_next, int64_t N, int64_t ld) {
+    float eps_next, half_t* __restrict__ xn_next, int64_t N, int64_t ld, int tpr) {
   using T = half_t;
   constexpr int D = KIN, CB = D / 16, PP = D / 16;  // column blocks; positions of o a lane loads (of 4 channels)
   constexpr int STEPS = RG<T, D>::STEPS, LDW = ldw_of<T, D>(), LDT = D + Pad<T>::v;
@@ -265,7 +271,7 @@ __global__ __launch_bounds__(64 * TAIL_WAVES) void trimul_tail_f16_k(
   const int l = threadIdx.x & 63, g = l >> 4, r = l & 15;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   T* ts = Ts[wave];
-  const int tpr = (int)tail_tiles_per_row(N), ntiles = (int)N * tpr, stride = gridDim.x * TAIL_WAVES;
+  const int ntiles = (int)N * tpr, stride = gridDim.x * TAIL_WAVES;
   // rounds are workgroup-uniform (the barrier below needs every wave in every round); a wave whose tile is past the
   // end of a round recomputes the last tile and stores nothing
   int tb = blockIdx.x * TAIL_WAVES;
@@ -370,7 +376,7 @@ constexpr int ATTN_ROWS = 4 * D + 16;
 // of the three output layouts do not fit the 128 VGPRs of 4 waves per SIMD.
 constexpr int ATTN_PROJ_WAVES = 12;
 
-template <typename T, int KIN>
+template <typename T, int KIN, int NG>
 __global__ __launch_bounds__(64 * ATTN_PROJ_WAVES) void triattn_proj_k(const T* __restrict__ xn,
                                                                         const T* __restrict__ w, int trans,
                                                                         float q_scale, float b_scale,
@@ -379,8 +385,13 @@ __global__ __launch_bounds__(64 * ATTN_PROJ_WAVES) void triattn_proj_k(const T* 
                                                                         int H, int C) {
   using RT = RunTile<T>;
   constexpr int RB = RT::RB, TW = RT::TW, STEPS = RG<T, KIN>::STEPS, LDW = ldw_of<T, KIN>();
-  __shared__ LDS_ALIGN T Ws[ATTN_ROWS * LDW];
-  lds_rows<T>(Ws, LDW, ATTN_ROWS, KIN, [&](int R) -> const T* {
+  constexpr int GR = 4 * D / NG;  // a group's rows; the last one has the bias block too
+  __shared__ LDS_ALIGN T Ws[(GR + 16) * LDW];
+  int grp, wg;
+  weight_group<NG>(grp, wg);
+  const int r_lo = grp * GR, r_hi = grp == NG - 1 ? ATTN_ROWS : r_lo + GR;
+  lds_rows<T>(Ws, LDW, r_hi - r_lo, KIN, [&](int lr) -> const T* {
+    const int R = r_lo + lr;
     if (R >= 4 * D) return R - 4 * D < H ? w + (int64_t)R * KIN : nullptr;
     if (R >= 2 * D && R < 3 * D) return w + (int64_t)R * KIN;
     const int q = R & 31, rr = q & 15;
@@ -389,8 +400,8 @@ __global__ __launch_bounds__(64 * ATTN_PROJ_WAVES) void triattn_proj_k(const T* 
   __syncthreads();
   const int l = threadIdx.x & 63, g = l >> 4, r = l & 15;
   const int64_t NN = N * N;
-  const int tpr = (int)(ldk / TW), ntiles = (int)N * tpr, stride = gridDim.x * ATTN_PROJ_WAVES;
-  int t = grid_wave(ATTN_PROJ_WAVES);
+  const int tpr = (int)(ldk / TW), ntiles = (int)N * tpr, stride = (int)(gridDim.x / NG) * ATTN_PROJ_WAVES;
+  int t = __builtin_amdgcn_readfirstlane(wg * ATTN_PROJ_WAVES + (int)(threadIdx.x >> 6));
   if (t >= ntiles) return;
 
   typename RG<T, KIN>::frag x[RB][STEPS];
@@ -409,8 +420,8 @@ __global__ __launch_bounds__(64 * ATTN_PROJ_WAVES) void triattn_proj_k(const T* 
     load(min(t + stride, ntiles - 1), xnext);
     // ROWS orientation: key j0 + RUN g + 4 rb + e is inside the row
     const auto valid = [&](int rb, int e) { return j0 + RT::RUN * g + 4 * rb + e < N ? 1.0f : 0.0f; };
-    for (int R = 0; R < ATTN_ROWS; R += 32) {
-      const T* wb = Ws + R * LDW;
+    for (int R = r_lo; R < r_hi; R += 32) {
+      const T* wb = Ws + (R - r_lo) * LDW;
       if (R >= 4 * D) {  // triangle bias (16-row block, H valid rows)
         f4 acc[RB][1];
         zero_acc(acc);
@@ -835,14 +846,24 @@ __global__ __launch_bounds__(64 * TRW, 8 / TRW) void transition_f16_k(const half
 
 // ---------------------------------------------------------------- launchers
 
-template <int HV, int KIN, typename T = half_t>
-static hipError_t tm_proj_hv(const void* xn, const void* w, const float* mask, float scale, int incoming, void* ab,
-                             int64_t N, int64_t ld, int resident, hipStream_t st) {
-  const int64_t ntiles = N * (ld / (HV * RunTile<T>::TW));  // ld is a multiple of 64
-  if (ntiles >= (1LL << 30)) return hipErrorInvalidValue;  // tile indices are 32-bit in the kernel
-  const dim3 grid((unsigned)std::min<int64_t>(resident, (ntiles + PROJ_WAVES - 1) / PROJ_WAVES));
-  trimul_proj_k<T, HV, KIN><<<grid, 64 * PROJ_WAVES, 0, st>>>(static_cast<const T*>(xn), static_cast<const T*>(w), mask,
-                                                        scale, incoming, static_cast<T*>(ab), N, ld);
+// Weight groups of a projection launch: the most whose tiles still fit one round of the GPU's waves. us at 128 channels, 1 /
+// 2 / 4 groups, trimul and attention projection (2,048 and 3,072 waves): N = 48 (96 tiles) 12.1 / 8.1 / 6.3 and 19.5 /
+// 13.0 / 10.3; N = 128 (512) 13.9 / 10.1 / 8.4 and 21.9 / 15.4 / 12.6; N = 160 (960) 14.7 / 10.7 / 11.7 and 20.4 / 14.2 /
+// 16.5; N = 203 (1,624) 16.5 / 16.5 / 17.5 and 21.7 / 23.4 / 21.8.
+static int weight_groups(int64_t ntiles, int64_t grid_waves) {
+  return 4 * ntiles <= grid_waves ? 4 : 2 * ntiles <= grid_waves ? 2 : 1;
+}
+
+template <int HV, int KIN, int NG, typename T = half_t>
+static hipError_t tm_proj_g(const void* xn, const void* w, const float* mask, float scale, int incoming, void* ab,
+                            int64_t N, int64_t ld, int64_t ntiles, hipStream_t st) {
+  static int cache[kMaxDevices];
+  const int resident = resident_grid(trimul_proj_k<T, HV, KIN, NG>, 64 * PROJ_WAVES, cache);
+  if (resident <= 0) return hipErrorInvalidDevice;
+  const unsigned grid = NG > 1 ? group_grid(resident, NG, ntiles, PROJ_WAVES)
+                               : (unsigned)std::min<int64_t>(resident, (ntiles + PROJ_WAVES - 1) / PROJ_WAVES);
+  trimul_proj_k<T, HV, KIN, NG><<<grid, 64 * PROJ_WAVES, 0, st>>>(static_cast<const T*>(xn), static_cast<const T*>(w),
+                                                                  mask, scale, incoming, static_cast<T*>(ab), N, ld);
   return hipGetLastError();
 }
 
@@ -851,14 +872,19 @@ static hipError_t tm_proj(const void* xn, const void* w, const float* mask, floa
                           int64_t N, int64_t ld, hipStream_t st) {
   static int cache[kMaxDevices];
   // both tile forms have the same resources (the LDS weights and 8 waves set the occupancy)
-  const int resident = resident_grid(trimul_proj_k<T, 2, KIN>, 64 * PROJ_WAVES, cache);
+  const int resident = resident_grid(trimul_proj_k<T, 2, KIN, 1>, 64 * PROJ_WAVES, cache);
   if (resident <= 0) return hipErrorInvalidDevice;
   // rounds of full tiles on the resident waves, against rounds of half tiles (counted in full tiles, with 10% for
   // the half tile's own overhead)
-  const int64_t waves = (int64_t)resident * PROJ_WAVES, full = N * (ld / (2 * RunTile<T>::TW));
+  const int64_t waves = (int64_t)resident * PROJ_WAVES, full = N * (ld / (2 * RunTile<T>::TW));  // ld: a multiple of 64
+  if (full >= (1LL << 29)) return hipErrorInvalidValue;  // tile indices are 32-bit in the kernel
   const int64_t r2 = (full + waves - 1) / waves, r1x2 = (2 * full + waves - 1) / waves;
-  return 10 * r1x2 < 18 * r2 ? tm_proj_hv<1, KIN>(xn, w, mask, scale, incoming, ab, N, ld, resident, st)
-                             : tm_proj_hv<2, KIN>(xn, w, mask, scale, incoming, ab, N, ld, resident, st);
+  if (10 * r1x2 >= 18 * r2) return tm_proj_g<2, KIN, 1>(xn, w, mask, scale, incoming, ab, N, ld, full, st);
+  switch (weight_groups(2 * full, waves)) {
+    case 4: return tm_proj_g<1, KIN, 4>(xn, w, mask, scale, incoming, ab, N, ld, 2 * full, st);
+    case 2: return tm_proj_g<1, KIN, 2>(xn, w, mask, scale, incoming, ab, N, ld, 2 * full, st);
+    default: return tm_proj_g<1, KIN, 1>(xn, w, mask, scale, incoming, ab, N, ld, 2 * full, st);
+  }
 }
 
 hipError_t launch_trimul_proj(const void* xn, const void* w, const float* mask, float scale, int incoming, void* ab,
@@ -888,13 +914,17 @@ static hipError_t tm_tail_f16(const void* o, const float* now, const float* nob,
   static int cache[kMaxDevices];
   const int resident = resident_grid(trimul_tail_f16_k<KIN>, 64 * TAIL_WAVES, cache);
   if (resident <= 0) return hipErrorInvalidDevice;
-  const int64_t ntiles = N * tail_tiles_per_row(N);  // the last tile of a row ends at ld (ld = N rounded up to 64)
+  // tiles of whole 64-position groups per row, or (where that saves one of the first rounds: N = 203, 1 round for 2, 27.4
+  // to 19.1 us) only those that hold positions
+  const int64_t round = (int64_t)resident * TAIL_WAVES, t4 = (N + 63) / 64 * 4, t1 = (N + 15) / 16;
+  const int64_t r4 = (N * t4 + round - 1) / round, r1 = (N * t1 + round - 1) / round;
+  const int64_t tpr = r1 < r4 && r4 <= 4 ? t1 : t4, ntiles = N * tpr;  // a row's last tile ends inside ld
   if (ntiles >= (1LL << 30)) return hipErrorInvalidValue;  // tile indices are 32-bit in the kernel
   const dim3 grid((unsigned)std::min<int64_t>(resident, (ntiles + TAIL_WAVES - 1) / TAIL_WAVES));
   trimul_tail_f16_k<KIN><<<grid, 64 * TAIL_WAVES, 0, st>>>(static_cast<const half_t*>(o), now, nob, eps_out,
                                                       static_cast<const half_t*>(w_po), static_cast<const half_t*>(xn),
                                                       static_cast<const half_t*>(w_go), z, accumulate, lnw, lnb,
-                                                      eps_next, static_cast<half_t*>(xn_next), N, ld);
+                                                      eps_next, static_cast<half_t*>(xn_next), N, ld, (int)tpr);
   return hipGetLastError();
 }
 
@@ -918,20 +948,34 @@ hipError_t launch_trimul_tail(const void* o, const float* now, const float* nob,
                                                     eps_next, xn_next, N, ld, st);
 }
 
+template <int KIN, int NG, typename T = half_t>
+static hipError_t ta_proj_g(const void* xn, const void* w, int trans, float q_scale, float b_scale, void* qkg, void* vt,
+                            void* tb, int64_t N, int64_t ldk, int H, int C, int64_t ntiles, hipStream_t st) {
+  static int cache[kMaxDevices];
+  const int resident = resident_grid(triattn_proj_k<T, KIN, NG>, 64 * ATTN_PROJ_WAVES, cache);
+  if (resident <= 0) return hipErrorInvalidDevice;
+  const unsigned grid = NG > 1 ? group_grid(resident, NG, ntiles, ATTN_PROJ_WAVES)
+                               : (unsigned)std::min<int64_t>(resident, (ntiles + ATTN_PROJ_WAVES - 1) / ATTN_PROJ_WAVES);
+  triattn_proj_k<T, KIN, NG><<<grid, 64 * ATTN_PROJ_WAVES, 0, st>>>(
+      static_cast<const T*>(xn), static_cast<const T*>(w), trans, q_scale, b_scale, static_cast<T*>(qkg),
+      static_cast<T*>(vt), static_cast<T*>(tb), N, ldk, H, C);
+  return hipGetLastError();
+}
+
 template <int KIN, typename T = half_t>
 static hipError_t ta_proj(const void* xn, const void* w, int trans, float q_scale, float b_scale, void* qkg, void* vt,
                           void* tb, int64_t N, int64_t ldk, int H, int C, hipStream_t st) {
   if (H * C != D || H > 16 || C % 8) return hipErrorInvalidValue;
   static int cache[kMaxDevices];
-  const int resident = resident_grid(triattn_proj_k<T, KIN>, 64 * ATTN_PROJ_WAVES, cache);
+  const int resident = resident_grid(triattn_proj_k<T, KIN, 1>, 64 * ATTN_PROJ_WAVES, cache);
   if (resident <= 0) return hipErrorInvalidDevice;
   const int64_t ntiles = N * (ldk / RunTile<T>::TW);  // ldk is a multiple of 64
   if (ntiles >= (1LL << 30)) return hipErrorInvalidValue;  // tile indices are 32-bit in the kernel
-  const dim3 grid((unsigned)std::min<int64_t>(resident, (ntiles + ATTN_PROJ_WAVES - 1) / ATTN_PROJ_WAVES));
-  triattn_proj_k<T, KIN><<<grid, 64 * ATTN_PROJ_WAVES, 0, st>>>(
-      static_cast<const T*>(xn), static_cast<const T*>(w), trans, q_scale, b_scale, static_cast<T*>(qkg),
-      static_cast<T*>(vt), static_cast<T*>(tb), N, ldk, H, C);
-  return hipGetLastError();
+  switch (weight_groups(ntiles, (int64_t)resident * ATTN_PROJ_WAVES)) {
+    case 4: return ta_proj_g<KIN, 4>(xn, w, trans, q_scale, b_scale, qkg, vt, tb, N, ldk, H, C, ntiles, st);
+    case 2: return ta_proj_g<KIN, 2>(xn, w, trans, q_scale, b_scale, qkg, vt, tb, N, ldk, H, C, ntiles, st);
+    default: return ta_proj_g<KIN, 1>(xn, w, trans, q_scale, b_scale, qkg, vt, tb, N, ldk, H, C, ntiles, st);
+  }
 }
 
 hipError_t launch_triattn_proj(const void* xn, const void* w, int trans, float q_scale, float b_scale, void* qkg,

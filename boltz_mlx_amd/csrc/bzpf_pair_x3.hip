@@ -26,15 +26,6 @@ namespace {
 constexpr int XW = 8, XT = 64 * XW;  // waves and threads of the persistent workgroups (2 per SIMD: 256 VGPRs)
 constexpr int XTW = 32;              // positions of a wave tile: two row blocks of 16
 
-// Block b of a launch over NG weight groups -> (group, workgroup within the group): the NG groups of one workgroup index
-// are blocks of one XCD (block b runs on XCD b % 8), so the x rows they share are fetched into its L2 once.
-template <int NG>
-__device__ __forceinline__ void xgroup(int& grp, int& wg) {
-  const int b = blockIdx.x, q = b >> 3;
-  grp = q % NG;
-  wg = q / NG * 8 + (b & 7);
-}
-
 // ---------------------------------------------------------------- triangle multiplication projection
 // A workgroup holds 64 projection and their 64 gate rows (104 KB of LDS at KIN = 128; all 256 + 256 rows in three parts
 // would take 418 KB) and streams tiles of 32 positions (i, k0 .. k0 + 31) of the padded rows; the 2 KIN / 64 groups of
@@ -46,7 +37,7 @@ __global__ __launch_bounds__(XT) void trimul_proj_x3_k(const float* __restrict__
   constexpr int NG = 2 * KIN / 64, PLANE_W = 128 * ldx<KIN>();
   __shared__ LDS_ALIGN __bf16 Ws[3 * PLANE_W];
   int grp, wg;
-  xgroup<NG>(grp, wg);
+  weight_group<NG>(grp, wg);
   const int nwg = (int)gridDim.x / NG, c_lo = 64 * grp;
   const int tpr = (int)(ld / XTW), ntiles = (int)N * tpr, stride = nwg * XW;
   if (wg * XW >= ntiles) return;  // whole workgroup
@@ -108,7 +99,7 @@ __global__ __launch_bounds__(XT) void triattn_proj_x3_k(const float* __restrict_
   constexpr int HC = 128, PLANE_W = (HC + 16) * ldx<KIN>();
   __shared__ LDS_ALIGN __bf16 Ws[3 * PLANE_W];
   int grp, wg;
-  xgroup<4>(grp, wg);
+  weight_group<4>(grp, wg);
   const int tpr = (int)(ldk / XTW), ntiles = (int)N * tpr, stride = (int)(gridDim.x / 4) * XW;
   if (wg * XW >= ntiles) return;  // whole workgroup
   const int l = threadIdx.x & 63, g = l >> 4, r = l & 15;
@@ -574,14 +565,6 @@ __global__ __launch_bounds__(XT) void transition_x3_small_k(const float* __restr
 template <typename Kern>
 int x3_resident(Kern kernel, int (&cache)[kMaxDevices]) { return resident_grid(kernel, XT, cache); }
 
-// Grid of a launch over `groups` weight groups: whole sets of 8 x groups blocks (xgroup), at most one round of resident
-// workgroups, no more than the tiles need.
-unsigned x3_grid(int resident, int groups, int64_t ntiles) {
-  const int64_t wgs = (ntiles + XW - 1) / XW, unit = 8 * groups;
-  const int64_t need = (wgs + 7) / 8, have = resident / unit > 0 ? resident / unit : 1;
-  return (unsigned)(std::min(need, have) * unit);
-}
-
 template <int KIN>
 hipError_t proj_x3(const float* xn, const float* w, const float* mask, float scale, int incoming, float* ab, int64_t N,
                    int64_t ld, hipStream_t st) {
@@ -590,7 +573,7 @@ hipError_t proj_x3(const float* xn, const float* w, const float* mask, float sca
   if (resident <= 0) return hipErrorInvalidDevice;
   const int64_t ntiles = N * (ld / XTW);
   if (ntiles >= (1LL << 30)) return hipErrorInvalidValue;  // tile indices are 32-bit in the kernel
-  trimul_proj_x3_k<KIN><<<x3_grid(resident, 2 * KIN / 64, ntiles), XT, 0, st>>>(xn, w, mask, scale, incoming, ab, N, ld);
+  trimul_proj_x3_k<KIN><<<group_grid(resident, 2 * KIN / 64, ntiles, XW), XT, 0, st>>>(xn, w, mask, scale, incoming, ab, N, ld);
   return hipGetLastError();
 }
 
@@ -614,7 +597,7 @@ hipError_t attn_proj_x3(const float* xn, const float* w, int trans, float q_scal
   if (resident <= 0) return hipErrorInvalidDevice;
   const int64_t ntiles = N * (ldk / XTW);
   if (ntiles >= (1LL << 30)) return hipErrorInvalidValue;
-  triattn_proj_x3_k<KIN><<<x3_grid(resident, 4, ntiles), XT, 0, st>>>(xn, w, trans, q_scale, b_scale, qkg, vt, tb, N,
+  triattn_proj_x3_k<KIN><<<group_grid(resident, 4, ntiles, XW), XT, 0, st>>>(xn, w, trans, q_scale, b_scale, qkg, vt, tb, N,
                                                                       ldk, H, C);
   return hipGetLastError();
 }

@@ -101,14 +101,21 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 template <typename T, typename RowFn>
 __device__ __forceinline__ void lds_rows(T* dst, int ld, int rows, int k, RowFn src) {
-  constexpr int VE = 16 / sizeof(T);
-  const int per = k / VE;
-  for (int e = threadIdx.x; e < rows * per; e += blockDim.x) {
-    const int r = e / per, c = (e - r * per) * VE;
-    const T* s = src(r);
-    u32x4 v = u32x4{0u, 0u, 0u, 0u};
-    if (s) v = *reinterpret_cast<const u32x4*>(s + c);
-    *reinterpret_cast<u32x4*>(dst + r * ld + c) = v;
+  constexpr int VE = 16 / sizeof(T), BATCH = 8;  // a batch's loads are issued together: one round trip, not eight
+  const int per = k / VE, total = rows * per, step = blockDim.x;
+  for (int e0 = threadIdx.x; e0 < total; e0 += BATCH * step) {
+    u32x4 v[BATCH];
+#pragma unroll
+    for (int b = 0; b < BATCH; b++) {
+      const int e = min(e0 + b * step, total - 1), r = e / per, c = (e - r * per) * VE;
+      const T* s = src(r);
+      v[b] = s ? *reinterpret_cast<const u32x4*>(s + c) : u32x4{0u, 0u, 0u, 0u};
+    }
+#pragma unroll
+    for (int b = 0; b < BATCH; b++) {
+      const int e = e0 + b * step, r = e / per, c = (e - r * per) * VE;
+      if (e < total) *reinterpret_cast<u32x4*>(dst + r * ld + c) = v[b];
+    }
   }
 }
 
@@ -355,6 +362,22 @@ __device__ __forceinline__ void resid_ln_pb_rows(const f4 (&y)[RB][8], ZRow zrow
 // uniform by itself, and tile coordinates derived from it would otherwise live (and be divided) in vector registers.
 __device__ __forceinline__ int grid_wave(int waves_per_block) {
   return __builtin_amdgcn_readfirstlane((int)(blockIdx.x * waves_per_block + (threadIdx.x >> 6)));
+}
+
+// Block b of a launch over NG weight groups -> (group, workgroup within the group): the NG groups of one workgroup index
+// are blocks of one XCD (block b runs on XCD b % 8), so the x rows they share are fetched into its L2 once. The grid is a
+// multiple of 8 NG blocks.
+template <int NG>
+__device__ __forceinline__ void weight_group(int& grp, int& wg) {
+  const int b = blockIdx.x, q = b >> 3;
+  grp = q % NG;
+  wg = q / NG * 8 + (b & 7);
+}
+// That grid for ntiles wave tiles: at most one round of resident workgroups, no more than the tiles need.
+static inline unsigned group_grid(int resident, int groups, int64_t ntiles, int waves) {
+  const int64_t wgs = (ntiles + waves - 1) / waves, unit = 8 * groups;
+  const int64_t need = (wgs + 7) / 8, have = resident / unit > 0 ? resident / unit : 1;
+  return (unsigned)((need < have ? need : have) * unit);
 }
 
 // Persistent launches: each wave walks tiles wave_id, wave_id + waves_in_grid, ... so the grid is sized to what stays

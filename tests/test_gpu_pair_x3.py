@@ -119,6 +119,46 @@ def test_linear_resid_ln(N, D):
                 assert _rel(xo.view(N, N, D), _ln(want, ln)) < TOL
 
 
+# the fp16 projections with 4, 2 and 1 weight groups: both sides of the tile counts where each form ends (512 and 1,024
+# tiles of 32 positions on 2,048 waves, 768 and 1,536 on 3,072), and the fp16 tail with and without empty tiles
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("N", [3, 100, 128, 129, 150, 170, 171, 203])
+def test_f16_projections_and_tail(N, D):
+    """Against float64 from the fp16 operands. The largest error of an fp16 store is 2^-11 of the value; 2^-9 of the largest
+    value leaves room for the fp16 LayerNorm output and gates inside the tail."""
+    from boltz_mlx_amd import kernels as K
+
+    K.set_precision("f16")
+    randn, ln = _make(N, D)
+    half = lambda *s: (randn(*s) * (s[-1] ** -0.5 if s[0] != N * N else 1.0)).half()
+    close = lambda a, ref: ((a.double() - ref).abs().max() <= ref.abs().max() * 2.0 ** -9).item()
+    proj, attn, tail = (K.trimul_proj64, K.triattn_proj64, K.trimul_tail64) if D == 64 else (
+        K.trimul_proj, K.triattn_proj, K.trimul_tail)
+    xn, w, wq = half(N * N, D), half(4 * D, D), half(4 * 128 + 4, D)
+    mask = (torch.rand((N, N), device="cuda") > 0.2).float()
+    p, gate = (xn.double() @ w.double().T).view(N, N, 4 * D).split(2 * D, -1)
+    ref = (p * torch.sigmoid(gate) * mask.double()[..., None]).permute(2, 0, 1)
+    q, k, v, g, b = (xn.double() @ wq.double().T).view(N, N, -1).split([128] * 4 + [4], -1)
+    off = torch.from_numpy(K.tri_bias_offsets(N, 4)).cuda()
+    for flip in (False, True):
+        turn = (lambda t: t.transpose(0, 1)) if flip else (lambda t: t)
+        ab = proj(xn, w, mask, 1.0, flip, N)
+        assert close(ab[..., :N], ref.transpose(1, 2) if flip else ref) and not ab[..., N:].any()
+        qkg, vt, tb = attn(xn, wq, flip, N, 4, 32)
+        heads = lambda t: turn(t).reshape(N * N, 4, 32).transpose(0, 1)
+        assert close(qkg, torch.cat([heads(q) * LOG2E / 32 ** 0.5, heads(k), heads(g)]))
+        assert close(vt[..., :N], turn(v).reshape(N, N, 4, 32).permute(2, 0, 3, 1)) and not vt[..., N:].any()
+        assert close(tb[off], turn(b).permute(2, 0, 1) * LOG2E)
+    with torch.no_grad():
+        o = torch.zeros((D, N, K.row_pitch(N)), device="cuda", dtype=torch.float16)
+        o[..., :N] = (randn(D, N, N) * 3).half()
+        w_po, w_go, z = half(D, D), half(D, D), torch.full((N, N, D), float("nan"), device="cuda")
+        y = (_ln(o[..., :N].double().permute(1, 2, 0), ln) @ w_po.double().T) * torch.sigmoid(
+            xn.double() @ w_go.double().T).view(N, N, D)
+        tail(o, ln, ln.eps, w_po, xn, w_go, z, False, None, N)
+        assert close(z, y)
+
+
 # masks whose last live column and row fall inside, at and past a 64-lane step; no live entry; one live entry
 @pytest.mark.parametrize("N,rows,cols", [(1, 1, 1), (5, 0, 0), (64, 40, 64), (65, 65, 1), (130, 64, 65), (200, 129, 70)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
