@@ -538,6 +538,20 @@ hipError_t launch_gemm_swiglu_f16(const void* x, const void* w, void* u, int64_t
           0, nullptr, 0, 1, (int)nr, (int)nm, per_xcd, mfast);
     return hipGetLastError();
   }
+  // fewer rows, three products: 192 x 64 tiles of the same form (us: 1200 rows 16.5 -> 13.6, 800 14.8 -> 11.8 in two
+  // stages; 400 10.3 -> 9.0, 64 10.0 -> 8.9 in three, 9.7 and 10.0 in two)
+  if (np == 3 && H % 64 == 0) {
+    const int64_t nr = (R + 63) / 64, nm = H / 64;
+    if (nr * nm >= (1LL << 31) - 8 || (int64_t)192 * K * 2 > 0x7fffffffLL) return hipErrorInvalidValue;
+    const int per_xcd = (int)((nr * nm + 7) / 8), mfast = xb / 8 + wb <= xb + wb / 8;
+    const auto run = [&](auto kernel) {
+      kernel<<<(unsigned)(8 * per_xcd), 256, 0, st>>>(static_cast<const half_t*>(x), static_cast<const half_t*>(w),
+                                                      nullptr, static_cast<half_t*>(u), R, K, 3 * H, 0, nullptr, 0, 1,
+                                                      (int)nr, (int)nm, per_xcd, mfast);
+      return hipGetLastError();
+    };
+    return R >= 640 ? run(gemm_lds_k<192, 64, 2, half_t, 3>) : run(gemm_lds_k<192, 64, 3, half_t, 3>);
+  }
   const int64_t nr = (R + 127) / 128, nq = H / 32;
   if (nr * nq >= (1LL << 31) - 8) return hipErrorInvalidValue;
   const int per_xcd = (int)((nr * nq + 7) / 8);
@@ -569,19 +583,23 @@ hipError_t launch_gemm_nt(const void* x, const void* w, const float* bias, void*
     return hipErrorInvalidValue;
   if (x_dt == DT_F32)  // fp32 operands: 64 x 64 tiles (the m track's 409,600-row projections)
     return gemm_t<64, 64, float>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st);
-  // below the large-grid case, for 2048 rows and more, the LDS-direct form with 3 stages (2 in flight) takes the
-  // same tiles: the diffusion transformer's 2000 x 768 -> 3072 projection 24.4 -> 22.1 us (128 x 64), its 768-wide
-  // gated outputs 12.6 -> 11.7 and 17.2 -> 16.1 us (64 x 64). Same sums in the same order. The s track's GEMMs
-  // (N rows) keep the register-staged form: they run beside the attention core, and there the LDS-direct form's
-  // workgroups found compute units far later (0.85 ms against 0.04 ms per launch at N = 1000).
+  // below the large-grid case the LDS-direct form takes the same tiles, for 1536 rows and more and for the diffusion
+  // transformer's GEMMs at any row count (the gated outputs, epi 2, and the wide projections of K >= 768): 64 x 64 in
+  // three stages, or 64 W rows x 128 x rows in two for the wide ones from 640 rows on. Measured in a graph over 24
+  // layers' weights, us: 2000 x 768 -> 3072 19.7 (192 x 128, three stages) -> 16.4 (a library's 16.6), 1200 rows 17.3
+  // (register-staged) -> 12.1, 800 13.5 -> 10.7, 400 10.2 -> 7.8 (64 x 64; 9.3 on 64 x 128), 200 6.6 -> 6.4; gated 768 ->
+  // 768 and 1536 -> 768 at 400 rows 7.9 -> 7.0 and 11.4 -> 9.9. Same sums in the same order. The s track's GEMMs (N rows,
+  // epi 0 of K = 384 and epi 1) keep the register-staged form: they run beside the attention core, and there the
+  // LDS-direct form's workgroups found compute units far later (0.85 ms against 0.04 ms per launch at N = 1000).
   // 128 columns over many rows (the outer product mean's proj_o, 160,000 x 1024 -> 128 at N = 400): one 128-wide
   // column tile, so each x row is read once (124.8 against 148.0 us on 64 x 64 tiles; 128 x 64 and 64 x 128 with
   // three stages 130.5 and 129.0)
   if (M == 128 && R >= 65536)
     return gemm_lds_t<128, 128, 2>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st);
-  if (gemm_tile_choice(R, M) != 0 && R >= 1536)
-    return M >= 2048 ? gemm_lds_t<192, 128, 3>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st)
-                     : gemm_lds_t<64, 64, 3>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st);
+  if (gemm_tile_choice(R, M) != 0 && (R >= 1536 || epi == 2 || (K >= 768 && M >= 2048)))
+    return M >= 2048 && R >= 640
+               ? gemm_lds_t<64, 128, 2>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st)
+               : gemm_lds_t<64, 64, 3>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st);
   switch (gemm_tile_choice(R, M)) {
     case 0: return gemm_t<128, 128, half_t>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st);
     case 1: return gemm_t<128, 64, half_t>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st);
