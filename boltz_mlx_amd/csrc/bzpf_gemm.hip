@@ -581,6 +581,12 @@ hipError_t launch_gemm_nt(const void* x, const void* w, const float* bias, void*
   if ((x_dt != DT_F16 && x_dt != DT_F32) || !gemm_nt_ok(x_dt, x, w, bias, y, R, K, M, gate, ld_gate) || epi < 0 ||
       epi > 3 || (epi >= 1 && y_dt != DT_F32) || (epi >= 2 && (gate == nullptr || gate_rows < 1)))
     return hipErrorInvalidValue;
+  // fp32 over few rows: up to 768 tiles of 16 columns x 32 rows, K split over a workgroup's waves (us, against the 64 x
+  // 64-tile form: 128 rows 384 -> 1536 (384 tiles) 6.5 / 10.0, 384 -> 3072 (768) 9.1 / 10.6, 1536 -> 384 (96) 10.3 / 31.1;
+  // 203 rows 384 -> 3072 (1,344) 14.5 / 11.0; 1000 rows 1536 -> 384 (768) 27.3 / 32.0, 1500 (1,128) 42.3 / 32.2)
+  if (x_dt == DT_F32 && (int64_t)((M + 15) / 16) * ((R + 31) / 32) <= 768)
+    return launch_linear_x3_small(static_cast<const float*>(x), static_cast<const float*>(w), bias, y, y_dt, R, K, M,
+                                  epi, gate, ld_gate, gate_rows, st);
   if (x_dt == DT_F32)  // fp32 operands: 64 x 64 tiles (the m track's 409,600-row projections)
     return gemm_t<64, 64, float>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st);
   // below the large-grid case the LDS-direct form takes the same tiles, for 1536 rows and more and for the diffusion

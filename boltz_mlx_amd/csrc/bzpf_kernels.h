@@ -32,6 +32,9 @@ hipError_t launch_linear_resid_ln_x3(const float* x, const float* w, int trans, 
 hipError_t launch_transition_x3(const float* xn, const float* w12, const float* w3, float* z, int accumulate,
                                 const float* lnw, const float* lnb, float eps, float* xn_next, int64_t rows,
                                 int hidden, hipStream_t st);
+hipError_t launch_linear_x3_small(const float* x, const float* w, const float* bias, void* y, int y_dt, int64_t R, int K,
+                                  int M, int epi, const float* gate, int64_t ld_gate, int64_t gate_rows,
+                                  hipStream_t st);
 hipError_t launch_trimul_contract(const void* ab, void* o, int dt, int64_t N, int64_t ld, int64_t k_len, const int* ext,
                                   int D, hipStream_t st);
 hipError_t launch_key_extents(const float* mask, int64_t N, int* ext, hipStream_t st);

@@ -202,3 +202,23 @@ def test_transition(rows, hidden):
             assert _rel(z, want) < TOL
             if nxt is not None:
                 assert _rel(xo.view(rows, 1, 128), _ln(want, ln)) < TOL
+
+
+# fp32 Linear over few rows: one row, ends of its 16- and 32-row tiles, a column count that ends inside a tile, fewer steps of
+# 32 k than waves and more, and both sides of its largest grid (768 tiles of 16 columns x 32 rows)
+@pytest.mark.parametrize("R,k,M", [(1, 384, 1536), (16, 32, 4), (17, 64, 20), (33, 288, 36), (128, 1536, 384),
+                                   (128, 384, 3072), (129, 384, 3072), (1024, 384, 384), (1025, 384, 384)])
+def test_linear_few_rows(R, k, M):
+    from boltz_mlx_amd import kernels as K
+
+    g = torch.Generator(device="cuda").manual_seed(R + k + M)
+    randn = lambda *s: torch.randn(s, generator=g, device="cuda")
+    x, w, b, y0 = randn(R, k), randn(M, k) * k ** -0.5, randn(M), randn(R, M)
+    ref = x.double() @ w.double().T + b.double()
+    assert _rel(K.linear(x, w, bias=b), ref) < TOL
+    assert _rel(K.linear(x, w, bias=b, out_dtype=torch.float16), ref) < 2.0 ** -11
+    assert _rel(K.linear(x, w, bias=b, out=y0.clone(), accumulate=True), y0.double() + ref) < TOL
+    gate = randn((R + 2) // 3, M)
+    sig = torch.sigmoid(gate.double())[torch.arange(R, device="cuda") % gate.shape[0]]
+    assert _rel(K.linear_gated(x, w, gate, y0.clone(), bias=b), y0.double() + sig * ref) < TOL
+    assert _rel(K.linear_residual(x, w, y0, torch.empty_like(y0), bias=b), y0.double() + ref) < TOL
