@@ -34,20 +34,28 @@ __device__ __forceinline__ int contract_stages(int all, int bk, const int* ext, 
 
 // ext[0] = 1 + the last column with a nonzero in any row of mask [N][N], ext[1] = 1 + the last row with a nonzero (both 0
 // before the launch). A wave takes a row and scans it from its end, so a mask of leading real tokens is read for its
-// padded part and one step more.
+// padded part and one step more. The maxima go out once a workgroup, and only where they raise what is there (an atomic a
+// row, all on two words, took 25 us at N = 1000; so 6.7).
 __global__ __launch_bounds__(256) void key_extents_k(const float* __restrict__ mask, int64_t N, int* __restrict__ ext) {
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= N) return;  // whole wave
-  const int l = threadIdx.x & 63;
-  const float* m = mask + row * N;
-  for (int64_t k0 = (N - 1) / 64 * 64; k0 >= 0; k0 -= 64) {
+  __shared__ int ks[4], rs[4];
+  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * 4 + wave;
+  const float* m = mask + min(row, N - 1) * N;
+  int kx = 0;
+  for (int64_t k0 = (N - 1) / 64 * 64; k0 >= 0 && kx == 0; k0 -= 64) {
     const uint64_t live = __ballot(k0 + l < N && m[min(k0 + l, N - 1)] != 0.0f);
-    if (live == 0) continue;
-    if (l == 0) {
-      atomicMax(ext, (int)(k0 + 64 - __clzll((long long)live)));
-      atomicMax(ext + 1, (int)(row + 1));
-    }
-    return;
+    if (live != 0) kx = (int)(k0 + 64 - __clzll((long long)live));
+  }
+  if (l == 0) {
+    ks[wave] = row < N ? kx : 0;
+    rs[wave] = row < N && kx > 0 ? (int)(row + 1) : 0;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    const int* v = threadIdx.x == 0 ? ks : rs;
+    const int top = max(max(v[0], v[1]), max(v[2], v[3]));
+    if (top > __hip_atomic_load(ext + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(ext + threadIdx.x, top);
   }
 }
 
