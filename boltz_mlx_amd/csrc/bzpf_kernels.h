@@ -29,6 +29,8 @@ hipError_t launch_triattn_proj_x3(const float* xn, const float* w, int trans, fl
 hipError_t launch_linear_resid_ln_x3(const float* x, const float* w, int trans, float* z, int accumulate,
                                      const float* lnw, const float* lnb, float eps, float* xn_next, int64_t N, int dim,
                                      hipStream_t st);
+hipError_t launch_pair_bias_x3(const float* z, const float* lnw, const float* lnb, float eps, const float* w, float* out,
+                               int64_t rows, int H, hipStream_t st);
 hipError_t launch_transition_x3(const float* xn, const float* w12, const float* w3, float* z, int accumulate,
                                 const float* lnw, const float* lnb, float eps, float* xn_next, int64_t rows,
                                 int hidden, hipStream_t st);

@@ -346,6 +346,64 @@ __global__ __launch_bounds__(XT) void linear_resid_ln_x3_k(const float* __restri
   }
 }
 
+// ---------------------------------------------------------------- pair bias = Linear(LN(z)) as [H][rows]
+// (boltz_mlx/layers/attentionv2.py:40-48.) Persistent and bound by its read of z: a wave holds W's fragments (16 rows, H of
+// them used) and streams tiles of 16 rows, the next tile loaded ahead; a row's LayerNorm stays in its four lanes. 160,000
+// rows 36 us (through LDS, fp32 MFMA) -> 25, 263,169 rows 56 -> 35 (z's 135 MB at 5.2 TB/s: 26).
+__global__ __launch_bounds__(256, 2) void pair_bias_x3_k(const float* __restrict__ z, const float* __restrict__ lnw,
+                                                         const float* __restrict__ lnb, float eps,
+                                                         const float* __restrict__ w, float* __restrict__ out,
+                                                         int64_t rows, int H) {
+  constexpr int D = 128;
+  __shared__ LnLds lns;
+  const int ntiles = (int)((rows + 15) / 16), stride = gridDim.x * 4;
+  const int l = threadIdx.x & 63, g = l >> 4, r = l & 15;
+  int t = grid_wave(4);
+  RawRow<D> raw;
+  const auto load = [&](int tt) { raw.load(z + min((int64_t)tt * 16 + r, rows - 1) * D, g); };
+  load(min(t, ntiles - 1));
+  X3Row<D> wx;
+  {
+    RawRow<D> wr = {};
+    if (r < H) wr.load(w + (int64_t)r * D, g);
+    split_row(wx, wr);
+  }
+  stage_ln(lns, lnw, lnb);
+  __syncthreads();
+  for (; t < ntiles; t += stride) {
+    float sum = 0.f, ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < D / 16; j++) sum += raw.v[j][0] + raw.v[j][1] + raw.v[j][2] + raw.v[j][3];
+    const float mean = xgroups_sum(sum) * (1.0f / D);
+#pragma unroll
+    for (int j = 0; j < D / 16; j++) {
+      raw.v[j] = raw.v[j] - mean;
+      ss += raw.v[j][0] * raw.v[j][0] + raw.v[j][1] * raw.v[j][1] + raw.v[j][2] * raw.v[j][2] + raw.v[j][3] * raw.v[j][3];
+    }
+    const float rstd = 1.0f / sqrtf(xgroups_sum(ss) * (1.0f / D) + eps);
+#pragma unroll
+    for (int j = 0; j < D / 16; j++) {
+      const int c = D / 4 * g + 4 * j;
+      raw.v[j] = raw.v[j] * rstd * ld4(lns.w + c) + ld4(lns.b + c);
+    }
+    X3Row<D> x;
+    split_row(x, raw);
+    load(min(t + stride, ntiles - 1));
+    f4 acc = {};
+#pragma unroll
+    for (int q = 0; q < 6; q++)
+#pragma unroll
+      for (int s = 0; s < D / 32; s++) acc = mfma_x3<true>(wx.p[X3_W[q]][s], x.p[X3_X[q]][s], acc);
+    if (r < H) {
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int64_t p = (int64_t)t * 16 + 4 * g + e;
+        if (p < rows) out[(int64_t)r * rows + p] = acc[e];
+      }
+    }
+  }
+}
+
 // ---------------------------------------------------------------- transition
 // h1, h2 = fc1 / fc2 rows . xn (16-unit blocks), a = silu(h1) * h2 in the accumulator layout, split in place: the B
 // operand of out += fc3 a, a lane's k slots 8 g + t being units 16 (t / 4) + 4 g + t % 4 of a 32-unit slice.
@@ -641,6 +699,17 @@ hipError_t launch_linear_resid_ln_x3(const float* x, const float* w, int trans, 
                                      const float* lnw, const float* lnb, float eps, float* xn_next, int64_t N, int dim,
                                      hipStream_t st) {
   return (dim == 64 ? lrl_x3<64> : lrl_x3<128>)(x, w, trans, z, accumulate, lnw, lnb, eps, xn_next, N, st);
+}
+
+hipError_t launch_pair_bias_x3(const float* z, const float* lnw, const float* lnb, float eps, const float* w, float* out,
+                               int64_t rows, int H, hipStream_t st) {
+  static int cache[kMaxDevices];
+  const int resident = resident_grid(pair_bias_x3_k, 256, cache);
+  if (resident <= 0) return hipErrorInvalidDevice;
+  const int64_t ntiles = (rows + 15) / 16;
+  if (rows < 1 || H < 1 || H > 16 || ntiles >= (1LL << 30)) return hipErrorInvalidValue;
+  pair_bias_x3_k<<<(unsigned)std::min<int64_t>(resident, (ntiles + 3) / 4), 256, 0, st>>>(z, lnw, lnb, eps, w, out, rows, H);
+  return hipGetLastError();
 }
 
 hipError_t launch_transition_x3(const float* xn, const float* w12, const float* w3, float* z, int accumulate,

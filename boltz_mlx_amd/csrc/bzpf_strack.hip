@@ -254,13 +254,10 @@ __global__ __launch_bounds__(256) void pair_bias_kernel(const float* __restrict_
 hipError_t launch_pair_bias(const float* z, const float* lnw, const float* lnb, float eps, const void* w, void* out,
                             int dt, int64_t rows, int H, hipStream_t st) {
   if (H > 16) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)((rows + 63) / 64));
-  if (dt == DT_F16)
-    pair_bias_kernel<half_t><<<grid, 256, 0, st>>>(z, lnw, lnb, eps, static_cast<const half_t*>(w),
-                                                   static_cast<half_t*>(out), rows, H);
-  else
-    pair_bias_kernel<float><<<grid, 256, 0, st>>>(z, lnw, lnb, eps, static_cast<const float*>(w),
-                                                  static_cast<float*>(out), rows, H);
+  if (dt == DT_F32)
+    return launch_pair_bias_x3(z, lnw, lnb, eps, static_cast<const float*>(w), static_cast<float*>(out), rows, H, st);
+  pair_bias_kernel<half_t><<<(unsigned)((rows + 63) / 64), 256, 0, st>>>(
+      z, lnw, lnb, eps, static_cast<const half_t*>(w), static_cast<half_t*>(out), rows, H);
   return hipGetLastError();
 }
 

@@ -181,6 +181,18 @@ def test_key_extent_device(N, rows, cols, dtype):
     assert K.key_extent_device(mask, N, False) == 0
 
 
+# one row, the end of a 16-row tile, more tiles than resident waves (65,536 rows and more), few and all 16 heads
+@pytest.mark.parametrize("N,H", [(1, 16), (3, 4), (16, 8), (37, 16), (270, 16), (333, 1)])
+def test_pair_bias(N, H):
+    from boltz_mlx_amd import kernels as K
+
+    randn, ln = _make(N, 128)
+    z, w = randn(N, N, 128) * 2 + 1, randn(H, 128) * 128 ** -0.5
+    with torch.no_grad():
+        ref = (_ln(z.double(), ln) @ w.double().T).permute(2, 0, 1)
+        assert _rel(K.pair_bias(z, ln, w), ref) < TOL
+
+
 # rows: ends of the 16-, 32-, 128- and 256-row tiles, both sides of the row counts where the form changes, and whole
 # rounds of 65,536 rows with a remainder in each form
 @pytest.mark.parametrize("rows,hidden", [(1, 64), (15, 512), (17, 320), (4096, 512), (4097, 64), (16384, 64),
