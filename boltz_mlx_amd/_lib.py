@@ -53,8 +53,6 @@ SIGNATURES = {
     "bzpf_triattn_pack": [vp, i32, f32, f32, vp, vp, vp, i32, i64, i64, i32, i32, vp],
     "bzpf_opm_split": [vp, i64, vp, vp, i32, i32, vp],
     "bzpf_opm_ln_split": [vp, vp, vp, f32, vp, vp, vp, i32, i32, vp],
-    "bzpf_opm_ln_split2": [vp, vp, vp, f32, vp, vp, vp, vp, vp, i32, i32, vp],
-    "bzpf_opm_outer2": [vp, vp, vp, vp, i32, i32, i32, i32, vp],
     "bzpf_opm_outer": [vp, vp, vp, i32, i32, i32, i32, i32, vp],
     "bzpf_pwa_softmax": [vp, vp, f32, vp, i32, i64, i32, vp],
     "bzpf_transition64_f16": [vp, vp, vp, f32, vp, vp, i64, i32, vp],

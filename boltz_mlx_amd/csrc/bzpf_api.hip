@@ -506,32 +506,6 @@ int bzpf_opm_outer(const void* planes, const float* num, void* out, int out_dt, 
   return done(bzpf::launch_opm_outer(planes, num, out, out_dt, n_seq, N, i_base, n_i, S(stream)), "bzpf_opm_outer");
 }
 
-int bzpf_opm_ln_split2(const float* m, const float* ln_w, const float* ln_b, float eps, const float* w_ab,
-                       const float* mask, const float* num, void* planes, float* inv_scale, int n_seq, int N,
-                       void* stream) {
-  REQUIRE(m && ln_w && ln_b && w_ab && mask && num && planes && inv_scale, "bzpf_opm_ln_split2: NULL pointer");
-  REQUIRE(reinterpret_cast<uintptr_t>(m) % 16 == 0 && reinterpret_cast<uintptr_t>(w_ab) % 16 == 0 &&
-              reinterpret_cast<uintptr_t>(ln_w) % 16 == 0 && reinterpret_cast<uintptr_t>(ln_b) % 16 == 0 &&
-              reinterpret_cast<uintptr_t>(planes) % 16 == 0,
-          "bzpf_opm_ln_split2: m, w_ab, ln_w, ln_b and planes must be 16-byte aligned");
-  REQUIRE(n_seq >= 1 && n_seq <= 16 * 65535 && N >= 1 && (int64_t)N * 6144 <= INT32_MAX,
-          "bzpf_opm_ln_split2: bad sizes (n_seq=%d N=%d)", n_seq, N);
-  return done(bzpf::launch_opm_ln_split2(m, ln_w, ln_b, eps, w_ab, mask, num, planes, inv_scale, n_seq, N, S(stream)),
-              "bzpf_opm_ln_split2");
-}
-
-int bzpf_opm_outer2(const void* planes, const float* inv_scale, const float* num, void* out, int n_seq, int N,
-                    int i_base, int n_i, void* stream) {
-  REQUIRE(planes && inv_scale && num && out, "bzpf_opm_outer2: NULL pointer");
-  REQUIRE(reinterpret_cast<uintptr_t>(planes) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0,
-          "bzpf_opm_outer2: planes must be 16-byte and out 8-byte aligned");
-  REQUIRE(n_seq >= 1 && n_seq <= 16 * 65535 && N >= 1 && (int64_t)N * 6144 <= INT32_MAX && i_base >= 0 &&
-              n_i >= 1 && i_base + n_i <= N,
-          "bzpf_opm_outer2: bad sizes (n_seq=%d N=%d i_base=%d n_i=%d)", n_seq, N, i_base, n_i);
-  return done(bzpf::launch_opm_outer2(planes, inv_scale, num, out, n_seq, N, i_base, n_i, S(stream)),
-              "bzpf_opm_outer2");
-}
-
 int bzpf_transition64_f16(float* x, const float* ln_w, const float* ln_b, float eps, const void* w12, const void* w3,
                           int64_t rows, int hidden, void* stream) {
   REQUIRE(x && ln_w && ln_b && w12 && w3, "bzpf_transition64_f16: NULL pointer");

@@ -109,11 +109,6 @@ hipError_t launch_opm_split(const float* ab, int64_t ld_ab, const float* mask, v
                             hipStream_t st);
 hipError_t launch_opm_outer(const void* planes, const float* num, void* out, int out_dt, int S, int N, int i_base,
                             int n_i, hipStream_t st);
-hipError_t launch_opm_ln_split2(const float* m, const float* lnw, const float* lnb, float eps, const float* w_ab,
-                                const float* mask, const float* num, void* planes, float* inv_scale, int S, int N,
-                                hipStream_t st);
-hipError_t launch_opm_outer2(const void* planes, const float* inv_scale, const float* num, void* out, int S, int N,
-                             int i_base, int n_i, hipStream_t st);
 hipError_t launch_opm_ln_split(const float* m, const float* lnw, const float* lnb, float eps, const float* w_ab,
                                const float* mask, void* planes, int S, int N, hipStream_t st);
 hipError_t launch_transition64_f16(float* x, const float* lnw, const float* lnb, float eps, const void* w12,

@@ -171,130 +171,6 @@ __global__ __launch_bounds__(256, 2) void opm_outer_k(const __bf16* __restrict__
     }
 }
 
-// The outer sum of the fp16 mode, over two fp16 parts per operand (split2; 4 KB a token and stage) and three part
-// products, the output in fp16. Bound by the matrix cores' power: at S = 1024, N = 400 888 us = 1.13 PFLOP/s of part
-// products, where a large fp16 library product on random operands reaches 1.10 (1.69 on zeros); the six-product form
-// took 1,720. The same 128 x 128 tiles, two workgroups of 4 waves per CU: 256 x 256 tiles of 8 waves, one workgroup per
-// CU, halve the LDS and L2 reads but took 918 (S = 16, where the store is all: 122 against 111). Operands swapped
-// against the six-product form: register r of a block holds channel d = 8 (r / 4) + 4 hl + r % 4 of b, lane r32 channel
-// c of a, so a lane stores 4 consecutive d at once.
-__global__ __launch_bounds__(256, 2) void opm_outer2_k(const half_t* __restrict__ planes,
-                                                       const float* __restrict__ inv_scale,
-                                                       const float* __restrict__ num, half_t* __restrict__ out, int G,
-                                                       int N, int i_base, int n_i) {
-  constexpr int WM = 2, MB = 2, WN = 2, NB = 2;  // waves and blocks per wave along i and j
-  constexpr int WAVES = WM * WN, TI = WM * MB, TJ = WN * NB, TOKB = 4 * OPM_CHUNK;
-  constexpr int NS = 3, STAGE = 2 * (TI + TJ) * OPM_CHUNK, LPW = 2 * (TI + TJ) / WAVES;
-  static_assert(2 * (TI + TJ) % WAVES == 0, "chunks divide over the waves");
-  __shared__ __attribute__((aligned(1024))) char lds[NS * STAGE];
-  const int t = threadIdx.x, l = t & 63, r32 = l & 31, hl = l >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int wm = wave / WN, wn = wave % WN;
-  const int i0 = i_base + TI * (int)blockIdx.y, j0 = TJ * (int)blockIdx.x;
-  const int i_end = min(i_base + n_i, N);
-  // chunk q of a stage: q < 2 TI: part q / TI of the a half of token i0 + q % TI, else part (q - 2 TI) / TJ of the b
-  // half of token j0 + (q - 2 TI) % TJ (tokens past the range load the last one; their outputs are not stored)
-  int voff[LPW];
-#pragma unroll
-  for (int v = 0; v < LPW; v++) {
-    const int q = wave + WAVES * v, isb = q >= 2 * TI, qq = isb ? q - 2 * TI : q, T = isb ? TJ : TI;
-    const int p = qq / T, tt = qq % T, n = isb ? min(j0 + tt, N - 1) : min(i0 + tt, i_end - 1);
-    voff[v] = (n * 4 + 2 * p + isb) * OPM_CHUNK + (l >> 1) * 32 + 16 * ((l & 1) ^ ((l >> 3) & 1));
-  }
-  constexpr int RSRC_CFG = 0x00020000;
-  auto issue = [&](int st, int slot) {
-    st = min(st, G - 1);  // issues past the last stage reload it into a slot that is never read
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(reinterpret_cast<const char*>(planes) + (int64_t)st * N * TOKB), 0, N * TOKB, RSRC_CFG);
-#pragma unroll
-    for (int v = 0; v < LPW; v++) {
-      char* dst = lds + slot * STAGE + (wave + WAVES * v) * OPM_CHUNK;
-      const int off = voff[v];
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, 0);
-    }
-  };
-  const int fro = r32 * 32 + 16 * (hl ^ ((r32 >> 2) & 1));
-  typedef half8 FragA[MB][2];
-  typedef half8 FragB[NB][2];
-  FragA fa0, fa1;  // two sets, named (an array indexed by the stage parity would live in scratch)
-  FragB fb0, fb1;
-  auto read = [&](FragA& fa, FragB& fb, int slot) {
-    const char* base = lds + slot * STAGE + fro;
-#pragma unroll
-    for (int p = 0; p < 2; p++) {
-#pragma unroll
-      for (int x = 0; x < MB; x++)
-        fa[x][p] = *reinterpret_cast<const half8*>(base + (p * TI + MB * wm + x) * OPM_CHUNK);
-#pragma unroll
-      for (int x = 0; x < NB; x++)
-        fb[x][p] = *reinterpret_cast<const half8*>(base + (2 * TI + p * TJ + NB * wn + x) * OPM_CHUNK);
-    }
-  };
-  f16x acc[MB][NB];
-#pragma unroll
-  for (int a = 0; a < MB; a++)
-#pragma unroll
-    for (int b = 0; b < NB; b++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) acc[a][b][e] = 0.0f;
-  constexpr int YOUNGER = (NS - 2) * LPW;  // loads of later stages in flight when a stage is waited for
-  constexpr int WAIT = (YOUNGER & 15) | ((YOUNGER >> 4) << 14) | (0x7 << 4) | (0xF << 8);  // vmcnt only
-#pragma unroll
-  for (int p = 0; p < NS - 1; p++) issue(p, p);
-  __builtin_amdgcn_s_waitcnt(WAIT);
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-  issue(NS - 1, NS - 1);
-  read(fa0, fb0, 0);
-  auto step = [&](int st, const FragA& ca, const FragB& cb, FragA& na, FragB& nb) {
-    if (st + 1 < G) {
-      // this wave's reads of slot st % NS are done and stage st + 1 has landed; after the barrier the slot takes
-      // stage st + NS, and the fragments of stage st + 1 are read while stage st computes
-      __builtin_amdgcn_s_waitcnt(WAIT & ~(0xF << 8));  // vmcnt as above, lgkmcnt(0)
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      issue(st + NS, st % NS);
-      read(na, nb, (st + 1) % NS);
-    }
-    constexpr int PA[3] = {1, 0, 0}, PB[3] = {0, 1, 0};  // smaller products first
-#pragma unroll
-    for (int q = 0; q < 3; q++)
-#pragma unroll
-      for (int bm = 0; bm < MB; bm++)
-#pragma unroll
-        for (int bn = 0; bn < NB; bn++)
-          acc[bm][bn] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cb[bn][PB[q]], ca[bm][PA[q]], acc[bm][bn], 0, 0, 0);
-  };
-  for (int st = 0; st < G; st += 2) {
-    step(st, fa0, fb0, fa1, fb1);
-    if (st + 1 < G) step(st + 1, fa1, fb1, fa0, fb0);
-  }
-  const float sa = inv_scale[r32];
-  float sb[16];
-#pragma unroll
-  for (int r = 0; r < 16; r++) sb[r] = inv_scale[32 + 8 * (r >> 2) + 4 * hl + (r & 3)];
-#pragma unroll
-  for (int bm = 0; bm < MB; bm++) {
-    const int i = i0 + MB * wm + bm;
-    if (i >= i_end) continue;  // wave-uniform
-    const float si = sa * ldexpf(1.0f, -opm_mask_exp(num[(int64_t)i * N + i]));
-#pragma unroll
-    for (int bn = 0; bn < NB; bn++) {
-      const int j = j0 + NB * wn + bn;
-      if (j >= N) continue;  // wave-uniform
-      const float sj = ldexpf(1.0f, -opm_mask_exp(num[(int64_t)j * N + j])) / fmaxf(num[(int64_t)i * N + j], 1.0f);
-      half_t* op = out + ((int64_t)(i - i_base) * N + j) * 1024 + r32 * 32 + 4 * hl;
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        half4 v;
-#pragma unroll
-        for (int e = 0; e < 4; e++) v[e] = (half_t)(acc[bm][bn][4 * q + e] * si * (sb[4 * q + e] * sj));
-        *reinterpret_cast<half4*>(op + 8 * q) = v;
-      }
-    }
-  }
-}
-
 // ---------------------------------------------------------------- pair-weighted averaging
 // One wave per row (h, i): x_j = logit + (1 - pm[i][j]) * -inf in fp32, softmax over j < N, zeros for N <= j < ldw.
 __global__ __launch_bounds__(256) void pwa_softmax_k(const float* __restrict__ logits, const float* __restrict__ pm,
@@ -478,20 +354,6 @@ hipError_t launch_opm_outer(const void* planes, const float* num, void* out, int
     opm_outer_k<half_t><<<grid, 256, 0, st>>>(pl, num, static_cast<half_t*>(out), G, N, i_base, n_i);
   else
     opm_outer_k<float><<<grid, 256, 0, st>>>(pl, num, static_cast<float*>(out), G, N, i_base, n_i);
-  return hipGetLastError();
-}
-
-hipError_t launch_opm_outer2(const void* planes, const float* inv_scale, const float* num, void* out, int S, int N,
-                             int i_base, int n_i, hipStream_t st) {
-  const auto al = [](const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; };
-  if (S < 1 || N < 1 || i_base < 0 || n_i < 1 || i_base + n_i > N || (int64_t)N * OPM_TOKB > INT32_MAX ||
-      !al(planes, 16) || !al(out, 8))
-    return hipErrorInvalidValue;
-  const int G = (S + 15) / 16;
-  const half_t* pl = static_cast<const half_t*>(planes);
-  half_t* o = static_cast<half_t*>(out);
-  opm_outer2_k<<<dim3((unsigned)((N + 3) / 4), (unsigned)((n_i + 3) / 4)), 256, 0, st>>>(pl, inv_scale, num, o, G, N,
-                                                                                        i_base, n_i);
   return hipGetLastError();
 }
 

@@ -142,18 +142,11 @@ __global__ __launch_bounds__(64 * WR * WC, 8 / (WR * WC)) void ln_linear_x3_k(co
 // past S). Replaces bzpf_layernorm + bzpf_linear (a | b) + bzpf_opm_split. A tile is stage g (MSA rows 16 g .. + 15)
 // of tokens 8 nb .. + 7: tile row 16 tl + k is (s = 16 g + k, n = 8 nb + tl). Wave w computes tile rows 32 w .. + 31
 // (tokens 2 w, 2 w + 1) against the 64 channels (blocks h = a, b), so its accumulators hold whole chunk rows.
-// TWO: two fp16 parts instead (chunk (g, n, p, h) at ((g N + n) 4 + 2 p + h) 1024), of x 2^(E_ch + F_n): F_n from the
-// token's mask (opm_mask_exp), E_ch from a bound on the channel, |LN(m) . W_ab[ch]| <= 8 |gamma W_ab[ch]| + |beta .
-// W_ab[ch]| (a normalised row of 64 has norm at most 8), so that no value leaves fp16's range whatever m holds.
-// inv_scale[ch] = 2^-E_ch goes to the outer sum.
-template <bool TWO>
 __global__ __launch_bounds__(256, 2) void opm_ln_split_k(const float* __restrict__ m, const float* __restrict__ lnw,
                                                          const float* __restrict__ lnb, float eps,
                                                          const float* __restrict__ w, const float* __restrict__ mask,
-                                                         const float* __restrict__ num, void* __restrict__ planes,
-                                                         float* __restrict__ inv_scale, int S, int N, int nnb,
+                                                         __bf16* __restrict__ planes, int S, int N, int nnb,
                                                          int ntiles) {
-  __shared__ float Es[TWO ? 64 : 1];
   __shared__ __attribute__((aligned(16))) char Ws[3 * 64 * LNP_ROWB];      // 24 KB: W_ab's three planes
   __shared__ __attribute__((aligned(16))) char Xs[3 * LNP_BR * LNP_ROWB];  // 48 KB: the tile's LN(m) planes
   __shared__ float Ms[LNP_BR];                                             // the tile rows' mask values
@@ -168,18 +161,6 @@ __global__ __launch_bounds__(256, 2) void opm_ln_split_k(const float* __restrict
     for (int p = 0; p < 3; p++)
       *reinterpret_cast<uint2*>(Ws + p * 64 * LNP_ROWB + lnp_off(row, kq >> 1) + 8 * (kq & 1)) =
           uint2{q01.p[p], q23.p[p]};
-  }
-  if (TWO && t < 64) {
-    float g2 = 0.f, bw = 0.f;
-    for (int j = 0; j < LNP_K; j++) {
-      const float a = w[t * LNP_K + j], ga = lnw[j] * a;
-      g2 += ga * ga;
-      bw += fabsf(lnb[j] * a);
-    }
-    const float bound = 1.01f * (8.0f * sqrtf(g2) + bw);
-    const int e = bound > 0.0f && bound < INFINITY ? min(max(14 - ilogbf(bound), -100), 100) : 0;
-    Es[t] = ldexpf(1.0f, e);  // bound 2^e <= 2^15
-    if (blockIdx.x == 0) inv_scale[t] = ldexpf(1.0f, -e);
   }
   // m rows: pass v takes tile row t / 16 + 16 v, lane c = t % 16 channels 4 c .. + 3 (rows past S or N read a valid
   // row; past S their mask is taken as 0, past N their outputs are not stored)
@@ -254,28 +235,11 @@ __global__ __launch_bounds__(256, 2) void opm_ln_split_k(const float* __restrict
     for (int tk = 0; tk < 2; tk++) {
       const int n = 8 * nb + 2 * wave + tk;
       if (n >= N) continue;  // wave-uniform
-      char* cbase = static_cast<char*>(planes) + ((int64_t)g * N + n) * (TWO ? 4096 : 6144) + r32 * 32;
-      const float sn = TWO ? ldexpf(1.0f, opm_mask_exp(num[(int64_t)n * N + n])) : 1.0f;
+      char* cbase = reinterpret_cast<char*>(planes) + ((int64_t)g * N + n) * 6144 + r32 * 32;
 #pragma unroll
       for (int j = 0; j < 2; j++) {
         const int e0 = 8 * tk + 4 * j, k = 8 * j + 4 * hl;
         const int trow = 32 * wave + 16 * tk + k;
-        if constexpr (TWO) {
-#pragma unroll
-          for (int h = 0; h < 2; h++) {
-            const float sc = Es[32 * h + r32];
-            half4 hi, lo;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-              const Half2 q = split2((acc[h][e0 + e] * sc) * (Ms[trow + e] * sn));
-              hi[e] = q.h;
-              lo[e] = q.l;
-            }
-            *reinterpret_cast<half4*>(cbase + h * 1024 + 2 * k) = hi;
-            *reinterpret_cast<half4*>(cbase + (2 + h) * 1024 + 2 * k) = lo;
-          }
-          continue;
-        }
 #pragma unroll
         for (int h = 0; h < 2; h++) {
           const Pair3 q01 = split3_pair(acc[h][e0] * Ms[trow], acc[h][e0 + 1] * Ms[trow + 1]);
@@ -441,10 +405,8 @@ hipError_t launch_transition64_f16(float* x, const float* lnw, const float* lnb,
   return hipGetLastError();
 }
 
-template <bool TWO>
-static hipError_t opm_ln_split_t(const float* m, const float* lnw, const float* lnb, float eps, const float* w_ab,
-                                 const float* mask, const float* num, void* planes, float* inv_scale, int S, int N,
-                                 hipStream_t st) {
+hipError_t launch_opm_ln_split(const float* m, const float* lnw, const float* lnb, float eps, const float* w_ab,
+                               const float* mask, void* planes, int S, int N, hipStream_t st) {
   const auto al = [](const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; };
   if (S < 1 || N < 1 || !lnw || !lnb || !al(m, 16) || !al(w_ab, 16) || !al(lnw, 16) || !al(lnb, 16) ||
       !al(planes, 16) || (int64_t)N * 6144 > INT32_MAX)
@@ -452,22 +414,12 @@ static hipError_t opm_ln_split_t(const float* m, const float* lnw, const float* 
   const int64_t G = (S + 15) / 16, nnb = (N + 7) / 8;
   if (G * nnb > INT32_MAX) return hipErrorInvalidValue;
   static int cache[kMaxDevices];
-  const int resident = resident_grid(opm_ln_split_k<TWO>, 256, cache);
+  const int resident = resident_grid(opm_ln_split_k, 256, cache);
   if (resident <= 0) return hipErrorInvalidDevice;
   const int ntiles = (int)(G * nnb);
-  opm_ln_split_k<TWO><<<min(ntiles, resident), 256, 0, st>>>(m, lnw, lnb, eps, w_ab, mask, num, planes, inv_scale, S, N,
-                                                            (int)nnb, ntiles);
+  opm_ln_split_k<<<min(ntiles, resident), 256, 0, st>>>(m, lnw, lnb, eps, w_ab, mask, static_cast<__bf16*>(planes), S,
+                                                       N, (int)nnb, ntiles);
   return hipGetLastError();
-}
-
-hipError_t launch_opm_ln_split(const float* m, const float* lnw, const float* lnb, float eps, const float* w_ab,
-                               const float* mask, void* planes, int S, int N, hipStream_t st) {
-  return opm_ln_split_t<false>(m, lnw, lnb, eps, w_ab, mask, nullptr, planes, nullptr, S, N, st);
-}
-hipError_t launch_opm_ln_split2(const float* m, const float* lnw, const float* lnb, float eps, const float* w_ab,
-                                const float* mask, const float* num, void* planes, float* inv_scale, int S, int N,
-                                hipStream_t st) {
-  return opm_ln_split_t<true>(m, lnw, lnb, eps, w_ab, mask, num, planes, inv_scale, S, N, st);
 }
 
 template <int BR, int BC, int WR, int WC>

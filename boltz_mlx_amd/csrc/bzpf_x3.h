@@ -51,23 +51,6 @@ __device__ __forceinline__ f16x mfma_parts6(const bf16x8 (&a)[3], const bf16x8 (
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], c, 0, 0, 0);
 }
 
-// Two fp16 parts of a value scaled into fp16's range, for an operand whose results are stored in fp16: x = h + l with
-// h = fp16(x) and l = fp16(x - h), 22 significant bits while |x| >= 2^-3 (an absolute error of 2^-25 below that), and a
-// product as the three part products h h, h l, l h (l l is below 2^-22 of |x y|): half the time of the six.
-struct Half2 {
-  half_t h, l;
-};
-__device__ __forceinline__ Half2 split2(float x) {
-#pragma clang fp contract(off)
-  const half_t h = (half_t)x;
-  return Half2{h, (half_t)(x - (float)h)};
-}
-// Exponent F <= 0 with |mask[s][n]| 2^F <= 1 for every s, from num_nn = sum_s mask[s][n]^2.
-__device__ __forceinline__ int opm_mask_exp(float num_nn) {
-  if (!(num_nn > 1.0f) || !(num_nn < INFINITY)) return 0;
-  return -((ilogbf(num_nn) + 2) >> 1);
-}
-
 // One stage of a wave's MB x NB blocks: fragments of the three planes (PA / PB bf16 apart) of A rows
 // 32 MB wm + 32 bm + r32 and B rows 32 NB wn + 32 bn + r32, k = 8 hl .. 8 hl + 7 (lane (r32, hl)).
 template <int MB = 2, int NB = 2, int PA = PLANE, int PB = PLANE>

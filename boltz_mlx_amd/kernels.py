@@ -820,38 +820,6 @@ def opm_outer_planes(planes: torch.Tensor, num: torch.Tensor, S: int, N: int, i_
     return out
 
 
-def opm_ln_split2(m: torch.Tensor, ln, w_ab: torch.Tensor, mask: torch.Tensor, num: torch.Tensor):
-    """opm_ln_split as two fp16 parts of the values scaled into fp16's range, for an fp16 outer sum
-    ([ceil(S / 16), N, 2, 2, 32, 16] fp16: stage, token, part, a | b, channel, MSA row), with the channels' inverse scales
-    [64]; num = opm_counts(mask), which bounds a token's mask values."""
-    _dev(m, w_ab, mask, num)
-    S, N, C = m.shape
-    if m.dtype != torch.float32 or C != 64 or w_ab.shape != (64, 64) or w_ab.dtype != torch.float32 \
-            or mask.shape != (S, N) or mask.dtype != torch.float32 or num.shape != (N, N) \
-            or num.dtype != torch.float32:
-        raise ValueError("opm_ln_split2: need contiguous fp32 m [S, N, 64], w_ab [64, 64], mask [S, N], num [N, N]")
-    planes = torch.empty(((S + 15) // 16, N, 2, 2, 32, 16), dtype=torch.float16, device=m.device)
-    inv_scale = torch.empty((64,), dtype=torch.float32, device=m.device)
-    call("bzpf_opm_ln_split2", _p(m), _p(f32c(ln.weight)), _p(f32c(ln.bias)), float(ln.eps), _p(w_ab), _p(mask),
-         _p(num), _p(planes), _p(inv_scale), S, N, _stream())
-    return planes, inv_scale
-
-
-def opm_outer2(planes: torch.Tensor, inv_scale: torch.Tensor, num: torch.Tensor, S: int, N: int, i_base: int = 0,
-               n_i: int | None = None) -> torch.Tensor:
-    """opm_outer_planes in fp16 over opm_ln_split2's planes and scales."""
-    _dev(planes, inv_scale, num)
-    n_i = N - i_base if n_i is None else n_i
-    if planes.shape != ((S + 15) // 16, N, 2, 2, 32, 16) or planes.dtype != torch.float16 \
-            or inv_scale.shape != (64,) or inv_scale.dtype != torch.float32:
-        raise ValueError("opm_outer2: planes and inv_scale must be opm_ln_split2's output for S, N")
-    if num.shape != (N, N) or num.dtype != torch.float32:
-        raise ValueError("opm_outer2: num must be the fp32 [N, N] pair counts")
-    out = torch.empty((n_i * N, 1024), dtype=torch.float16, device=planes.device)
-    call("bzpf_opm_outer2", _p(planes), _p(inv_scale), _p(num), _p(out), S, N, int(i_base), int(n_i), _stream())
-    return out
-
-
 def opm_outer(ab: torch.Tensor, mask: torch.Tensor, i_base: int = 0, n_i: int | None = None,
               out_dtype=torch.float16, num: torch.Tensor | None = None) -> torch.Tensor:
     """OuterProductMean's outer sum for one MSA: ab fp32 [S, N, 64] (LN(m) [W_a; W_b]^T, unmasked), mask fp32

@@ -1,8 +1,7 @@
 """OuterProductMean on the bzpf kernels: same constructor, parameter names and call signature as
 boltz_mlx/layers/outer_product_mean.py:12-50 (inference).
 
-  x = mask * (LN(m) [W_a; W_b]^T) as three bf16 parts      bzpf_opm_ln_split (one kernel, fp32 accuracy); with an
-                                                           fp16 output two fp16 parts (bzpf_opm_ln_split2 / _outer2)
+  x = mask * (LN(m) [W_a; W_b]^T) as three bf16 parts      bzpf_opm_ln_split (one kernel, fp32 accuracy)
   num = mask^T mask                                        bzpf_linear (fp32, the pair counts)
   z16 = (sum_s mask_si mask_sj a_si (x) b_sj) / max(num, 1)  bzpf_opm_outer (fp32-accurate: six bf16 part products
                                                            per product, fp32 sums; fp16 out in f16 mode)
@@ -56,22 +55,17 @@ class OuterProductMean(torch.nn.Module):
         w_ab, w_o = K.kernel_weight(self, "w_ab"), K.kernel_weight(self, "w_o")
         mk = mask.to(torch.float32).reshape(S, N).contiguous()
         m3 = m.to(torch.float32).reshape(S, N, c_in)
-        num = K.opm_counts(mk)
-        fused = c_in == 64 and self.c_hidden == 32
-        two = fused and w_o.dtype == torch.float16  # an fp16 outer sum: two fp16 parts per operand are enough
-        if two:
-            planes, inv_scale = K.opm_ln_split2(m3.contiguous(), self.norm, w_ab, mk, num)
-        elif fused:
+        if c_in == 64 and self.c_hidden == 32:
             planes = K.opm_ln_split(m3.contiguous(), self.norm, w_ab, mk)
         else:
             mn = K.layer_norm(m3.reshape(S * N, c_in), self.norm.weight, self.norm.bias, self.norm.eps)
             planes = K.opm_split(K.linear(mn, w_ab).view(S, N, 2 * self.c_hidden), mk)
         z2 = z.view(N * N, co)
+        num = K.opm_counts(mk)
         step = max(1, min(N, OPM_PAIRS_PER_CHUNK // N))
         for i0 in range(0, N, step):
             n = min(step, N - i0)
-            zz = K.opm_outer2(planes, inv_scale, num, S, N, i0, n) if two else \
-                K.opm_outer_planes(planes, num, S, N, i0, n, out_dtype=w_o.dtype)
+            zz = K.opm_outer_planes(planes, num, S, N, i0, n, out_dtype=w_o.dtype)
             if resid is not None:
                 r2 = resid.reshape(N * N, co)[i0 * N:(i0 + n) * N]
                 K.linear_residual(zz, w_o, r2, z2[i0 * N:(i0 + n) * N], bias=self.proj_o.bias)

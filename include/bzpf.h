@@ -299,18 +299,6 @@ int bzpf_opm_ln_split(const float* m, const float* ln_w, const float* ln_b, floa
 int bzpf_opm_outer(const void* planes, const float* num, void* out, int out_dt, int n_seq, int N, int i_base, int n_i,
                    void* stream);
 
-/* The outer sum for fp16 outputs over two fp16 parts per operand: bzpf_opm_ln_split2 writes x 2^(E_ch + F_n) (E_ch a
- * power of two from a bound on the channel, F_n one from num[n][n], so that every value is inside fp16's range) as
- * x1 = fp16(x), x2 = fp16(x - x1), chunk (g, n, p, h) at byte ((g * N + n) * 4 + 2 * p + h) * 1024 of planes
- * (ceil(n_seq / 16) * N * 4096 bytes), and inv_scale[64] = 2^-E_ch; bzpf_opm_outer2 takes both, undoes the scales and
- * stores fp16: the sums err by about 2^-22 against the 2^-11 of the store. Other arguments as for bzpf_opm_ln_split and
- * bzpf_opm_outer, whose fp16 output they replace (boltz_mlx/layers/outer_product_mean.py:37-45). */
-int bzpf_opm_ln_split2(const float* m, const float* ln_w, const float* ln_b, float eps, const float* w_ab,
-                       const float* mask, const float* num, void* planes, float* inv_scale, int n_seq, int N,
-                       void* stream);
-int bzpf_opm_outer2(const void* planes, const float* inv_scale, const float* num, void* out, int n_seq, int N,
-                    int i_base, int n_i, void* stream);
-
 /* The 64-channel Transition in fp16, in place, in one kernel: x += fc3(silu(xn fc1^T) * (xn fc2^T)) with
  * xn = fp16(LN(x; ln_w, ln_b, eps)), for x fp32 [rows, 64], w12 fp16 [2 hidden, 64] = [fc1; fc2], w3 fp16
  * [64, hidden] (hidden a multiple of 64, at most 384); fp32 accumulation, the SwiGLU product rounded to fp16 as the

@@ -124,9 +124,9 @@ def test_opm_ln_split(S, N):
 @pytest.mark.parametrize("S,N,i_base,n_i,mscale,wscale", [(37, 5, 0, 5, 1.0, 1.0), (16, 130, 3, 126, 1.0, 1.0),
                                                           (1, 9, 0, 9, 3.0, 1.0), (33, 181, 0, 181, 1.0, 1.0),
                                                           (50, 190, 2, 177, 1.0, 300.0), (64, 37, 0, 37, 1e4, 1e-6)])
-def test_opm_outer2(S, N, i_base, n_i, mscale, wscale):
-    """The fp16 outer sum over two fp16 parts against float64: the error of the fp16 store, 2^-11 of the value, and the
-    sum's own, 2^-20 of the largest value (split parts: 2^-22 of a product)."""
+def test_opm_outer_f16_store(S, N, i_base, n_i, mscale, wscale):
+    """The fp16 outer sum against float64: the error of the fp16 store, 2^-11 of the value, and the sum's own, 2^-20 of
+    the largest value (split parts: 2^-22 of a product)."""
     from boltz_mlx_amd import kernels as K
 
     rng = np.random.default_rng(S * N)
@@ -142,9 +142,9 @@ def test_opm_outer2(S, N, i_base, n_i, mscale, wscale):
         eps = 1e-5
 
     num = K.opm_counts(dev(mask))
-    planes, inv = K.opm_ln_split2(dev(m), LN, dev(w_ab), dev(mask), num)
+    planes = K.opm_ln_split(dev(m), LN, dev(w_ab), dev(mask))
     assert torch.isfinite(planes).all()
-    got = K.opm_outer2(planes, inv, num, S, N, i_base, n_i).double()
+    got = K.opm_outer_planes(planes, num, S, N, i_base, n_i).double()
     mn = torch.nn.functional.layer_norm(dev(m).double(), (64,), LN.weight.double(), LN.bias.double(), 1e-5)
     x = (mn @ dev(w_ab).double().T) * dev(mask).double()[..., None]
     a, b = x[:, i_base:i_base + n_i, :32].reshape(S, -1), x[..., 32:].reshape(S, -1)
@@ -158,6 +158,32 @@ def test_opm_outer2(S, N, i_base, n_i, mscale, wscale):
         small = ref.abs() < 6e4
         assert ((got - ref).abs()[small] <= ref.abs()[small] * 2.0 ** -11 + top * 2.0 ** -20).all()
         assert torch.isinf(got[ref.abs() > 6.6e4]).all()
+
+
+def test_opm_f16_sum_is_the_fp32_sum_rounded_once():
+    """The f16 mode holds the operands of the outer sum in full and rounds only the sum: with proj_o picking 128 of the
+    1,024 sums, its output is the fp32 mode's rounded to fp16, bit for bit."""
+    from boltz_mlx_amd import kernels as K
+    from boltz_mlx_amd.layers.outer_product_mean import OuterProductMean
+
+    rng = np.random.default_rng(5)
+    S, N = 45, 37
+    with torch.no_grad():
+        mod = OuterProductMean(64, 32, 128).cuda().eval()
+        mod.proj_a.weight.copy_(dev(rng.standard_normal((32, 64)) / 8))
+        mod.proj_b.weight.copy_(dev(rng.standard_normal((32, 64)) / 8))
+        mod.proj_o.bias.zero_()
+        m, mask = dev(rng.standard_normal((1, S, N, 64))), dev(rng.random((1, S, N)) > 0.1)
+        old = K.PRECISION
+        try:
+            for c0 in range(0, 1024, 128):
+                mod.proj_o.weight.copy_(torch.eye(1024, device="cuda")[c0:c0 + 128])
+                K.set_precision("fp32")
+                exact = mod(m, mask)
+                K.set_precision("f16")
+                assert torch.equal(mod(m, mask), exact.half().float()), c0
+        finally:
+            K.set_precision(old)
 
 
 def test_opm_outer_zero_count_pair():
