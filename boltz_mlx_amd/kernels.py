@@ -16,6 +16,7 @@ from __future__ import annotations
 import contextlib
 import functools
 import os
+import threading
 from typing import NamedTuple
 
 import torch
@@ -373,29 +374,45 @@ def trimul_contract(ab: torch.Tensor, N: int, k_len=0) -> torch.Tensor:
     return o
 
 
-# Per-mask values derived once inside pair_mask_scope(): {key: {"t": transposed copy, ("ext", incoming): k_len}}
-_MASK_SCOPE: dict | None = None
+class _MaskScope(threading.local):
+    """The thread's innermost pair_mask_scope: entries is None outside one, else {key: {"mask": the mask, "t": its
+    transposed copy, "dev": its key extents on the device}}; capturing: it was entered during a stream capture."""
+
+    entries = None
+    capturing = False
+
+
+_MASK_SCOPE = _MaskScope()
+
+
+def _capturing() -> bool:
+    return torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
 
 
 @contextlib.contextmanager
 def pair_mask_scope():
     """Inside the block, the values derived from a pair mask (the ending-node core's transposed copy, the
-    contraction's key extent) are computed once per mask (keyed by its storage, shape, strides and version) and
-    reused by every later call with the same mask: a module run derives them once instead of once per layer.
-    Outside a scope each call transposes for itself and the contraction runs over every key."""
-    global _MASK_SCOPE
-    prev, _MASK_SCOPE = _MASK_SCOPE, {}
+    contraction's key extents) are computed once per mask (keyed by its storage, shape, strides and version, the mask
+    kept alive for as long) and reused by every later call with the same mask: a module run derives them once instead
+    of once per layer. They are device tensors with no other order than their stream's, so they are shared within one
+    thread and one stream only, and never between a stream capture and work outside it (a replay would read what the
+    mask held at the capture). Outside a scope each call transposes for itself and the contraction runs over every
+    key."""
+    sc = _MASK_SCOPE
+    prev = sc.entries, sc.capturing
+    sc.entries, sc.capturing = {}, _capturing()
     try:
         yield
     finally:
-        _MASK_SCOPE = prev
+        sc.entries, sc.capturing = prev
 
 
 def _mask_entry(mask: torch.Tensor):
-    if _MASK_SCOPE is None:
+    sc = _MASK_SCOPE
+    if sc.entries is None or (mask.is_cuda and _capturing() != sc.capturing):
         return None
-    key = (mask.data_ptr(), tuple(mask.shape), tuple(mask.stride()), mask._version)
-    return _MASK_SCOPE.setdefault(key, {})
+    key = (_stream() if mask.is_cuda else None, mask.data_ptr(), tuple(mask.shape), tuple(mask.stride()), mask._version)
+    return sc.entries.setdefault(key, {"mask": mask})
 
 
 def mask_transposed(mask: torch.Tensor, N: int) -> torch.Tensor:

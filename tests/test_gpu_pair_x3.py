@@ -181,6 +181,41 @@ def test_key_extent_device(N, rows, cols, dtype):
     assert K.key_extent_device(mask, N, False) == 0
 
 
+def test_mask_scope_around_a_capture():
+    """Triangle multiplication and ending-node attention captured inside a scope that is older than the capture: replays
+    follow the mask that they find, not the one of the warm-up."""
+    from boltz_mlx_amd import kernels as K
+    from boltz_mlx_amd.layers.triangular_attention.attention import TriangleAttentionEndingNode
+    from boltz_mlx_amd.layers.triangular_mult import TriangleMultiplicationOutgoing
+
+    N = 150
+    torch.manual_seed(2)
+    old = K.PRECISION
+    K.set_precision("f16")
+    try:
+        with torch.no_grad(), torch.device("cuda"):
+            mods = [TriangleMultiplicationOutgoing(128), TriangleAttentionEndingNode(128, 32, 4)]
+            z = torch.randn(1, N, N, 128)
+            mask = torch.zeros(1, N, N)
+            mask[:, :40, :40] = 1
+            run = lambda: [mod(z, mask) for mod in mods]  # noqa: E731
+            with K.pair_mask_scope():
+                run()
+                graph = torch.cuda.CUDAGraph()
+                torch.cuda.synchronize()
+                with torch.cuda.graph(graph):
+                    out = run()
+            for live in (150, 90, 20, 150):
+                mask.zero_()
+                mask[:, :live, :live] = 1
+                want = run()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert all(torch.equal(a, b) for a, b in zip(out, want)), live
+    finally:
+        K.set_precision(old)
+
+
 # one row, the end of a 16-row tile, more tiles than resident waves (65,536 rows and more), few and all 16 heads
 @pytest.mark.parametrize("N,H", [(1, 16), (3, 4), (16, 8), (37, 16), (270, 16), (333, 1)])
 def test_pair_bias(N, H):

@@ -56,6 +56,110 @@ def test_pair_mask_scope_extent_and_transpose():
     assert K.key_extent(m, N, False) == 0
 
 
+class _DeviceMask(torch.Tensor):
+    """A CPU tensor that says it is on the GPU, so that what a scope shares can be followed without one."""
+
+    is_cuda = True
+
+
+@pytest.fixture
+def fake_device(monkeypatch):
+    """Streams and captures as the wrappers see them, and the launches they make, without a GPU."""
+    from boltz_mlx_amd import kernels as K
+
+    state = {"stream": 1, "capturing": False, "calls": []}
+    monkeypatch.setattr(K, "_stream", lambda: state["stream"])
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state["capturing"])
+    monkeypatch.setattr(K, "call", lambda name, *args: state["calls"].append((name, args[-1])))
+    return state
+
+
+def _mask(n=70):
+    return torch.ones((n, n)).as_subclass(_DeviceMask)
+
+
+def test_pair_mask_scope_shares_within_one_stream(fake_device):
+    """A mask's device values have no order but their stream's: a reader on another stream makes its own."""
+    from boltz_mlx_amd import kernels as K
+
+    m = _mask()
+    with K.pair_mask_scope():
+        a, t = K.key_extent_device(m, 70, False), K.mask_transposed(m, 70)
+        assert K.key_extent_device(m, 70, True).data_ptr() == a.data_ptr() + 4 and K.mask_transposed(m, 70) is t
+        fake_device["stream"] = 2
+        b, u = K.key_extent_device(m, 70, False), K.mask_transposed(m, 70)
+        assert b.data_ptr() != a.data_ptr() and u is not t
+        fake_device["stream"] = 1
+        assert K.key_extent_device(m, 70, False).data_ptr() == a.data_ptr()
+    assert fake_device["calls"] == [("bzpf_key_extents", 1), ("bzpf_key_extents", 2)]
+
+
+def test_pair_mask_scope_and_captures(fake_device):
+    """A scope that outlives a capture shares nothing with it (a replay would read the mask of the capture, work outside
+    it a value that only a replay computes); one entered inside it does, as a captured module run enters."""
+    from boltz_mlx_amd import kernels as K
+
+    m = _mask()
+    with K.pair_mask_scope():
+        t = K.mask_transposed(m, 70)
+        fake_device["capturing"] = True
+        assert K.mask_transposed(m, 70) is not t
+        assert K.key_extent_device(m, 70, False) == 0  # every key
+        with K.pair_mask_scope():
+            a = K.key_extent_device(m, 70, False)
+            assert K.key_extent_device(m, 70, False).data_ptr() == a.data_ptr()
+            assert K.mask_transposed(m, 70) is K.mask_transposed(m, 70)
+            fake_device["capturing"] = False
+            assert K.key_extent_device(m, 70, False) == 0
+        assert K.mask_transposed(m, 70) is t
+
+
+def test_pair_mask_scope_is_the_threads_own(fake_device):
+    """A scope of one thread is not another's, and leaving them in any order leaves none behind."""
+    import threading
+
+    from boltz_mlx_amd import kernels as K
+
+    m, seen = _mask(), []
+    entered, left = threading.Event(), threading.Event()
+
+    def other():
+        seen.append(K.key_extent_device(m, 70, False))  # outside: every key
+        with K.pair_mask_scope():
+            entered.set()
+            left.wait(10)
+        seen.append(K.key_extent_device(m, 70, False))
+
+    t = threading.Thread(target=other)
+    with K.pair_mask_scope():
+        K.key_extent_device(m, 70, False)
+        t.start()
+        assert entered.wait(10)
+    left.set()
+    t.join()
+    seen.append(K.key_extent_device(m, 70, False))
+    assert not any(isinstance(v, torch.Tensor) for v in seen)
+
+
+def test_pair_mask_scope_keeps_its_masks(fake_device):
+    """A scope knows a mask by its address, so it holds the mask: one made where a dropped one was is not taken for it."""
+    import gc
+    import weakref
+
+    from boltz_mlx_amd import kernels as K
+
+    m = _mask()
+    alive = weakref.ref(m)
+    with K.pair_mask_scope():
+        K.mask_transposed(m, 70)
+        del m
+        gc.collect()
+        assert alive() is not None
+    gc.collect()
+    assert alive() is None
+
+
 # ---------------------------------------------------------------- kernel index maps and buffer ranges (host build)
 
 @pytest.fixture(scope="module")
