@@ -444,6 +444,8 @@ def key_extent_device(mask: torch.Tensor, N: int, incoming: bool):
     """key_extent as an int32 tensor [1] on the device (0 for a mask without a nonzero, which the contraction takes as
     every key), so that a module run neither waits for the mask nor launches torch's reductions: inside pair_mask_scope
     one kernel finds both directions' extents once per mask; 0 (every key) outside."""
+    if mask.dtype != torch.float32 or mask.numel() != N * N:
+        raise ValueError("key_extent_device: mask must be fp32 [N, N]")
     ent = _mask_entry(mask)
     if ent is None:
         return 0

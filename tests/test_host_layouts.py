@@ -95,6 +95,20 @@ def test_pair_mask_scope_shares_within_one_stream(fake_device):
     assert fake_device["calls"] == [("bzpf_key_extents", 1), ("bzpf_key_extents", 2)]
 
 
+@pytest.mark.parametrize("bad", [torch.ones(70, 70, dtype=torch.bool), torch.ones(70, 70, dtype=torch.float16),
+                                 torch.ones(69, 70), torch.ones(70)])
+def test_key_extent_device_checks_its_mask(fake_device, bad):
+    """Its kernel reads N * N floats: nothing else gets there, inside a scope or outside."""
+    from boltz_mlx_amd import kernels as K
+
+    bad = bad.as_subclass(_DeviceMask)
+    with pytest.raises(ValueError):
+        K.key_extent_device(bad, 70, False)
+    with K.pair_mask_scope(), pytest.raises(ValueError):
+        K.key_extent_device(bad, 70, False)
+    assert fake_device["calls"] == []
+
+
 def test_pair_mask_scope_and_captures(fake_device):
     """A scope that outlives a capture shares nothing with it (a replay would read the mask of the capture, work outside
     it a value that only a replay computes); one entered inside it does, as a captured module run enters."""
