@@ -190,7 +190,8 @@ def wcache(owner: torch.nn.Module, name: str, *params: torch.Tensor, dtype=None)
 
 
 def f32c(t: torch.Tensor) -> torch.Tensor:
-    """t in fp32, contiguous, for its data pointer (t itself where it is both already)."""
+    """t in fp32, contiguous, for its data pointer (t itself where it is both already). A caller holds the result until
+    its launch is made: a temporary that is dropped before gives its block to the next allocation."""
     if t.dtype == torch.float32 and t.is_contiguous():
         return t
     return t.detach().float().contiguous()
@@ -281,7 +282,8 @@ def trimul_tail64(o, norm_out, eps_out: float, w_po, xn, w_go, z, accumulate: bo
     if next_ln is not None:
         nxt = torch.empty((N * N, 64), dtype=xn.dtype, device=xn.device)
         nw, nb, neps = f32c(next_ln.weight), f32c(next_ln.bias), next_ln.eps
-    call("bzpf_trimul_tail64", _p(o), _p(f32c(norm_out.weight)), _p(f32c(norm_out.bias)), float(eps_out), _p(w_po),
+    ow, ob = f32c(norm_out.weight), f32c(norm_out.bias)
+    call("bzpf_trimul_tail64", _p(o), _p(ow), _p(ob), float(eps_out), _p(w_po),
          _p(xn), _p(w_go), _p(z), int(accumulate), _p(nw), _p(nb), float(neps), _p(nxt), _dt(xn), N, ld, _stream())
     return nxt
 
@@ -469,7 +471,8 @@ def trimul_tail(o, norm_out, eps_out: float, w_po, xn, w_go, z, accumulate: bool
     if next_ln is not None:
         nxt = torch.empty((N * N, D), dtype=xn.dtype, device=xn.device)
         nw, nb, neps = f32c(next_ln.weight), f32c(next_ln.bias), next_ln.eps
-    call("bzpf_trimul_tail", _p(o), _p(f32c(norm_out.weight)), _p(f32c(norm_out.bias)), float(eps_out), _p(w_po),
+    ow, ob = f32c(norm_out.weight), f32c(norm_out.bias)
+    call("bzpf_trimul_tail", _p(o), _p(ow), _p(ob), float(eps_out), _p(w_po),
          _p(xn), _p(w_go), _p(z), int(accumulate), _p(nw), _p(nb), float(neps), _p(nxt), _dt(xn), N, ld, D,
          _stream())
     return nxt
@@ -580,8 +583,9 @@ def transition(xn, w12, w3, z, accumulate: bool, next_ln=None, pair_bias=None):
         raise ValueError("transition: pair-bias weight must be [H, D] in the storage dtype")
     N = z.shape[0]
     bias = torch.empty((H, N, rows // N), dtype=w.dtype, device=z.device)
+    lw, lb = f32c(ln.weight), f32c(ln.bias)
     call("bzpf_transition_pb", _p(xn), _p(w12), _p(w3), _p(z), int(accumulate), _p(nw), _p(nb), float(neps),
-         _p(nxt), _p(w), _p(f32c(ln.weight)), _p(f32c(ln.bias)), float(ln.eps), _p(bias), H, _dt(xn), rows, D, hidden,
+         _p(nxt), _p(w), _p(lw), _p(lb), float(ln.eps), _p(bias), H, _dt(xn), rows, D, hidden,
          _stream())
     return nxt, bias
 
@@ -613,7 +617,8 @@ def attn_out_transition(o, w_o, trans: bool, z, ln, w12, w3, next_ln=None, pair_
             raise ValueError("attn_out_transition: pair-bias weight must be [H, D] in fp16")
         plw, plb, peps = f32c(ln_pb.weight), f32c(ln_pb.bias), ln_pb.eps
         bias = torch.empty((H, N, N), dtype=pw.dtype, device=z.device)
-    call("bzpf_attn_out_transition", _p(o), _p(w_o), int(trans), _p(f32c(ln.weight)), _p(f32c(ln.bias)),
+    lw, lb = f32c(ln.weight), f32c(ln.bias)
+    call("bzpf_attn_out_transition", _p(o), _p(w_o), int(trans), _p(lw), _p(lb),
          float(ln.eps), _p(w12), _p(w3), _p(z), _p(nw), _p(nb), float(neps), _p(nxt), _p(pw), _p(plw), _p(plb),
          float(peps), _p(bias), H, _dt(o), N, D, hidden, _stream())
     return nxt if pair_bias is None else (nxt, bias)
@@ -860,7 +865,8 @@ def transition64_f16(x: torch.Tensor, ln, w12: torch.Tensor, w3: torch.Tensor) -
             or w3.shape != (64, H) or w12.dtype != torch.float16 or w3.dtype != torch.float16 \
             or not w12.is_contiguous() or not w3.is_contiguous():
         raise ValueError("transition64_f16: need contiguous fp32 x [rows, 64], fp16 w12 [2H, 64] and w3 [64, H]")
-    call("bzpf_transition64_f16", _p(x), _p(f32c(ln.weight)), _p(f32c(ln.bias)), float(ln.eps), _p(w12), _p(w3),
+    lw, lb = f32c(ln.weight), f32c(ln.bias)
+    call("bzpf_transition64_f16", _p(x), _p(lw), _p(lb), float(ln.eps), _p(w12), _p(w3),
          rows, H, _stream())
 
 
@@ -931,6 +937,7 @@ def pair_bias(z: torch.Tensor, ln, w: torch.Tensor) -> torch.Tensor:
     N, D = z.shape[0], z.shape[-1]
     H = w.shape[0]
     out = torch.empty((H, N, N), dtype=w.dtype, device=z.device)
-    call("bzpf_pair_bias", _p(z), _p(f32c(ln.weight)), _p(f32c(ln.bias)), float(ln.eps), _p(w), _p(out), _dt(w),
+    lw, lb = f32c(ln.weight), f32c(ln.bias)
+    call("bzpf_pair_bias", _p(z), _p(lw), _p(lb), float(ln.eps), _p(w), _p(out), _dt(w),
          N * N, D, H, _stream())
     return out

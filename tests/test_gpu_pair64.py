@@ -58,6 +58,38 @@ def test_trimul64(dt, N):
         assert _rel(nxt.view(N, N, 64), nx(got.double())) <= tol
 
 
+def test_half_layernorm_parameters():
+    """LayerNorm parameters held in fp16 give what the same values in fp32 give, bit for bit."""
+    from boltz_mlx_amd import kernels as K
+
+    N = 37
+    g = torch.Generator(device="cuda").manual_seed(N)
+
+    class Half:
+        eps = 1e-5
+
+        def __init__(self, ln):
+            self.weight, self.bias = ln.weight.half(), ln.bias.half()
+
+    class Full(Half):
+        def __init__(self, ln):
+            super().__init__(ln)
+            self.weight, self.bias = self.weight.float(), self.bias.float()
+
+    no, nx = _Ln(g, 64), _Ln(g, 64)
+    o, xn = _rand(g, torch.float16, 64, N, K.row_pitch(N)), _rand(g, torch.float16, N * N, 64)
+    w_po, w_go = (_rand(g, torch.float32, 64, 64).mul(0.125).half() for _ in range(2))
+    z = torch.randn((N, N, 64), generator=g, device="cuda")
+    out = []
+    for kind in (Full, Half):
+        got = z.clone()
+        out.append((got, K.trimul_tail64(o, kind(no), 1e-4, w_po, xn, w_go, got, True, kind(nx), N)))
+    assert all(torch.equal(a, b) for a, b in zip(*out))
+    z, w = torch.randn((N, N, 128), generator=g, device="cuda"), _rand(g, torch.float16, 16, 128)
+    ln = _Ln(g, 128)
+    assert torch.equal(K.pair_bias(z, Full(ln), w), K.pair_bias(z, Half(ln), w))
+
+
 @pytest.mark.parametrize("dt,N", CASES)
 def test_triattn64(dt, N):
     from boltz_mlx_amd import kernels as K

@@ -56,6 +56,61 @@ def test_pair_mask_scope_extent_and_transpose():
     assert K.key_extent(m, N, False) == 0
 
 
+class _HalfLN:
+    """LayerNorm parameters that the kernels cannot read as they are."""
+
+    def __init__(self, d):
+        self.weight, self.bias, self.eps = torch.ones(d, dtype=torch.float16), torch.zeros(d, dtype=torch.float16), 1e-5
+
+
+def _ln_calls():
+    from boltz_mlx_amd import kernels as K
+
+    N, h = 3, torch.float16
+    ld = K.row_pitch(N)
+    z, o = torch.zeros(N, N, 128), torch.zeros(128, N, ld, dtype=h)
+    xn, w, w12, w3 = (torch.zeros(*s, dtype=h) for s in ((N * N, 128), (128, 128), (512, 128), (128, 256)))
+    z64, o64, xn64, w64 = torch.zeros(N, N, 64), o[:64], xn[:, :64].contiguous(), torch.zeros(64, 64, dtype=h)
+    ln, ln64, pw = _HalfLN(128), _HalfLN(64), torch.zeros(4, 128, dtype=h)
+    return {
+        "layer_norm": lambda: K.layer_norm(xn, ln.weight, ln.bias),
+        "add_ln": lambda: K.add_ln(z, z, ln),
+        "trimul_tail": lambda: K.trimul_tail(o, ln, 1e-5, w, xn, w, z, True, ln, N),
+        "trimul_tail64": lambda: K.trimul_tail64(o64, ln64, 1e-5, w64, xn64, w64, z64, True, ln64, N),
+        "linear_resid_ln": lambda: K.linear_resid_ln(xn, w, False, z, True, ln, N),
+        "linear_resid_ln64": lambda: K.linear_resid_ln64(xn, w[:64], False, z64, True, ln64, N),
+        "transition": lambda: K.transition(xn, w12, w3, z, True, ln, (ln, pw)),
+        "attn_out_transition": lambda: K.attn_out_transition(xn, w, True, z, ln, w12, w3, ln, (ln, pw)),
+        "transition64_f16": lambda: K.transition64_f16(z64.view(-1, 64), ln64, w12[:, :64].contiguous(), w3[:64]),
+        "ln_linear_f32": lambda: K.ln_linear_f32(z64.view(-1, 64), ln64, torch.zeros(256, 64)),
+        "opm_ln_split": lambda: K.opm_ln_split(torch.zeros(2, N, 64), ln64, torch.zeros(64, 64), torch.zeros(2, N)),
+        "pair_bias": lambda: K.pair_bias(z, ln, pw),
+    }
+
+
+@pytest.mark.parametrize("name", _ln_calls())
+def test_converted_parameters_outlive_the_launch(monkeypatch, name):
+    """A LayerNorm parameter that is not fp32 is converted for the call; the copy has to live until the launch is made,
+    or the allocator gives its block to the next parameter's copy and the kernel reads one for the other."""
+    import weakref
+
+    from boltz_mlx_amd import kernels as K
+
+    copies, calls = [], []
+
+    def f32c(t):
+        c = t.float()
+        copies.append(weakref.ref(c))
+        return c
+
+    monkeypatch.setattr(K, "f32c", f32c)
+    monkeypatch.setattr(K, "_dev", lambda *ts: None)
+    monkeypatch.setattr(K, "_stream", lambda: 0)
+    monkeypatch.setattr(K, "call", lambda *args: calls.append([c() is not None for c in copies]))
+    _ln_calls()[name]()
+    assert len(calls) == 1 and len(copies) >= 2 and all(calls[0])
+
+
 class _DeviceMask(torch.Tensor):
     """A CPU tensor that says it is on the GPU, so that what a scope shares can be followed without one."""
 
