@@ -358,8 +358,8 @@ def triattn_pack(P: torch.Tensor, trans: bool, N: int, H: int, C: int):
 
 def trimul_contract(ab: torch.Tensor, N: int, k_len=0) -> torch.Tensor:
     """o [D, N, ld] = per-channel a b^T; k_len > 0: columns k >= k_len of ab are zero and the sum stops there (the
-    trailing padded tokens; key_extent gives it for a pair mask). k_len may be an int32 tensor [1] on the device
-    (key_extent_device), which the kernel reads: the host need not know it."""
+    trailing padded tokens). k_len may be an int32 tensor [1] on the device (key_extent_device makes it of a pair mask),
+    which the kernel reads: the host need not know it."""
     _dev(ab)
     D = ab.shape[0] // 2
     ld = row_pitch(N)
@@ -427,25 +427,11 @@ def mask_transposed(mask: torch.Tensor, N: int) -> torch.Tensor:
     return ent["t"]
 
 
-def key_extent(mask: torch.Tensor, N: int, incoming: bool) -> int:
-    """1 + the last token k whose pair-mask column (outgoing; row for incoming) is not all zero: bzpf_trimul_proj
-    writes zeros in ab for every k past it. Computed (one host sync) only inside pair_mask_scope, once per mask;
-    0 (every key) outside, and during stream capture (no sync there)."""
-    ent = _mask_entry(mask)
-    if ent is None or (mask.is_cuda and torch.cuda.is_current_stream_capturing()):
-        return 0
-    if ("ext", incoming) not in ent:
-        m = mask.reshape(N, N) != 0
-        live = m.any(dim=1 if incoming else 0)
-        idx = torch.nonzero(live)
-        ent[("ext", incoming)] = int(idx[-1, 0].item()) + 1 if idx.numel() else N
-    return ent[("ext", incoming)]
-
-
 def key_extent_device(mask: torch.Tensor, N: int, incoming: bool):
-    """key_extent as an int32 tensor [1] on the device (0 for a mask without a nonzero, which the contraction takes as
-    every key), so that a module run neither waits for the mask nor launches torch's reductions: inside pair_mask_scope
-    one kernel finds both directions' extents once per mask; 0 (every key) outside."""
+    """1 + the last token k whose pair-mask column (outgoing; row for incoming) is not all zero, past which
+    bzpf_trimul_proj writes zeros in ab, as an int32 tensor [1] on the device (0 for a mask without a nonzero, which the
+    contraction takes as every key), so that a module run neither waits for the mask nor launches torch's reductions:
+    inside pair_mask_scope one kernel finds both directions' extents once per mask; 0 (every key) outside."""
     if mask.dtype != torch.float32 or mask.numel() != N * N:
         raise ValueError("key_extent_device: mask must be fp32 [N, N]")
     ent = _mask_entry(mask)

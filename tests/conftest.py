@@ -177,3 +177,10 @@ def pair_inputs(N: int, D: int, seed: int, n_pad: int = 0, B: int = 1, dtype=np.
 @pytest.fixture
 def rng():
     return np.random.default_rng(1234)
+
+
+def mask_key_extent(mask, incoming: bool) -> int:
+    """1 + the last token whose pair-mask column (outgoing; row for incoming) is not all zero; 0 for a mask without a
+    nonzero."""
+    live = np.asarray(mask.cpu() != 0).any(axis=1 if incoming else 0).nonzero()[0]
+    return int(live[-1]) + 1 if live.size else 0

@@ -17,7 +17,8 @@ import pytest
 import torch
 
 import oracle as O
-from conftest import pair_inputs, rand_params, shapes_attention, shapes_layer, shapes_transition, shapes_tri_att, shapes_tri_mul
+from conftest import (mask_key_extent, pair_inputs, rand_params, shapes_attention, shapes_layer, shapes_transition,
+                      shapes_tri_att, shapes_tri_mul)
 
 pytestmark = pytest.mark.gpu
 
@@ -165,7 +166,7 @@ def test_trimul_contract_key_extent_exact(N, dt):
 
 @pytest.mark.parametrize("precision", ["f16"], indirect=True)
 @pytest.mark.parametrize("outgoing", [True, False])
-def test_tri_mul_in_mask_scope_equals_plain(precision, outgoing):
+def test_tri_mul_in_mask_scope_equals_plain(precision, outgoing, monkeypatch):
     """Inside pair_mask_scope the module contracts only up to the key extent of its (asymmetric, trailing-padded)
     mask; the update equals the call outside a scope (every key) bit for bit, in f16."""
     from boltz_mlx_amd import kernels as K
@@ -185,10 +186,16 @@ def test_tri_mul_in_mask_scope_equals_plain(precision, outgoing):
     xn = m.norm_in.to_storage(z).reshape(N * N, D)
     z1, z2 = z.clone(), z.clone()
     m.fused(xn, mask, z1, True)
+    extents, contract = [], K.trimul_contract
+
+    def counting(ab, N, k_len=0):
+        extents.append(k_len)
+        return contract(ab, N, k_len)
+
+    monkeypatch.setattr(K, "trimul_contract", counting)
     with K.pair_mask_scope():
-        assert K.key_extent(mask, N, not outgoing) <= N - 70
         m.fused(xn, mask, z2, True)
-    torch.cuda.synchronize()
+    assert len(extents) == 1 and 0 < int(extents[0]) == mask_key_extent(mask, not outgoing) <= N - 70
     assert torch.equal(z1, z2)
 
 

@@ -26,11 +26,11 @@ def test_group_swiglu_rows():
 
 
 def test_pair_mask_scope_extent_and_transpose():
-    """key_extent / mask_transposed: nothing is derived outside a scope (extent 0 = every key, a fresh transposed
-    copy per call); inside, the extent is 1 + the last live token (columns for outgoing, rows for incoming, checked
-    by brute force on an asymmetric mask), each value is made once per mask, and an in-place change of the mask
-    (a new version) is seen."""
+    """mask_transposed: nothing is kept outside a scope (a fresh transposed copy per call); inside, it is made once per
+    mask, and an in-place change of the mask (a new version) is seen. The tests' own key extent is 1 + the last live
+    token (columns for outgoing, rows for incoming), checked by brute force on an asymmetric mask."""
     from boltz_mlx_amd import kernels as K
+    from conftest import mask_key_extent
 
     N = 70
     g = torch.Generator().manual_seed(5)
@@ -40,20 +40,19 @@ def test_pair_mask_scope_extent_and_transpose():
     brute_out = 1 + max(k for k in range(N) if any(m[i, k] != 0 for i in range(N)))
     brute_in = 1 + max(k for k in range(N) if any(m[k, i] != 0 for i in range(N)))
     assert (brute_out, brute_in) == (61, 55)
-    assert K.key_extent(m, N, False) == 0 and K.key_extent(m, N, True) == 0
+    assert mask_key_extent(m, False) == brute_out and mask_key_extent(m, True) == brute_in
+    assert mask_key_extent(torch.zeros(N, N), False) == 0
     t0 = K.mask_transposed(m, N)
     assert torch.equal(t0, m.t()) and t0.is_contiguous() and K.mask_transposed(m, N) is not t0
     with K.pair_mask_scope():
-        assert K.key_extent(m, N, False) == brute_out and K.key_extent(m, N, True) == brute_in
         t1 = K.mask_transposed(m, N)
         assert torch.equal(t1, m.t()) and K.mask_transposed(m.view(N, N), N) is t1  # a view of the same storage
         m[:, 69] = 1  # in place: a new version
-        assert K.key_extent(m, N, False) == N and K.key_extent(m, N, True) == N
         assert torch.equal(K.mask_transposed(m, N), m.t())
         with K.pair_mask_scope():  # nested scopes start empty and restore the outer one
-            assert K.key_extent(torch.zeros(N, N), N, False) == N
+            assert not K._MASK_SCOPE.entries
         assert K.mask_transposed(m, N) is K.mask_transposed(m, N)
-    assert K.key_extent(m, N, False) == 0
+    assert K.mask_transposed(m, N) is not K.mask_transposed(m, N)
 
 
 class _HalfLN:
