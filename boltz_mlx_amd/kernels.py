@@ -96,9 +96,15 @@ def _dt(t: torch.Tensor) -> int:
     raise TypeError(f"unsupported dtype {t.dtype}")
 
 
+# The current stream's handle without the Stream object (6 us of a launch's 20 on the host), where torch has these two.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream():
-    # torch.cuda.current_stream().cuda_stream without the Stream object (6 us of a launch's 20 on the host)
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    if _raw_stream is None or _device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_device())
 
 
 def _p(t):

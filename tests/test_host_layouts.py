@@ -55,6 +55,20 @@ def test_pair_mask_scope_extent_and_transpose():
     assert K.mask_transposed(m, N) is not K.mask_transposed(m, N)
 
 
+def test_stream_without_torchs_raw_handle(monkeypatch):
+    """A torch without the private calls gives the same handle through its public Stream."""
+    from boltz_mlx_amd import kernels as K
+
+    class Stream:
+        cuda_stream = 1234
+
+    monkeypatch.setattr(torch.cuda, "current_stream", Stream)
+    for name in ("_raw_stream", "_device"):
+        with monkeypatch.context() as mp:
+            mp.setattr(K, name, None)
+            assert K._stream() == 1234
+
+
 class _HalfLN:
     """LayerNorm parameters that the kernels cannot read as they are."""
 
