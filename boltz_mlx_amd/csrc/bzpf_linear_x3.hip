@@ -55,6 +55,20 @@ __global__ __launch_bounds__(64 * LXW) void linear_x3_small_k(const float* __res
 #pragma unroll
       for (int rb = 0; rb < RB; rb++) acc[rb] = mfma_x3<false>(wf[X3_W[q]], xf[rb][X3_X[q]], acc[rb]);
   }
+  if (wave_nonfinite(acc)) {  // (bzpf_rowgemm_x3.h)
+#pragma unroll
+    for (int rb = 0; rb < RB; rb++) acc[rb] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int st = 2 * wave; st < 2 * steps; st += (st & 1) ? 2 * LXW - 1 : 1) {  // halves 2 st, 2 st + 1 of a step
+      const f4 wv = ld4(wp + 32 * (st >> 1) + 4 * (st & 1));
+#pragma unroll
+      for (int rb = 0; rb < RB; rb++) {
+        const f4 xv = ld4(xp[rb] + 32 * (st >> 1) + 4 * (st & 1));
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[rb] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[e], xv[e], acc[rb], 0, 0, 0);
+      }
+    }
+  }
 #pragma unroll
   for (int rb = 0; rb < RB; rb++) st4(&Part[wave][16 * rb + r][4 * g], acc[rb]);
   __syncthreads();

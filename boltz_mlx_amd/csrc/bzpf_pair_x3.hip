@@ -12,8 +12,9 @@
 //   triattn_proj     63 / 72 / 237 / 396  ->  16 / 22 / 150 / 240   (675 MB at N = 513: 2.8 TB/s)
 //   linear_resid_ln  13 / 14 /  62 / 100  ->  12 / 14 /  53 /  94   (540 MB at N = 513: 5.7 TB/s)
 //   transition       84 / 90 / 563 / 935  ->  27 / 65 / 342 / 538   (1.15 PFLOP/s of part products)
-// A value that is infinite, or rounds to a bf16 infinity, has no parts: its products are NaN (not inf).
+// Sums that come out not finite are formed again on the fp32 instructions (wave_nonfinite, bzpf_rowgemm_x3.h).
 #include <algorithm>
+#include <type_traits>
 
 #include "bzpf_common.h"
 #include "bzpf_kernels.h"
@@ -45,12 +46,15 @@ __global__ __launch_bounds__(XT) void trimul_proj_x3_k(const float* __restrict__
   int t = __builtin_amdgcn_readfirstlane(wg * XW + (int)(threadIdx.x >> 6));
   RawRow<KIN> raw[2];
   float mk[2];
+  const auto position = [&](int i, int64_t k) {  // of the xn row of output position (i, k)
+    const int64_t kc = k < N ? k : N - 1;
+    return incoming ? kc * N + i : (int64_t)i * N + kc;
+  };
   const auto load = [&](int tt) {
     const int i = tt / tpr, k0 = (tt - i * tpr) * XTW;
 #pragma unroll
     for (int rb = 0; rb < 2; rb++) {
-      const int64_t k = k0 + 16 * rb + r, kc = k < N ? k : N - 1;
-      const int64_t src = incoming ? kc * N + i : (int64_t)i * N + kc;
+      const int64_t src = position(i, k0 + 16 * rb + r);
       raw[rb].load(xn + src * KIN, g);
       mk[rb] = mask[src];
     }
@@ -77,6 +81,15 @@ __global__ __launch_bounds__(XT) void trimul_proj_x3_k(const float* __restrict__
       f4 pa[2] = {}, ga[2] = {};
       mma_x3<2, true, KIN>(pa, x, Ws + 16 * cb * ldx<KIN>(), PLANE_W);
       mma_x3<2, true, KIN>(ga, x, Ws + (64 + 16 * cb) * ldx<KIN>(), PLANE_W);
+      const f4 all[4] = {pa[0], pa[1], ga[0], ga[1]};
+      if (wave_nonfinite(all)) {
+        const float* xr[2];
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++) xr[rb] = xn + position(i, k0 + 16 * rb + r) * KIN;
+        const float* wr = w + (int64_t)(c_lo + 16 * cb + r) * KIN;
+        mma_f32<2, true, KIN>(pa, wr, xr);
+        mma_f32<2, true, KIN>(ga, wr + (int64_t)2 * KIN * KIN, xr);
+      }
 #pragma unroll
       for (int rb = 0; rb < 2; rb++) {
         f4 v;
@@ -106,13 +119,14 @@ __global__ __launch_bounds__(XT) void triattn_proj_x3_k(const float* __restrict_
   int t = __builtin_amdgcn_readfirstlane(wg * XW + (int)(threadIdx.x >> 6));
   const int64_t NN = N * N;
   RawRow<KIN> raw[2];
+  const auto xrow = [&](int i, int64_t j) {
+    const int64_t jc = j < N ? j : N - 1;
+    return xn + (trans ? jc * N + i : (int64_t)i * N + jc) * KIN;
+  };
   const auto load = [&](int tt) {
     const int i = tt / tpr, j0 = (tt - i * tpr) * XTW;
 #pragma unroll
-    for (int rb = 0; rb < 2; rb++) {
-      const int64_t j = j0 + 16 * rb + r, jc = j < N ? j : N - 1;
-      raw[rb].load(xn + (trans ? jc * N + i : (int64_t)i * N + jc) * KIN, g);
-    }
+    for (int rb = 0; rb < 2; rb++) raw[rb].load(xrow(i, j0 + 16 * rb + r), g);
   };
   load(min(t, ntiles - 1));
   const float* wg0 = w + (int64_t)grp * HC * KIN;
@@ -131,6 +145,13 @@ __global__ __launch_bounds__(XT) void triattn_proj_x3_k(const float* __restrict_
 #pragma unroll
     for (int rb = 0; rb < 2; rb++) split_row(x[rb], raw[rb]);
     load(min(t + stride, ntiles - 1));
+    // a block again in fp32 (sums that are not finite): LDS weight rows rr0 .. rr0 + 15
+    const auto again = [&](auto rows, f4 (&acc)[2], int rr0) {
+      if (!wave_nonfinite(acc)) return;
+      const float* wr = wrow(rr0 + r);
+      const float* const xr[2] = {xrow(i, j0 + r), xrow(i, j0 + 16 + r)};
+      mma_f32<2, decltype(rows)::value, KIN>(acc, wr != nullptr ? wr : w, xr);  // (no row: a bias row that is not stored)
+    };
     // ROWS orientation: key j0 + 16 rb + 4 g + e is inside the row
     const auto valid = [&](int rb, int e) { return j0 + 16 * rb + 4 * g + e < N ? 1.0f : 0.0f; };
     if (grp == 2) {
@@ -138,6 +159,7 @@ __global__ __launch_bounds__(XT) void triattn_proj_x3_k(const float* __restrict_
       for (int cb = 0; cb < 8; cb++) {
         f4 acc[2] = {};
         mma_x3<2, true, KIN>(acc, x, Ws + 16 * cb * ldx<KIN>(), PLANE_W);
+        again(std::true_type(), acc, 16 * cb);
         const int ch = 16 * cb + r, h = ch / C, d = ch - h * C;
         float* vp = vt + (((int64_t)h * N + i) * C + d) * ldk + j0 + 4 * g;
 #pragma unroll
@@ -154,6 +176,8 @@ __global__ __launch_bounds__(XT) void triattn_proj_x3_k(const float* __restrict_
       f4 a0[2] = {}, a1[2] = {};
       mma_x3<2, false, KIN>(a0, x, Ws + 32 * m * ldx<KIN>(), PLANE_W);
       mma_x3<2, false, KIN>(a1, x, Ws + (32 * m + 16) * ldx<KIN>(), PLANE_W);
+      again(std::false_type(), a0, 32 * m);
+      again(std::false_type(), a1, 32 * m + 16);
       const int within = 32 * m + 8 * g, h = within / C, d = within - h * C;
       const int64_t plane = (int64_t)(grp == 3 ? 2 : grp) * H + h;
 #pragma unroll
@@ -168,6 +192,7 @@ __global__ __launch_bounds__(XT) void triattn_proj_x3_k(const float* __restrict_
     if (grp == 3) {
       f4 acc[2] = {};
       mma_x3<2, true, KIN>(acc, x, Ws + HC * ldx<KIN>(), PLANE_W);
+      again(std::true_type(), acc, HC);
       if (r < H) {
 #pragma unroll
         for (int rb = 0; rb < 2; rb++) {
@@ -201,6 +226,7 @@ __global__ __launch_bounds__(256, 3) void trimul_tail_x3_k(const float* __restri
   const int t = threadIdx.x, wave = t >> 6, l = t & 63, g = l >> 4, r = l & 15;
   const int64_t jp = j0 + 16 * wave + r, zr = jp < N ? (int64_t)i * N + jp : -1;
   const auto zrow = [&](int) { return zr; };
+  const auto xrow = [&]() { return xn + ((int64_t)i * N + (jp < N ? jp : N - 1)) * D; };
   // o block of this thread: 4 channels 4 cq .. + 3, positions 4 (4 u + t % 4) .. + 3
   constexpr int UN = D / 64;  // (D / 4) x 16 blocks of the tile on 256 threads
 #pragma unroll
@@ -242,23 +268,26 @@ __global__ __launch_bounds__(256, 3) void trimul_tail_x3_k(const float* __restri
   // LN_out of this lane's position, channels D / 4 g .. + D / 4 - 1 (the rest in lanes l ^ 16, l ^ 32, l ^ 48)
   RawRow<D> of;
   of.load(Ts + (16 * wave + r) * LDT, g);
-  float sum = 0.f, ss = 0.f;
+  const auto ln_out = [&]() {
+    float sum = 0.f, ss = 0.f;
 #pragma unroll
-  for (int j = 0; j < D / 16; j++) sum += of.v[j][0] + of.v[j][1] + of.v[j][2] + of.v[j][3];
-  const float mean = xgroups_sum(sum) * (1.0f / D);
+    for (int j = 0; j < D / 16; j++) sum += of.v[j][0] + of.v[j][1] + of.v[j][2] + of.v[j][3];
+    const float mean = xgroups_sum(sum) * (1.0f / D);
 #pragma unroll
-  for (int j = 0; j < D / 16; j++) {
-    of.v[j] = of.v[j] - mean;
-    ss += of.v[j][0] * of.v[j][0] + of.v[j][1] * of.v[j][1] + of.v[j][2] * of.v[j][2] + of.v[j][3] * of.v[j][3];
-  }
-  const float rstd = 1.0f / sqrtf(xgroups_sum(ss) * (1.0f / D) + eps_out);
-#pragma unroll
-  for (int j = 0; j < D / 16; j++)
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const int c = D / 4 * g + 4 * j + e;
-      of.v[j][e] = of.v[j][e] * rstd * now[c] + nob[c];
+    for (int j = 0; j < D / 16; j++) {
+      of.v[j] = of.v[j] - mean;
+      ss += of.v[j][0] * of.v[j][0] + of.v[j][1] * of.v[j][1] + of.v[j][2] * of.v[j][2] + of.v[j][3] * of.v[j][3];
     }
+    const float rstd = 1.0f / sqrtf(xgroups_sum(ss) * (1.0f / D) + eps_out);
+#pragma unroll
+    for (int j = 0; j < D / 16; j++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int c = D / 4 * g + 4 * j + e;
+        of.v[j][e] = of.v[j][e] * rstd * now[c] + nob[c];
+      }
+  };
+  ln_out();
   __syncthreads();  // every wave has read its o rows: the chunks take the LDS
   wstore(0);
   wload(1);
@@ -274,15 +303,30 @@ __global__ __launch_bounds__(256, 3) void trimul_tail_x3_k(const float* __restri
       const int cb = 2 * (q % NCH) + h;
       f4 acc[1] = {};
       mma_x3<1, false, D>(acc, x, W + 16 * h * ldx<D>(), PLANE_W);
+      if (q >= NCH && wave_nonfinite(acc)) {
+        const float* const xr[1] = {xrow()};
+        mma_f32<1, false, D>(acc, opaque_ptr(w_go) + (16 * cb + r) * D, xr);
+      }
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         if (q < NCH) y[0][cb][e] = acc[0][e];
         else y[0][cb][e] *= sigmoidf_(acc[0][e]);
       }
     }
-    if (q == NCH - 1) {  // the gates' input rows, loaded once the LN_out parts are done with
+    if (q == NCH - 1) {
+      if (wave_nonfinite(y[0])) {
+        const float* op = opaque_ptr(o) + ((int64_t)(D / 4 * g) * N + i) * ld + jp;
+#pragma unroll
+        for (int j = 0; j < D / 16; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++, op += N * ld) of.v[j][e] = *op;
+        ln_out();
+#pragma unroll
+        for (int cb2 = 0; cb2 < CB; cb2++) y[0][cb2] = mma_f32<false, D>(w_po + (16 * cb2 + r) * D, of);
+      }
+      // the gates' input rows, loaded once the LN_out parts are done with
       RawRow<D> raw;
-      raw.load(xn + ((int64_t)i * N + (jp < N ? jp : N - 1)) * D, g);
+      raw.load(xrow(), g);
       split_row(x[0], raw);
     }
     if (q + 1 < 2 * NCH) {
@@ -341,6 +385,15 @@ __global__ __launch_bounds__(XT) void linear_resid_ln_x3_k(const float* __restri
       y[0][cb] = acc[0];
       __builtin_amdgcn_sched_barrier(0);
     }
+    if (wave_nonfinite(y[0])) {
+      const float* const xr[1] = {x_in + min((int64_t)t * 16 + r, NN - 1) * K};
+#pragma unroll
+      for (int cb = 0; cb < CB; cb++) {
+        f4 acc[1];
+        mma_f32<1, false, K>(acc, w + (16 * cb + r) * K, xr);
+        y[0][cb] = acc[0];
+      }
+    }
     const int64_t zr = zrow_of(t);
     resid_ln_apply<float, 1>(y, zv, [&](int) { return zr; }, z, lw, lns.b, eps, xn_next);
   }
@@ -370,22 +423,25 @@ __global__ __launch_bounds__(256, 2) void pair_bias_x3_k(const float* __restrict
   }
   stage_ln(lns, lnw, lnb);
   __syncthreads();
-  for (; t < ntiles; t += stride) {
+  const auto ln = [&](RawRow<D>& v) {
     float sum = 0.f, ss = 0.f;
 #pragma unroll
-    for (int j = 0; j < D / 16; j++) sum += raw.v[j][0] + raw.v[j][1] + raw.v[j][2] + raw.v[j][3];
+    for (int j = 0; j < D / 16; j++) sum += v.v[j][0] + v.v[j][1] + v.v[j][2] + v.v[j][3];
     const float mean = xgroups_sum(sum) * (1.0f / D);
 #pragma unroll
     for (int j = 0; j < D / 16; j++) {
-      raw.v[j] = raw.v[j] - mean;
-      ss += raw.v[j][0] * raw.v[j][0] + raw.v[j][1] * raw.v[j][1] + raw.v[j][2] * raw.v[j][2] + raw.v[j][3] * raw.v[j][3];
+      v.v[j] = v.v[j] - mean;
+      ss += v.v[j][0] * v.v[j][0] + v.v[j][1] * v.v[j][1] + v.v[j][2] * v.v[j][2] + v.v[j][3] * v.v[j][3];
     }
     const float rstd = 1.0f / sqrtf(xgroups_sum(ss) * (1.0f / D) + eps);
 #pragma unroll
     for (int j = 0; j < D / 16; j++) {
       const int c = D / 4 * g + 4 * j;
-      raw.v[j] = raw.v[j] * rstd * ld4(lns.w + c) + ld4(lns.b + c);
+      v.v[j] = v.v[j] * rstd * ld4(lns.w + c) + ld4(lns.b + c);
     }
+  };
+  for (; t < ntiles; t += stride) {
+    ln(raw);
     X3Row<D> x;
     split_row(x, raw);
     load(min(t + stride, ntiles - 1));
@@ -394,6 +450,13 @@ __global__ __launch_bounds__(256, 2) void pair_bias_x3_k(const float* __restrict
     for (int q = 0; q < 6; q++)
 #pragma unroll
       for (int s = 0; s < D / 32; s++) acc = mfma_x3<true>(wx.p[X3_W[q]][s], x.p[X3_X[q]][s], acc);
+    const f4 all[1] = {acc};
+    if (wave_nonfinite(all)) {
+      RawRow<D> v;
+      v.load(z + min((int64_t)t * 16 + r, rows - 1) * D, g);
+      ln(v);
+      acc = mma_f32<true, D>(w + (int64_t)min(r, H - 1) * D, v);
+    }
     if (r < H) {
 #pragma unroll
       for (int e = 0; e < 4; e++) {
@@ -409,6 +472,47 @@ __global__ __launch_bounds__(256, 2) void pair_bias_x3_k(const float* __restrict
 // operand of out += fc3 a, a lane's k slots 8 g + t being units 16 (t / 4) + 4 g + t % 4 of a 32-unit slice.
 __device__ __forceinline__ void split_units(X3Row<32>& b, const f4& lo, const f4& hi) {
   split8(lo, hi, b.p[0][0], b.p[1][0], b.p[2][0]);
+}
+
+// out = fc3 (silu(fc1 x) * fc2 x) over the 32-unit slices sl0, sl0 + step, ... on the fp32 matrix instructions, for a wave
+// whose sums came out not finite (xr[rb]: the lane's rows of xn). A lane holds units 4 g + e of its row: step e of fc3.
+template <int RB>
+__device__ __forceinline__ void transition_f32(f4 (&out)[RB][8], const float* const (&xr)[RB], const float* w12,
+                                               const float* w3, int hidden, int sl0, int step) {
+  constexpr int D = 128;
+  const int l = threadIdx.x & 63, g = l >> 4, r = l & 15;
+  zero_acc(out);
+#pragma unroll 1
+  for (int u0 = 32 * sl0; u0 < hidden; u0 += (u0 & 16) ? 32 * step - 16 : 16) {
+    f4 a[RB], h2[RB];
+    mma_f32<RB, false, D>(a, w12 + (int64_t)(u0 + r) * D, xr);
+    mma_f32<RB, false, D>(h2, w12 + (int64_t)(hidden + u0 + r) * D, xr);
+#pragma unroll
+    for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) a[rb][e] = siluf_(a[rb][e]) * h2[rb][e];
+#pragma unroll
+    for (int ob = 0; ob < 8; ob++) {
+      const f4 wv = ld4(w3 + (int64_t)(16 * ob + r) * hidden + u0 + 4 * g);
+#pragma unroll
+      for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          out[rb][ob] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[e], a[rb][e], out[rb][ob], 0, 0, 0);
+    }
+  }
+}
+template <int RB, typename RowFn>
+__device__ __forceinline__ void transition_finite(f4 (&out)[RB][8], const float* xn, RowFn row, int64_t rows_total,
+                                                  const float* w12, const float* w3, int hidden, int sl0, int step) {
+  bool bad = false;
+#pragma unroll
+  for (int rb = 0; rb < RB; rb++) bad = wave_nonfinite(out[rb]) || bad;
+  if (!bad) return;
+  const float* xr[RB];
+#pragma unroll
+  for (int rb = 0; rb < RB; rb++) xr[rb] = xn + min(row(rb), rows_total - 1) * 128;
+  transition_f32<RB>(out, xr, w12, w3, hidden, sl0, step);
 }
 
 // Large inputs: tiles of 128 RB rows (8 waves of 16 RB), the hidden units streamed through LDS in chunks of 32 (fc1, fc2 rows
@@ -502,6 +606,7 @@ __global__ __launch_bounds__(XT) void transition_x3_k(const float* __restrict__ 
         for (int rb = 0; rb < RB; rb++) out[rb][ob] = mfma_x3<false>(wf[X3_W[q]], b[rb].p[X3_X[q]][0], out[rb][ob]);
     }
   }
+  transition_finite<RB>(out, xn, [&](int rb) { return row[rb]; }, rows_total, w12, w3, hidden, 0, 1);
   resid_ln_rows<float, RB>(out, [&](int rb) -> int64_t { return row[rb] < rows_total ? row[rb] : -1; }, z, accumulate,
                           lnw, lnb, eps, xn_next);
 }
@@ -582,6 +687,7 @@ __global__ __launch_bounds__(XT) void transition_x3_small_k(const float* __restr
         for (int rb = 0; rb < RB; rb++) out[rb][ob] = mfma_x3<false>(wf[X3_W[q]], b[rb].p[X3_X[q]][0], out[rb][ob]);
     }
   }
+  transition_finite<RB>(out, xn, [&](int rb) { return r0 + 16 * rb + r; }, rows_total, w12, w3, hidden, wave, XW);
 #pragma unroll
   for (int rb = 0; rb < RB; rb++)
 #pragma unroll

@@ -69,6 +69,55 @@ __device__ __forceinline__ void mma_x3(f4 (&acc)[RB], const X3Row<KIN> (&x)[RB],
       for (int rb = 0; rb < RB; rb++) acc[rb] = mfma_x3<ROWS>(a[X3_W[q]][s], x[rb].p[X3_X[q]][s], acc[rb]);
 }
 
+// Values without parts. An infinity, and a finite value from 2^128 - 2^119 on (it rounds to a bf16 infinity), splits into
+// an infinity and NaNs, and a product within 2^-8 of the largest fp32 value may pass it where its rounded parts meet.
+// Each way the sum comes out not finite, so a wave that finds such a sum forms its block again on the fp32 matrix
+// instructions, operands straight from memory, and gives what an fp32 product gives: the infinity, the NaN of inf - inf
+// or 0 inf, or the finite value. Finite sums pay one v_fma each and a branch.
+template <int NV>
+__device__ __forceinline__ bool wave_nonfinite(const f4 (&v)[NV]) {
+  float t = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; i++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) t = fmaf(v[i][e], 0.f, t);
+  return __any(t != t);
+}
+// acc[rb] = W[0 .. 15][0 : KIN] . X[rb]^T (ROWS: transposed) in fp32: wrow and xrow[rb] are the lane's rows (l % 16) in
+// memory.
+template <int RB, bool ROWS, int KIN>
+__device__ __forceinline__ void mma_f32(f4 (&acc)[RB], const float* wrow, const float* const (&xrow)[RB]) {
+  const int c0 = KIN / 4 * ((threadIdx.x & 63) >> 4);
+#pragma unroll
+  for (int rb = 0; rb < RB; rb++) acc[rb] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int j = 0; j < KIN / 4; j += 4) {
+    const f4 a = ld4(wrow + c0 + j);
+#pragma unroll
+    for (int rb = 0; rb < RB; rb++) {
+      const f4 b = ld4(xrow[rb] + c0 + j);
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+        acc[rb] = ROWS ? __builtin_amdgcn_mfma_f32_16x16x4f32(b[t], a[t], acc[rb], 0, 0, 0)
+                       : __builtin_amdgcn_mfma_f32_16x16x4f32(a[t], b[t], acc[rb], 0, 0, 0);
+    }
+  }
+}
+// The same over a row in registers.
+template <bool ROWS, int KIN>
+__device__ __forceinline__ f4 mma_f32(const float* wrow, const RawRow<KIN>& x) {
+  f4 acc = {};
+#pragma unroll
+  for (int j = 0; j < KIN / 16; j++) {
+    const f4 a = ld4(wrow + KIN / 4 * ((threadIdx.x & 63) >> 4) + 4 * j);
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+      acc = ROWS ? __builtin_amdgcn_mfma_f32_16x16x4f32(x.v[j][t], a[t], acc, 0, 0, 0)
+                 : __builtin_amdgcn_mfma_f32_16x16x4f32(a[t], x.v[j][t], acc, 0, 0, 0);
+  }
+  return acc;
+}
+
 // Stage ROWS weight rows of KIN fp32 values, split, into LDS planes; row r comes from src(r) (nullptr: zeros). The
 // loads of a batch are issued together (a weight block is cold in a CU's caches: one round trip, not one per vector).
 template <int NROWS, int KIN, int THREADS, typename RowFn>

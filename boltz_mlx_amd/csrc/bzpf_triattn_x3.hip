@@ -20,8 +20,9 @@
 // unmasked key are skipped where that cannot change a bit: a masked key's logit is about inf*log2(e) below the
 // maximum, and 2^x is exactly zero in fp32 below x = -150 (inf >= 1e6 leaves room for any spread of the logits).
 // The maximum is raised lazily: probabilities are formed against the current one, and only a lane whose sum of a tile's
-// passes 2^15 (or is not a number) makes the wave raise it. Operands that are not finite give NaN where the fp32
-// product would give an infinity (an infinity has no finite second part).
+// passes 2^15 (or is not a number) makes the wave raise it. v_exp_f32 gives 0 below 2^-126, so a key whose weight is less than
+// 2^-126 of the row's largest has none. A wave whose sums come out not finite (an operand without parts, bzpf_rowgemm_x3.h;
+// values so large that 2^15 of them overflow) forms its queries again in fp32.
 // Reference behaviour: boltz_mlx/layers/triangular_attention/attention.py:27-93, kernels.py:538-600.
 #include "bzpf_common.h"
 #include "bzpf_kernels.h"
@@ -251,6 +252,60 @@ __global__ __launch_bounds__(256, 3) void triattn_core_x3_k(const float* __restr
     }
   }
   if (!wact) return;
+  float t0 = lsum * 0.f;
+#pragma unroll
+  for (int e = 0; e < 16; e++) t0 = fmaf(oacc[e], 0.f, t0);
+  if (__any(jq < N && t0 != t0)) {
+    // Sums that are not finite: the wave's queries again in fp32 throughout (v_mfma_f32_32x32x2_f32, one k of each lane
+    // half a step), operands straight from memory, probabilities relative to the true running maximum.
+    const float* qr = qp + (int64_t)(jq < N ? jq : N - 1) * C + 4 * hl;
+    const float* vr = vp + (int64_t)qi * ldk + 4 * hl;
+    m_run = -INFINITY;
+    lsum = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; e++) oacc[e] = 0.f;
+#pragma unroll 1
+    for (int kb = 0; kb < nblk; kb++) {
+      const int k0 = kb * XBK;
+      const float* kr = kp + (int64_t)min(k0 + qi, N - 1) * C + 4 * hl;
+      f16x s;
+#pragma unroll
+      for (int e = 0; e < 16; e++) s[e] = 0.f;
+#pragma unroll 1
+      for (int c = 0; c < C; c += 8) {
+        const f4 kv = *reinterpret_cast<const f4*>(kr + c), qv = *reinterpret_cast<const f4*>(qr + c);
+#pragma unroll
+        for (int e = 0; e < 4; e++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[e], qv[e], s, 0, 0, 0);
+      }
+      float mx = -INFINITY;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const f4 b = ldb(brs, xcore_b_lane(q, l), xcore_b_stage(kb));
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int k = k0 + 8 * q + 4 * hl + e;
+          const float mb = k < N ? inf * (mrow[(int64_t)k * mask_sk] - 1.0f) * LOG2E : -INFINITY;
+          s[4 * q + e] = k < N ? (s[4 * q + e] + mb) + b[e] : -INFINITY;
+          mx = fmaxf(mx, s[4 * q + e]);
+        }
+      }
+      const float mn = fmaxf(m_run, halves_max(mx)), corr = exp2f(m_run - mn);
+      oacc *= corr;
+      lsum *= corr;
+      m_run = mn;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        f4 vv = *reinterpret_cast<const f4*>(vr + k0 + 8 * q);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          if (k0 + 8 * q + 4 * hl + e >= N) vv[e] = 0.0f;
+          const float p = exp2f(s[4 * q + e] - mn);
+          lsum += p;
+          oacc = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[e], p, oacc, 0, 0, 0);
+        }
+      }
+    }
+  }
   const float ltot = halves_sum(lsum);
   if (jq >= N) return;
   const float inv = 1.0f / ltot;

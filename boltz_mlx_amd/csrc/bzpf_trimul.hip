@@ -137,6 +137,16 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void trimul_contract_x3_k(const fl
 #pragma unroll
       for (int n = 0; n < NB; n++) acc[m][n] = mfma_parts6(fa[m], fb[n], acc[m][n]);
   }
+  // sums that are not finite: the wave's blocks again on the fp32 matrix instructions, rows straight from memory
+  // (bzpf_rowgemm_x3.h says which operands lead here)
+  float t0 = 0.f;
+#pragma unroll
+  for (int m = 0; m < MB; m++)
+#pragma unroll
+    for (int n = 0; n < NB; n++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) t0 = fmaf(acc[m][n][e], 0.f, t0);
+  const bool again = __any(t0 != t0);
   // acc[m][n][4 q + e] = o[i0 + 32 MB wi + 32 m + 8 q + 4 hl + e][j0 + 32 NB wj + 32 n + r32]
   float* oc = o + c * N * ld;
 #pragma unroll
@@ -144,6 +154,19 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void trimul_contract_x3_k(const fl
 #pragma unroll
     for (int n = 0; n < NB; n++) {
       const int64_t j = j0 + 32 * NB * wj + 32 * n + r32;
+      if (again) {
+        const float* ar = a + min((int64_t)(i0 + 32 * (MB * wi + m) + r32), N - 1) * ld + 4 * hl;
+        const float* br = b + min(j, N - 1) * ld + 4 * hl;
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[m][n][e] = 0.f;
+#pragma unroll 1
+        for (int k0 = 0; k0 < nst * KS; k0 += 8) {
+          const f4 va = ld4(ar + k0), vb = ld4(br + k0);
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[e], vb[e], acc[m][n], 0, 0, 0);
+        }
+      }
       if (j >= ld) continue;
 #pragma unroll
       for (int q = 0; q < 4; q++)

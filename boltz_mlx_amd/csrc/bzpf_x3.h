@@ -3,7 +3,9 @@
 // together), and a product is taken as the six part products x_a y_b with a + b <= 4, accumulated in fp32 by
 // v_mfma_f32_32x32x16_bf16 (exact bf16 products, fp32 sums); the three left out (x2 y3, x3 y2, x3 y3) are below
 // 2^-23 of |x y| together. That is the fp32 matrix cores' accuracy at 6 / 16 of their time (the bf16 rate is 16
-// times the fp32 one). Operands sit in LDS as three K-contiguous planes (one per part) of KS = 16 bf16 per row.
+// times the fp32 one). Limits: parts end at bf16's smallest value, 2^-133, so an operand below 2^-112 keeps fewer than 24 bits
+// (an absolute 2^-134 at most is lost: beside operands of ordinary size nothing, in sums of such operands alone 6e-7 of the
+// result at 2^-114, 1e-3 at 2^-125); and an operand that rounds to a bf16 infinity has no parts. Operands sit in LDS as three K-contiguous planes (one per part) of KS = 16 bf16 per row.
 #pragma once
 #include "bzpf_common.h"
 
