@@ -1,5 +1,5 @@
-// Layout kernels of the pair updates at any channel count (the template stack's c_z = 64; the fused kernels in
-// bzpf_pair_gemm.hip are built for 128 channels). The projections themselves are bzpf_linear GEMMs whose [N*N, cols]
+// Layout kernels of the pair updates at the channel counts and head shapes that have no fused kernels (those of
+// bzpf_pair_gemm.hip and bzpf_pair_x3.hip are built for 128 and 64 channels, H C = 128). The projections themselves are bzpf_linear GEMMs whose [N*N, cols]
 // outputs these kernels gate, mask and move into the layouts the contraction and the attention core read:
 //   trimul_pack      : ab[c][i][k] = P[p][c] * sigmoid(P[p][2D + c]) * mask[p] * scale, p = (i, k) outgoing or (k, i)
 //                      incoming, from P = xn [p_in; g_in]^T (boltz_mlx/layers/triangular_mult.py:40-65);

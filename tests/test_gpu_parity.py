@@ -241,6 +241,45 @@ def test_tri_att(precision, starting, N):
     check(f"tri_att_{'start' if starting else 'end'} N={N}", got, ref, precision)
 
 
+# a width without fused kernels; inside one 64-position step of the layout kernels and past it
+@pytest.mark.parametrize("precision", ["fp32", "f16"], indirect=True)
+@pytest.mark.parametrize("first", [True, False])
+@pytest.mark.parametrize("N", [17, 70])
+def test_triangle_modules_at_192_channels(precision, first, N):
+    """The GEMM + layout path (csrc/bzpf_pack.hip) as the modules take it where no fused kernel is built."""
+    from boltz_mlx_amd.layers.triangular_attention.attention import (TriangleAttentionEndingNode,
+                                                                     TriangleAttentionStartingNode)
+    from boltz_mlx_amd.layers.triangular_mult import TriangleMultiplicationIncoming, TriangleMultiplicationOutgoing
+
+    D, C, H = 192, 32, 4
+    x, _, pm = pair_inputs(N, D, seed=N, n_pad=N // 5)
+    pm[0, 1, 2] = 0
+    p = rand_params(shapes_tri_mul(D), seed=100 + N, std=0.1)
+    odt = oracle_dtype(precision)
+    ref = O.tri_mul(x.astype(odt), pm.astype(odt), cast(p, odt), first)
+    mod = load((TriangleMultiplicationOutgoing if first else TriangleMultiplicationIncoming)(D), p)
+    check(f"tri_mul D={D} N={N}", mod(dev(x), dev(pm)).cpu().numpy(), ref, precision)
+    p = rand_params(shapes_tri_att(D, C, H), seed=200 + N, std=0.1)
+    ref = O.tri_att(x.astype(np.float32), pm.astype(np.float32), cast(p, np.float32), first, row_chunk=16)
+    mod = load((TriangleAttentionStartingNode if first else TriangleAttentionEndingNode)(D, C, H), p)
+    check(f"tri_att D={D} N={N}", mod(dev(x), dev(pm)).cpu().numpy(), ref, precision)
+
+
+@pytest.mark.parametrize("precision", ["fp32", "f16"], indirect=True)
+@pytest.mark.parametrize("starting", [True, False])
+def test_tri_att_64_channels_other_head_shape(precision, starting):
+    """2 heads of 32 channels at c_in = 64: H * C = 64 has no fused kernels either."""
+    from boltz_mlx_amd.layers.triangular_attention.attention import (TriangleAttentionEndingNode,
+                                                                     TriangleAttentionStartingNode)
+
+    N, D, C, H = 70, 64, 32, 2
+    p = rand_params(shapes_tri_att(D, C, H), seed=7, std=0.1)
+    x, _, pm = pair_inputs(N, D, seed=8, n_pad=9)
+    ref = O.tri_att(x.astype(np.float32), pm.astype(np.float32), cast(p, np.float32), starting, row_chunk=16)
+    mod = load(TriangleAttentionStartingNode(D, C, H) if starting else TriangleAttentionEndingNode(D, C, H), p)
+    check("tri_att D=64 H=2", mod(dev(x), dev(pm)).cpu().numpy(), ref, precision)
+
+
 @pytest.mark.parametrize("precision", ["fp32", "f16"], indirect=True)
 @pytest.mark.parametrize("starting", [True, False])
 @pytest.mark.parametrize("N", [17, 117])

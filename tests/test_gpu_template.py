@@ -1,7 +1,7 @@
-"""The pair updates at 64 channels (the template stack's PairformerNoSeqLayer / Module, c_z = 64) on the GEMM +
-layout-kernel path (csrc/bzpf_pack.hip), against the oracle (oracle/msa.py::pairformer_noseq_layer, which is
-generic in the channel count). The layout kernels are also pinned at 128 channels against the fused projection
-kernels they stand in for: the same buffers from the same inputs."""
+"""The pair updates at 64 channels (the template stack's PairformerNoSeqLayer / Module, c_z = 64) on the fused pair
+kernels' 64-channel forms, against the oracle (oracle/msa.py::pairformer_noseq_layer, which is generic in the channel
+count). The layout kernels of the other widths (csrc/bzpf_pack.hip) are pinned at 128 channels against the fused
+projection kernels they stand in for: the same buffers from the same inputs."""
 
 from __future__ import annotations
 
