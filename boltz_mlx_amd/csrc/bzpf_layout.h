@@ -91,6 +91,17 @@ BZPF_HD inline int64_t xcore_k_extent(int64_t N, int C) { return N * C * 4; }
 BZPF_HD inline int64_t xcore_v_extent(int64_t ldk, int C) { return C * ldk * 4; }
 BZPF_HD inline int64_t xcore_b_extent(int64_t ldk) { return ldk / 64 * 8192; }
 
+// ---- the fp32 transition (bzpf_pair_x3.hip) over `cus` compute units: `full` rows in whole rounds of one 256-row tile a
+// CU, then the remaining rows in tiles of `tile` rows.
+struct TransitionSplit {
+  int64_t full;
+  int tile;
+};
+BZPF_HD inline TransitionSplit transition_split(int64_t rows, int64_t cus) {
+  const int64_t full = rows / (256 * cus) * (256 * cus), rem = rows - full;
+  return {full, rem <= 16 * cus ? 16 : rem <= 64 * cus ? 32 : rem <= 128 * cus ? 128 : 256};
+}
+
 // ---- the fp16 contraction (bzpf_trimul.hip): per channel, rows of ld fp16 values; a load's lane offset holds the
 // row (rows of a 256-row tile, past N reading as zero) and its 16-byte chunk, the scalar offset the 64-element stage.
 BZPF_HD inline int64_t contract_extent(int64_t N, int64_t ld) { return N * ld * 2; }

@@ -822,26 +822,32 @@ hipError_t launch_transition_x3(const float* xn, const float* w12, const float* 
                                 const float* lnw, const float* lnb, float eps, float* xn_next, int64_t rows,
                                 int hidden, hipStream_t st) {
   if (hidden % 32 || rows > (1LL << 34)) return hipErrorInvalidValue;
-  // Whole rounds of 256-row tiles over the 256 CUs, then the remaining rows in the form that takes them soonest
-  // (512 hidden units, us): 16-row tiles with the hidden units split over the waves 27 up to 4,096 rows, 32-row ones 31
-  // a round of 8,192 rows (16,384: 64), 128-row tiles 74 up to 32,768 (32-row ones
-  // 120), 256-row tiles 105 to 128 up to 65,536. 263,169 rows: 538 (1,029 256-row tiles alone 561, fp32 MFMA 935).
-  constexpr int64_t ROUND = 256 * 256;
+  // Whole rounds of one 256-row tile a CU (the kernel's LDS lets one workgroup in), then the remaining rows in the form that
+  // takes them soonest (transition_split). On 256 CUs, 512 hidden units, us: 16-row tiles with the hidden units split over
+  // the waves 27 up to 4,096 rows, 32-row ones 31 a round of 8,192 rows (16,384: 64), 128-row tiles 74 up to 32,768
+  // (32-row ones 120), 256-row tiles 105 to 128 up to 65,536. 263,169 rows: 538 (1,029 256-row tiles alone 561, fp32 MFMA
+  // 935).
+  static int cache[kMaxDevices];
+  const int cus = x3_resident(transition_x3_k<2>, cache);
+  if (cus <= 0) return hipErrorInvalidDevice;
   const auto part = [&](int64_t r0, int64_t n, auto kernel, int64_t tile) {
     kernel<<<(unsigned)((n + tile - 1) / tile), XT, 0, st>>>(xn + r0 * 128, w12, w3, z + r0 * 128, accumulate, lnw, lnb,
                                                              eps, xn_next != nullptr ? xn_next + r0 * 128 : nullptr, n,
                                                              hidden);
     return hipGetLastError();
   };
-  const int64_t full = rows / ROUND * ROUND, rem = rows - full;
+  const TransitionSplit split = transition_split(rows, cus);
+  const int64_t full = split.full, rem = rows - full;
   if (full > 0) {
     const hipError_t e = part(0, full, transition_x3_k<2>, 256);
     if (e != hipSuccess || rem == 0) return e;
   }
-  if (rem <= 4096) return part(full, rem, transition_x3_small_k<1>, 16);
-  if (rem <= 16384) return part(full, rem, transition_x3_small_k<2>, 32);
-  if (rem <= 32768) return part(full, rem, transition_x3_k<1>, 128);
-  return part(full, rem, transition_x3_k<2>, 256);
+  switch (split.tile) {
+    case 16: return part(full, rem, transition_x3_small_k<1>, 16);
+    case 32: return part(full, rem, transition_x3_small_k<2>, 32);
+    case 128: return part(full, rem, transition_x3_k<1>, 128);
+    default: return part(full, rem, transition_x3_k<2>, 256);
+  }
 }
 
 }  // namespace bzpf

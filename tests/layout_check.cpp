@@ -180,6 +180,18 @@ extern "C" int lc_check(char* out, int cap) {
                                4 * tb_offset(0, l & 31, 32 * st + 8 * v + 4 * (l >> 5) + e, N, ldk);
     rep.line(same, "fp32 core bias loads follow tb_offset N=" + std::to_string(N));
   }
+  // The fp32 transition's split: whole rounds of the device's CUs, the rest in at most one round of the form it takes (two
+  // of the 32-row form), on devices of 256 CUs and of fewer.
+  for (int64_t cus : {1, 32, 64, 256, 304}) {
+    bool ok = true;
+    for (int64_t rows : {(int64_t)1, 16 * cus, 16 * cus + 1, 64 * cus, 64 * cus + 1, 128 * cus, 128 * cus + 1, 256 * cus - 1,
+                         256 * cus, 256 * cus + 1, 5 * 256 * cus + 64 * cus}) {
+      const TransitionSplit t = transition_split(rows, cus);
+      const int64_t rem = rows - t.full, tiles = (rem + t.tile - 1) / t.tile;
+      ok = ok && t.full % (256 * cus) == 0 && rem >= 0 && rem < 256 * cus && tiles <= (t.tile == 32 ? 2 : 1) * cus;
+    }
+    rep.line(ok, "fp32 transition rounds on " + std::to_string(cus) + " CUs");
+  }
   // The contraction: the largest N its launcher accepts, and one past it.
   {
     int64_t nmax = 0;
