@@ -8,7 +8,7 @@
 // Reference behaviour: the nn.Linear / lin16 calls these replace (boltz_mlx/kernels.py:1360-1370;
 // boltz_mlx/modules/transformersv2.py:199-264).
 //
-// A 256-thread workgroup owns a BM x BR tile of y^T (BM, BR = 64 or 128; gemm_tile_choice picks), 4 waves of
+// A 256-thread workgroup owns a BM x BR tile of y^T (64 x 64, or 128 x 128 on large grids: gemm_large_grid), 4 waves of
 // BM / 2 x BR / 2 on v_mfma_f32_32x32x16_f16. The tile is computed transposed (y^T = W x^T: A = rows of W, B = rows
 // of x), so an accumulator lane holds 4 runs of 4 consecutive output columns of one row and stores 8- or 16-byte
 // vectors. K stages of 64 are double-buffered in LDS (36-72 KB) and two register sets carry the next two stages.
@@ -502,15 +502,11 @@ hipError_t gemm_lds_t(const void* x, const void* w, const float* bias, void* y, 
   return hipGetLastError();
 }
 
-// Tile choice (W rows x x rows per workgroup): 0 = 128 x 128, 1 = 128 x 64, 2 = 64 x 128, 3 = 64 x 64. The loop
-// is latency-bound at these sizes (each stage's loads have two stages of compute to land), so more, smaller
-// workgroups per CU win up to the 2000 x 768 x 4608 projections (64 x 64: 403-434 TF/s against 373-393 for
-// 128 x 128, and 1.5-2.3x faster on the 768-wide outputs); 128 x 128 wins only on grids of thousands of its tiles
-// (2000 x 768 x 36864: 454 against 378 TF/s).
-int gemm_tile_choice(int64_t R, int M) {
-  const int64_t n128 = ((R + 127) / 128) * ((M + 127) / 128);
-  return n128 >= 2048 ? 0 : 3;
-}
+// Whether a grid is large enough for 128 x 128 tiles (W rows x x rows per workgroup) instead of 64 x 64. The loop is
+// latency-bound at these sizes (each stage's loads have two stages of compute to land), so more, smaller workgroups per CU
+// win up to the 2000 x 768 x 4608 projections (64 x 64: 403-434 TF/s against 373-393 for 128 x 128, and 1.5-2.3x faster on
+// the 768-wide outputs); 128 x 128 wins only on grids of thousands of its tiles (2000 x 768 x 36864: 454 against 378 TF/s).
+bool gemm_large_grid(int64_t R, int M) { return ((R + 127) / 128) * ((M + 127) / 128) >= 2048; }
 
 }  // namespace
 
@@ -581,37 +577,40 @@ hipError_t launch_gemm_nt(const void* x, const void* w, const float* bias, void*
   if ((x_dt != DT_F16 && x_dt != DT_F32) || !gemm_nt_ok(x_dt, x, w, bias, y, R, K, M, gate, ld_gate) || epi < 0 ||
       epi > 3 || (epi >= 1 && y_dt != DT_F32) || (epi >= 2 && (gate == nullptr || gate_rows < 1)))
     return hipErrorInvalidValue;
-  // fp32 over few rows: up to 768 tiles of 16 columns x 32 rows, K split over a workgroup's waves (us, against the 64 x
-  // 64-tile form: 128 rows 384 -> 1536 (384 tiles) 6.5 / 10.0, 384 -> 3072 (768) 9.1 / 10.6, 1536 -> 384 (96) 10.3 / 31.1;
-  // 203 rows 384 -> 3072 (1,344) 14.5 / 11.0; 1000 rows 1536 -> 384 (768) 27.3 / 32.0, 1500 (1,128) 42.3 / 32.2)
+  // fp32 over few rows: up to 768 tiles of 16 columns x 32 rows, K split over a workgroup's waves. us in a graph, this form /
+  // the 64 x 64-tile form (tiles): 128 rows 1536 -> 384 (96) 10.1 / 31.1, 384 -> 1536 (384) 6.3 / 10.0, 384 -> 3072 (768) 8.5 /
+  // 10.2; 1000 rows 384 -> 384 (768) 8.6 / 10.1, 1536 -> 384 (768) 26.4 / 31.5; past the line 400 rows 384 -> 1536 (1,248)
+  // 14.4 / 10.5, 2000 rows 1536 -> 384 (1,512) 49.9 / 32.0. Narrow ones, where most waves have no step, are on the same side:
+  // 24,576 rows (768) 32 -> 16 3.2 / 4.6, 64 -> 16 3.7 / 4.9, 128 -> 4 4.1 / 6.6; 4,096 rows 64 -> 64 (512) 3.3 / 4.0. Beside
+  // the attention core a trunk block at N = 1000, whose attention output lies on the line, takes the same time in either
+  // form (11.16 and 11.16-11.27 ms for two).
   if (x_dt == DT_F32 && (int64_t)((M + 15) / 16) * ((R + 31) / 32) <= 768)
     return launch_linear_x3_small(static_cast<const float*>(x), static_cast<const float*>(w), bias, y, y_dt, R, K, M,
                                   epi, gate, ld_gate, gate_rows, st);
   if (x_dt == DT_F32)  // fp32 operands: 64 x 64 tiles (the m track's 409,600-row projections)
     return gemm_t<64, 64, float>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st);
-  // below the large-grid case the LDS-direct form takes the same tiles, for 1536 rows and more and for the diffusion
-  // transformer's GEMMs at any row count (the gated outputs, epi 2, and the wide projections of K >= 768): 64 x 64 in
-  // three stages, or 64 W rows x 128 x rows in two for the wide ones from 640 rows on. Measured in a graph over 24
-  // layers' weights, us: 2000 x 768 -> 3072 19.7 (192 x 128, three stages) -> 16.4 (a library's 16.6), 1200 rows 17.3
-  // (register-staged) -> 12.1, 800 13.5 -> 10.7, 400 10.2 -> 7.8 (64 x 64; 9.3 on 64 x 128), 200 6.6 -> 6.4; gated 768 ->
-  // 768 and 1536 -> 768 at 400 rows 7.9 -> 7.0 and 11.4 -> 9.9. Same sums in the same order. The s track's GEMMs (N rows,
-  // epi 0 of K = 384 and epi 1) keep the register-staged form: they run beside the attention core, and there the
-  // LDS-direct form's workgroups found compute units far later (0.85 ms against 0.04 ms per launch at N = 1000).
+  // below the large-grid case the LDS-direct form takes the same tiles, for 1536 rows and more, for gated outputs (epi 2) and
+  // for wide projections (K >= 768, M >= 2048): 64 x 64 in three stages, or 64 W rows x 128 x rows in two for the wide ones
+  // from 640 rows on. Measured in a graph over 24 weights, us, register-staged / LDS-direct: 2000 x 768 -> 3072 19.7 (192 x
+  // 128, three stages) / 16.4 (a library's 16.6), 1200 rows 16.2 / 12.1, 800 13.2 / 10.6, 400 10.2 / 7.7 (64 x 64; 9.3 on 64
+  // x 128), 200 6.5 / 6.3; gated, at 400 rows: 768 -> 768 7.8 / 6.9, 1536 -> 768 11.2 / 9.8, 384 -> 384 6.3 / 5.5, 384 ->
+  // 3072 9.4 / 7.8, 256 -> 64 5.1 / 4.4. Same sums in the same order. The other shapes gain up to a tenth at best (400 rows
+  // 384 -> 384 4.5 / 4.5, 1536 -> 384 8.9 / 8.9, 384 -> 1152 4.7 / 4.4, accumulating 5.6 / 5.0; 384 -> 3072 6.9 / 5.9) and are
+  // the s track's (N rows), which run beside the attention core: there the LDS-direct form's workgroups found compute units
+  // later (0.85 ms against 0.04 ms per launch at N = 1000) and the trunk takes the same time with either (11.62 against
+  // 11.64-11.67 ms for two blocks), so they keep the register-staged form.
   // 128 columns over many rows (the outer product mean's proj_o, 160,000 x 1024 -> 128 at N = 400): one 128-wide
   // column tile, so each x row is read once (124.8 against 148.0 us on 64 x 64 tiles; 128 x 64 and 64 x 128 with
   // three stages 130.5 and 129.0)
   if (M == 128 && R >= 65536)
     return gemm_lds_t<128, 128, 2>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st);
-  if (gemm_tile_choice(R, M) != 0 && (R >= 1536 || epi == 2 || (K >= 768 && M >= 2048)))
+  if (!gemm_large_grid(R, M) && (R >= 1536 || epi == 2 || (K >= 768 && M >= 2048)))
     return M >= 2048 && R >= 640
                ? gemm_lds_t<64, 128, 2>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st)
                : gemm_lds_t<64, 64, 3>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st);
-  switch (gemm_tile_choice(R, M)) {
-    case 0: return gemm_t<128, 128, half_t>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st);
-    case 1: return gemm_t<128, 64, half_t>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st);
-    case 2: return gemm_t<64, 128, half_t>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st);
-    default: return gemm_t<64, 64, half_t>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st);
-  }
+  if (gemm_large_grid(R, M))
+    return gemm_t<128, 128, half_t>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st);
+  return gemm_t<64, 64, half_t>(x, w, bias, y, y_dt, R, K, M, epi, gate, ld_gate, gate_rows, st);
 }
 
 }  // namespace bzpf
