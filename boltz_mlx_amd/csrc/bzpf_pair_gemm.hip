@@ -219,10 +219,12 @@ __global__ __launch_bounds__(256) void trimul_tail_k(const T* __restrict__ o, co
 // row fragments back, with no barrier (a wave's LDS accesses complete in order). The next tile's o block and gate
 // inputs are loaded while the current tile computes; its residual rows are issued at the start of the tile. The
 // gates are computed first and held as fp16 (sigmoid values in (0, 1)), which keeps the tile within 168 VGPRs.
-// One 128-byte line of an o channel row holds 64 positions, i.e. four tiles. Tiles per row are a multiple of four
-// (tiles past N store nothing), so the workgroup's 12 consecutive tiles hold whole lines, and one barrier per round
+// One 128-byte line of an o channel row holds 64 positions, i.e. four tiles. With tiles per row a multiple of four
+// (tiles past N store nothing) the workgroup's 12 consecutive tiles hold whole lines, and one barrier per round
 // keeps its waves in step: the four loads of a line reach L2 together and it is read from HBM once. Without the
-// barrier the waves drift apart by more than the L2 residency of a line and o is read about 2.3 times.
+// barrier the waves drift apart by more than the L2 residency of a line and o is read about 2.3 times. The launcher's
+// other form has only the tiles that hold positions: there a line's tiles may fall to two workgroups, which costs 4 to 8%
+// (N = 257 and 270 33 -> 35.8 us, 400 66.6 -> 69.7) and is paid only where it saves a whole round of few.
 constexpr int TAIL_WAVES = 12;
 
 template <int KIN>
@@ -914,8 +916,10 @@ static hipError_t tm_tail_f16(const void* o, const float* now, const float* nob,
   static int cache[kMaxDevices];
   const int resident = resident_grid(trimul_tail_f16_k<KIN>, 64 * TAIL_WAVES, cache);
   if (resident <= 0) return hipErrorInvalidDevice;
-  // tiles of whole 64-position groups per row, or (where that saves one of the first rounds: N = 203, 1 round for 2, 27.4
-  // to 19.1 us) only those that hold positions
+  // Tiles of whole 64-position groups per row, or only those that hold positions where that saves one of the first four
+  // rounds (us in a graph, whole groups / only those: N = 203, 2 rounds for 1, 33.0 / 23.9, at 64 channels 16.3 / 11.8; the
+  // same rounds: N = 100 18.0 / 18.8, 220 33.5 / 30.2, 350 55.3 / 55.0, 450 88.3 / 89.6, 480 93.3 / 94.4). Past four a saved
+  // round is a small part of the whole (N = 530, 7 for 6: 125 / 118).
   const int64_t round = (int64_t)resident * TAIL_WAVES, t4 = (N + 63) / 64 * 4, t1 = (N + 15) / 16;
   const int64_t r4 = (N * t4 + round - 1) / round, r1 = (N * t1 + round - 1) / round;
   const int64_t tpr = r1 < r4 && r4 <= 4 ? t1 : t4, ntiles = N * tpr;  // a row's last tile ends inside ld
