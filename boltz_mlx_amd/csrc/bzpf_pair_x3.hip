@@ -5,13 +5,14 @@
 //   linear_resid_ln           (kernels_nax3.py:176-198);
 //   transition                (transition.py:27-54, 148-154).
 // The fp32 matrix instructions these ran on (v_mfma_f32_16x16x4_f32) take 2.7 times the six part products' time, and a
-// short input was bound by one workgroup's chain of staging and tiles. us at N = 29 / 128 / 400 / 513 (wrapper calls one
-// after another, fp32 MFMA form -> this one; the smallest are the host's time):
-//   trimul_proj      43 / 48 / 237 / 366  ->  15 / 21 / 117 / 195   (0.207 TFLOP of part products at N = 513: 1.06 PFLOP/s)
-//   trimul_tail      22 / 26 / 189 / 345  ->  14 / 17 / 110 / 200   (675 MB at N = 513: 3.4 TB/s)
-//   triattn_proj     63 / 72 / 237 / 396  ->  16 / 22 / 150 / 240   (675 MB at N = 513: 2.8 TB/s)
-//   linear_resid_ln  13 / 14 /  62 / 100  ->  12 / 14 /  53 /  94   (540 MB at N = 513: 5.7 TB/s)
-//   transition       84 / 90 / 563 / 935  ->  27 / 65 / 342 / 538   (1.15 PFLOP/s of part products)
+// short input was bound by one workgroup's chain of staging and tiles. us at N = 29 / 128 / 400 / 513 (launches of one kernel
+// in a graph, fp32 MFMA form -> this one):
+//   trimul_proj      42 / 46 / 224 / 363  ->  14 / 21 / 114 / 195   (0.207 TFLOP of part products at N = 513: 1.06 PFLOP/s)
+//   trimul_tail      22 / 27 / 218 / 362  ->  14 / 19 / 124 / 196   (675 MB at N = 513: 3.4 TB/s)
+//   triattn_proj     63 / 70 / 236 / 395  ->  15 / 23 / 152 / 241   (675 MB at N = 513: 2.8 TB/s)
+//   linear_resid_ln  12 / 15 /  74 / 122  ->  14 / 17 /  68 / 119   (540 MB at N = 513: 4.5 TB/s)
+//     transposed     13 / 15 /  82 / 136  ->  14 / 17 /  76 / 133
+//   transition       84 / 88 / 573 / 962  ->  27 / 64 / 315 / 527   (1.18 PFLOP/s of part products)
 // Sums that come out not finite are formed again on the fp32 instructions (wave_nonfinite, bzpf_rowgemm_x3.h).
 #include <algorithm>
 #include <type_traits>
@@ -517,6 +518,7 @@ __device__ __forceinline__ void transition_finite(f4 (&out)[RB][8], const float*
 
 // Large inputs: tiles of 128 RB rows (8 waves of 16 RB), the hidden units streamed through LDS in chunks of 32 (fc1, fc2 rows
 // and fc3 columns, split as they are written), the next chunk's values loaded while the current one computes.
+// RB = 2 is at the 256 VGPRs of two waves per SIMD: 12 spill (52 bytes a lane), one 16-byte store and load of them a chunk.
 constexpr int XH = 32;
 template <int RB>
 __global__ __launch_bounds__(XT) void transition_x3_k(const float* __restrict__ xn, const float* __restrict__ w12,

@@ -246,8 +246,8 @@ hipError_t launch_seq_attention(const void* q, const void* k, const void* v, con
 // Core dispatch (impl mirrors the reference's scalar / mma choice, boltz_mlx/kernels.py:902-945): 0 = the matrix cores
 // for C = 32 (fp16, or fp32 as split operands), else the VALU kernel; 1 = the VALU kernel; 2 = MFMA (fp16, C = 32
 // only). The fp32 matrix-core kernel takes every N and mask stride that its 32-bit buffer offsets hold; at every size
-// measured it is the faster one (VALU -> matrix cores: N = 29 26 -> 18 us, 128 137 -> 15, 400 2,410 -> 285,
-// 640 8,980 -> 832).
+// measured it is the faster one (VALU -> matrix cores: N = 29 24 -> 5 us, 128 133 -> 15, 400 2,405 -> 249,
+// 640 8,967 -> 807).
 hipError_t launch_triattn_core(const void* qkg, const void* vt, const void* tb, const float* mask, int64_t mask_si,
                                int64_t mask_sk, float inf, void* out, int dt, int64_t N, int64_t ldk, int H, int C,
                                int impl, hipStream_t st) {

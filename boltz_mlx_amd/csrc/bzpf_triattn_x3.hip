@@ -3,12 +3,13 @@
 // (bzpf_x3.h), so logits, softmax, probabilities and sums all keep fp32 accuracy.
 //
 // What bounds it: a 32-key x 32-query tile costs 24 v_mfma_f32_32x32x16_bf16 (768 cycles) and about 210 VALU
-// instructions (the probabilities' split is 88 of them); at N = 640 a tile takes 1,400-1,700 cycles of its SIMD, so the
-// two pipes overlap in part. N = 400: 285 us (207 TFLOP/s), against 2,410 us on the VALU kernel (kept for the other head
-// widths and as the caller's choice); the true fp32 MFMA (v_mfma_f32_32x32x2f32) would need 2,048 cycles a tile.
+// instructions (the probabilities' split is 88 of them); at N = 640 (807 us, 1.02 M tiles on 1,024 SIMDs) a tile takes about
+// 1,940 cycles of its SIMD at the nominal 2.4 GHz (fewer at the clock held under load): the two pipes overlap little. N = 400: 249 us (132 TFLOP/s of the 32.8
+// GFLOP without padding), against 2,405 us on the VALU kernel (kept for the other head widths and as the caller's choice);
+// the true fp32 MFMA (v_mfma_f32_32x32x2f32) would need 2,048 cycles a tile.
 //
-// Work unit: one (head h, row i, 128 queries), 4 waves of 32 queries; 124 VGPRs and 31 KB of LDS, so four workgroups
-// share a CU (64-key stages at 187 VGPRs and two workgroups: 324 us). S^T = K Q^T as in the fp16 core: lane l = 32 hl + q
+// Work unit: one (head h, row i, 128 queries), 4 waves of 32 queries; 128 VGPRs and 31 KB of LDS, so four workgroups
+// share a CU (64-key stages at 187 VGPRs and two workgroups took 1.14 times as long). S^T = K Q^T as in the fp16 core: lane l = 32 hl + q
 // owns query q and keys 8 (e / 4) + 4 hl + e % 4 of each 32-key tile, so its statistics need one cross-half step and its
 // probabilities are, split in place, already the B operand of O^T = V^T P^T for V^T staged in the matching key order.
 // 32 keys of K and V^T per stage are loaded a stage ahead, split by the threads that loaded them and written to one of

@@ -22,8 +22,8 @@ namespace bzpf {
 // Tiles are ordered (channel, tile) and dealt to the XCDs in contiguous ranges, so one channel's a and b stay in
 // one XCD's L2.
 // Bound by the matrix cores and the split beside them (a stage of a 64 x 64 wave tile is 768 MFMA cycles and 88 VALU
-// instructions): N = 640 402 us (167 TFLOP/s, 0.4 of the bf16 peak in part products), N = 513 276, N = 333 79, against
-// 626, 555 and 160 us for the fp32 MFMA kernel this replaces; error against float64 3.8e-7 -> 3.2e-7 (N = 513).
+// instructions): N = 640 382 us (176 TFLOP/s, 0.42 of the bf16 peak in part products), N = 513 260, N = 400 164, against
+// 622, 554 and 276 us for the fp32 MFMA kernel this replaces; error against float64 4.1e-7 -> 3.5e-7 (N = 513).
 // The stages of bk columns to contract: `all` of them, or those up to the extent the device holds (rounded up to 64
 // columns; 0 or >= N: all).
 __device__ __forceinline__ int contract_stages(int all, int bk, const int* ext, int64_t N) {
@@ -386,9 +386,9 @@ static hipError_t contract_x3(const float* ab, float* o, int64_t N, int64_t ld, 
   return hipGetLastError();
 }
 
-// 192 x 192 tiles (3 x 3 blocks a wave: half again the products per LDS read of 2 x 2) where their padded area is not much
-// larger than that of 128 x 128 tiles: they measure 0.83-0.85 ns per 1,000 padded outputs and channel against 0.98
-// (N = 513: 276 against 359 us; N = 333, equal areas: 79 against 93; N = 400: 226 against 186; N = 640: 502 against 402).
+// 192 x 192 tiles (3 x 3 blocks a wave: half again the products per LDS read of 2 x 2) where their padded area is at most 8/7
+// of that of 128 x 128 tiles: per padded output they take 0.85 to 0.96 of the time (us, 192 / 128 wide: N = 513 276 / 359 at
+// 0.81 times the area; N = 333, equal areas, 79 / 93; N = 400, 1.27 times the area, 226 / 186; N = 640, 1.44 times, 502 / 402).
 static hipError_t contract_f32(const float* ab, float* o, int64_t N, int64_t ld, int64_t kl, const int* ext, int D,
                                hipStream_t st) {
   const int64_t t128 = (N + 127) / 128 * 128, t192 = (N + 191) / 192 * 192;
