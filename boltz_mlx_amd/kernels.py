@@ -417,7 +417,7 @@ def pair_mask_scope():
 
 def _mask_entry(mask: torch.Tensor):
     sc = _MASK_SCOPE
-    if sc.entries is None or (mask.is_cuda and _capturing() != sc.capturing):
+    if sc.entries is None or (mask.is_cuda and torch.cuda.is_current_stream_capturing() != sc.capturing):
         return None
     key = (_stream() if mask.is_cuda else None, mask.data_ptr(), tuple(mask.shape), tuple(mask.stride()), mask._version)
     return sc.entries.setdefault(key, {"mask": mask})
